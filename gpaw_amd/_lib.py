@@ -12,6 +12,7 @@ LIB_PATH = os.path.join(_HERE, 'libgpaw_amd.so')
 
 GPAW_F64, GPAW_C128, GPAW_F32, GPAW_C64 = 0, 1, 2, 3
 GPAW_OK, GPAW_EINVAL, GPAW_EUNSUPPORTED = 0, -1, -2
+GPAW_RENORMALIZE_MAX, GPAW_RENORMALIZE_WORK = 7, 1024
 GPAW_EDEVICE, GPAW_ENOMEM, GPAW_ENOCONV = -3, -4, -5
 
 _vp = ctypes.c_void_p
@@ -66,6 +67,8 @@ PROTOTYPES = {
     'gpaw_dots': (_i, [_vp, _vp, _l, _l, _d, _vp, _vp]),
     'gpaw_dots_noalloc': (_i, [_vp, _vp, _l, _l, _d, _vp, _vp]),
     'gpaw_axpby': (_i, [_vp, _vp, _d, _d, _l, _vp]),
+    'gpaw_axpby_shared': (_i, [_vp, _vp, _d, _d, _l, _l, _vp]),
+    'gpaw_renormalize': (_i, [_vp, _l, _l, _d, _d, _vp, _vp]),
     'gpaw_sub_scalar': (_i, [_vp, _vp, _d, _l, _vp]),
     'gpaw_cast': (_i, [_vp, _i, _vp, _i, _l, _vp]),
     'gpaw_copy': (_i, [_vp, _vp, _l, _vp]),

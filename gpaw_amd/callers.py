@@ -21,7 +21,7 @@ stencil / transfer launch.
 """
 import numpy as np
 
-from . import _arrays, ops
+from . import _arrays, _lib, ops
 from ._arrays import Arg
 
 
@@ -59,8 +59,11 @@ def interpolate_density(interpolator, finegd, nt_sG, nt_sg, charge=0.0,
     if not finegd.pbc_c.all():
         pseudo_charge = -(charge + comp_charge)
         if abs(pseudo_charge) > 1.0e-14:
-            x = pseudo_charge / np.sum(finegd.integrate(out.tensor))
-            ops.scale(out.tensor, x)
+            if np.prod(out.shape[:-3]) <= _lib.GPAW_RENORMALIZE_MAX:
+                ops.renormalize(finegd, out.tensor, pseudo_charge)
+            else:   # numpy adds 8 and more integrals in another order
+                x = pseudo_charge / np.sum(finegd.integrate(out.tensor))
+                ops.scale(out.tensor, x)
     out.finish()
 
 
@@ -73,11 +76,7 @@ def restrict_potential(restrictor, vt_sg, vHt_g, vt_sG):
     vH = Arg(vHt_g, name='vHt_g')
     out = Arg(vt_sG, write=True, name='vt_sG')
     t = fine.tensor
-    if t.dim() == 3:
-        ops.axpby(t, vH.tensor, 1.0, 1.0)
-    else:
-        for s in range(t.shape[0]):
-            ops.axpby(t[s], vH.tensor, 1.0, 1.0)
+    ops.axpby_shared(t, vH.tensor, 1.0, 1.0, 1 if t.dim() == 3 else t.shape[0])
     restrictor.apply(t, out.tensor)
     fine.finish()
     out.finish()

@@ -420,7 +420,7 @@ extern "C" int gpaw_sum(const double* a, long n, double scale, double* result, v
 {
     if (!a || !result || n < 0) return gpaw_fail(GPAW_EINVAL, "sum: bad argument");
     double* partial = nullptr;
-    hipError_t e = hipMallocAsync((void**)&partial, sizeof(double) * 1024, (hipStream_t)stream);
+    hipError_t e = hipMallocAsync((void**)&partial, sizeof(double) * SUM_PARTIALS, (hipStream_t)stream);
     if (e != hipSuccess) return gpaw_check(e, "sum: partials");
     int np = 0;
     e = launch_sum(a, n, partial, &np, (hipStream_t)stream);
@@ -507,6 +507,25 @@ extern "C" int gpaw_axpby(double* y, const double* x, double a, double b, long n
 {
     if (!y || (!x && b != 0.0) || n < 0) return gpaw_fail(GPAW_EINVAL, "axpby: bad argument");
     return gpaw_check(launch_axpby(y, x ? x : y, a, b, n, (hipStream_t)stream), "axpby");
+}
+
+extern "C" int gpaw_axpby_shared(double* y, const double* x, double a, double b, long nin, long n,
+                                 void* stream)
+{
+    if (n < 0 || nin < 0 || nin > 0x7fffffffL || (n > 0 && nin > 0 && (!y || !x)))
+        return gpaw_fail(GPAW_EINVAL, "axpby_shared: bad argument");
+    return gpaw_check(launch_axpby_shared(y, x, a, b, (int)nin, n, (hipStream_t)stream),
+                      "axpby_shared");
+}
+
+extern "C" int gpaw_renormalize(double* y, long nin, long n, double scale, double target,
+                                double* work, void* stream)
+{
+    if (!y || !work || n < 0 || nin < 0 || nin > GPAW_RENORMALIZE_MAX)
+        return gpaw_fail(GPAW_EINVAL, "renormalize: bad argument (at most %d functions)",
+                         GPAW_RENORMALIZE_MAX);
+    return gpaw_check(launch_renormalize(y, (int)nin, n, scale, target, work, (hipStream_t)stream),
+                      "renormalize");
 }
 
 extern "C" int gpaw_sub_scalar(double* y, const double* x, double b, long n, void* stream)

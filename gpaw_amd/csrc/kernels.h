@@ -187,8 +187,13 @@ hipError_t launch_reduce_partials(const double* partial, int n, double scale, do
 // launch_reduce_partials sums it
 hipError_t launch_reduce_rows(const double* partial, int nrows, int ncols, double scale,
                               double* result, hipStream_t st);
+constexpr int SUM_PARTIALS = 1024;   // partial sums of launch_sum, at most
 hipError_t launch_sum(const double* a, long long n, double* partial, int* npartial,
                       hipStream_t st);
+// y *= target / sum_k (scale * sum of y_k), k < nin functions of n points;
+// partial holds nin * SUM_PARTIALS doubles
+hipError_t launch_renormalize(double* y, int nin, long long n, double scale, double target,
+                              double* partial, hipStream_t st);
 // result[j] = scale * sum_g a[g] * b[j n + g] for j < nb (nb <= 65535);
 // partial holds nb * dots_chunks(n) doubles.
 int dots_chunks(long long n);
@@ -196,6 +201,8 @@ hipError_t launch_dots(const double* a, const double* b, int nb, long long n, do
                        double* partial, double* result, hipStream_t st);
 hipError_t launch_axpby(double* y, const double* x, double a, double b, long long n,
                         hipStream_t st);   // y = a*y + b*x
+hipError_t launch_axpby_shared(double* y, const double* x, double a, double b, int nin,
+                               long long n, hipStream_t st);   // y_k = a*y_k + b*x
 hipError_t launch_sub_scalar(double* y, const double* x, double b, long long n,
                              hipStream_t st);  // y = x - b
 hipError_t launch_fill(void* y, int dtype, long long n, hipStream_t st);

@@ -27,9 +27,10 @@ __global__ __launch_bounds__(256) void k_sum(const double* __restrict__ a, i64 n
     __shared__ double red[256];
     double s = 0.0;
     const i64 stride = (i64)gridDim.x * 256;
+    a += (i64)blockIdx.y * n;   // one row of partials per function
     for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) s += a[i];
     s = block_sum<256>(s, red);
-    if (threadIdx.x == 0) partial[blockIdx.x] = s;
+    if (threadIdx.x == 0) partial[(i64)blockIdx.y * gridDim.x + blockIdx.x] = s;
 }
 
 // Row j of a block of dot products: partial sums of a[g] * b[j n + g] over
@@ -66,6 +67,18 @@ __global__ __launch_bounds__(256) void k_axpby(double* __restrict__ y, const dou
 {
     const i64 i = (i64)blockIdx.x * 256 + threadIdx.x;
     if (i < n) y[i] = a * y[i] + b * x[i];
+}
+
+// y_k = a*y_k + b*x for nin functions of n points, x shared by them (one
+// read of x and one launch instead of nin of each; bound by HBM)
+__global__ __launch_bounds__(256) void k_axpby_shared(double* __restrict__ y,
+                                                      const double* __restrict__ x, double a,
+                                                      double b, int nin, i64 n)
+{
+    const i64 i = (i64)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const double bx = b * x[i];
+    for (int k = 0; k < nin; k++) y[k * n + i] = a * y[k * n + i] + bx;
 }
 
 // y = x - b  (numpy's rho - background, phi -= phi_ave)
@@ -110,6 +123,31 @@ __global__ __launch_bounds__(256) void k_scale(double* __restrict__ y, double a,
     if (i < n) y[i] = y[i] * a;
 }
 
+// y *= target / sum_k (scale * sum of y_k) over nin functions of n points
+// (nt_sg *= -charge / integral, gpaw/density.py:230-234), from the partial
+// sums that k_sum left in rows of np.  Every block sums the rows itself,
+// each in the order and tree of k_reduce_partials, then the rows in index
+// order as numpy adds fewer than 8 numbers: no reduction launch and no
+// readback between the sum and the scaling (with the chunked interpolation,
+// 2 spins 63^3 -> 127^3 went from 119 to 38 us a call; the readback alone left
+// the GPU idle for about 30 us).
+__global__ __launch_bounds__(256) void k_renormalize(double* __restrict__ y,
+                                                     const double* __restrict__ partial, int nin,
+                                                     int np, double scale,
+                                                     double target, i64 total)
+{
+    __shared__ double red[256];
+    double all = 0.0;
+    for (int k = 0; k < nin; k++) {
+        double s = 0.0;
+        for (int i = threadIdx.x; i < np; i += 256) s += partial[(i64)k * np + i];
+        all += block_sum<256>(s, red) * scale;
+    }
+    const double f = target / all;
+    const i64 step = (i64)gridDim.x * 256;
+    for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < total; i += step) y[i] = y[i] * f;
+}
+
 // 16-byte copy, four loads in flight per thread, grid-stride over blocks of
 // 4 x 256 vectors (the attainable HBM read + write rate)
 __global__ __launch_bounds__(256) void k_copy16_flat(uint4* __restrict__ y,
@@ -150,13 +188,39 @@ hipError_t launch_reduce_partials(const double* partial, int n, double scale, do
     return launch_error();
 }
 
+// blocks (partial sums) of a sum over n points, at most SUM_PARTIALS
+static int sum_blocks(long long n)
+{
+    const long long nb = (n + 255) / 256;
+    return (int)(nb < 1 ? 1 : nb > SUM_PARTIALS ? SUM_PARTIALS : nb);
+}
+
 hipError_t launch_sum(const double* a, long long n, double* partial, int* npartial, hipStream_t st)
 {
-    int nb = (int)((n + 255) / 256);
-    if (nb > 1024) nb = 1024;
-    if (nb < 1) nb = 1;
-    *npartial = nb;
-    launch_kernel(k_sum, dim3(nb), dim3(256), 0, st, a, (i64)n, partial);
+    *npartial = sum_blocks(n);
+    launch_kernel(k_sum, dim3(*npartial), dim3(256), 0, st, a, (i64)n, partial);
+    return launch_error();
+}
+
+hipError_t launch_renormalize(double* y, int nin, long long n, double scale, double target,
+                              double* partial, hipStream_t st)
+{
+    if (n <= 0 || nin <= 0) return hipSuccess;
+    const int np = sum_blocks(n);
+    launch_kernel(k_sum, dim3(np, nin), dim3(256), 0, st, (const double*)y, (i64)n, partial);
+    const i64 total = (i64)nin * n;
+    i64 nb = (total + 1023) / 1024;   // 4 points a thread; at most 8 blocks per CU
+    if (nb > 2048) nb = 2048;
+    launch_kernel(k_renormalize, dim3((unsigned)nb), dim3(256), 0, st, y, (const double*)partial,
+                  nin, np, scale, target, total);
+    return launch_error();
+}
+
+hipError_t launch_axpby_shared(double* y, const double* x, double a, double b, int nin,
+                               long long n, hipStream_t st)
+{
+    if (n <= 0 || nin <= 0) return hipSuccess;
+    launch_kernel(k_axpby_shared, grid1(n), dim3(256), 0, st, y, x, a, b, nin, (i64)n);
     return launch_error();
 }
 

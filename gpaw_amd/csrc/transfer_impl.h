@@ -66,6 +66,31 @@ __global__ __launch_bounds__(256) void k_interp2(const V* __restrict__ in, V* __
                           k1, k2, ph);
 }
 
+// Tiles and i0 chunks of the tile kernels.  A block's planes are a serial
+// chain of about 1 us each, so few bands on one chunk leave the chip idle:
+// 2 x 127^3 -> 63^3 K = 6 is 32 blocks of 135 planes.  The axis is split until
+// there are TR_BLOCKS_RESTRICT / TR_BLOCKS_INTERP blocks (two / four per CU);
+// beyond that the 2 K - 3 (K - 1) planes that every chunk sweeps again cost
+// more than the blocks gain.  Measured, 1 / 256 / 512 / 1024 / 2048 blocks:
+// that restriction 121 / 27 / 25 / 36 / 54 us, the K = 6 interpolation
+// 2 x 63^3 -> 127^3 54 / 31 / 21 / 18.5 / 20 us.
+constexpr i64 TR_BLOCKS_RESTRICT = 512, TR_BLOCKS_INTERP = 1024;
+
+inline TileTr tile_tr(const TrArgs& t, bool interpolate, int nin)
+{
+    TileTr tt;
+    tt.nt1 = (t.nout[1] + 7) / 8;
+    tt.nt2 = (t.nout[2] + 31) / 32;
+    const int n0 = interpolate ? interp2_cells(t, 0) : t.nout[0];   // outputs or centres
+    const i64 base = (i64)tt.nt1 * tt.nt2 * nin;
+    const i64 want = interpolate ? TR_BLOCKS_INTERP : TR_BLOCKS_RESTRICT;
+    i64 nch = (want + base - 1) / base;
+    if (nch > n0) nch = n0;
+    tt.cq = (int)((n0 + nch - 1) / nch);
+    tt.nch = (n0 + tt.cq - 1) / tt.cq;
+    return tt;
+}
+
 template <class V, int K>
 hipError_t tr_launch(const Transfer& tr, int mode, const void* in, void* out, void* zero_out,
                      const Phases& ph, int nin, hipStream_t st)
@@ -92,12 +117,18 @@ hipError_t tr_launch(const Transfer& tr, int mode, const void* in, void* out, vo
     const bool big2 = K == 2 && !tr.interpolate && t.ngout * nin >= (1 << 20);
     if ((K >= 4 || big2) && t.nout[1] >= 4 && t.nout[2] >= 16 &&
         (long)t.gin.n[1] * t.gin.n[2] < PLANE_REF_MAX && !getenv("GPAW_AMD_POINTWISE_TRANSFER")) {
-        TileTr tt;
-        tt.nt1 = (t.nout[1] + 7) / 8;
-        tt.nt2 = (t.nout[2] + 31) / 32;
-        dim3 gt((unsigned)(tt.nt1 * tt.nt2 * nin));
-        if (!tr.interpolate)
-            launch_kernel((k_restrict_tile<V, K, 8, 32>), gt, dim3(256), 0, st, (const V*)in,
+        const TileTr tt = tile_tr(t, tr.interpolate, nin);
+        const dim3 gt((unsigned)(tt.nt1 * tt.nt2 * tt.nch * nin));
+        // chunked real restrictions (few blocks per CU) take two planes per
+        // step: 25 us against 27 on 2 x 127^3 -> 63^3, K = 6; one plane is
+        // faster where blocks hide each other's waits (256 x 64^3: 174 us
+        // against 181), and complex slabs have no registers for two
+        constexpr int PL2 = VT<V>::cplx ? 1 : 2;
+        if (!tr.interpolate && tt.nch > 1)
+            launch_kernel((k_restrict_tile<V, K, 8, 32, PL2>), gt, dim3(256), 0, st,
+                               (const V*)in, (V*)out, t, tt, ph);
+        else if (!tr.interpolate)
+            launch_kernel((k_restrict_tile<V, K, 8, 32, 1>), gt, dim3(256), 0, st, (const V*)in,
                                (V*)out, t, tt, ph);
         else if (mode == TR_SUBTRACT)
             launch_kernel((k_interp_tile<V, K, 8, 32, TR_SUBTRACT>), gt, dim3(256), 0, st,

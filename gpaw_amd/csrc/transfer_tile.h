@@ -3,7 +3,9 @@
 // input many times.
 //
 // Both kernels own a tile of the output (i1, i2) plane (256 threads, one
-// output column each) and sweep the input planes along i0 in order:
+// output column each) and a chunk of the i0 axis, and sweep the chunk's input
+// planes in order (a step is bound by its load wait, two barriers and the
+// LDS passes, about 1 us a plane, so what counts is blocks in flight):
 //   1. the tile's slab of the current input plane (with its halo) is stored
 //      into LDS from registers, ghost-indexed (periodic + Bloch phase or
 //      zero); the next plane's slab is loaded into those registers while
@@ -26,27 +28,42 @@ namespace gpaw {
 
 struct TileTr {
     int nt1, nt2;   // output tiles along i1, i2
+    int nch, cq;    // chunks along i0: cq output planes (restriction) or cq
+                    // coarse centre planes (interpolation) each
 };
 
 // ------------------------------------------------------------ restriction
-template <class V, int K, int T1, int T2>
+// PL input planes per step (one wait, two barriers): the slabs of the next
+// PL planes are in flight while the current ones are combined.  Real slab
+// rows are stored de-interleaved (even columns, then odd ones from column
+// SE, half the banks away): the z-pass reads columns 2 z + const, a 2-way
+// bank conflict on an interleaved row.
+template <class V, int K, int T1, int T2, int PL>
 __global__ __launch_bounds__(256) void k_restrict_tile(const V* __restrict__ in, V* __restrict__ out,
                                                        TrArgs t, TileTr tt, Phases ph)
 {
     constexpr int SR = 2 * T1 + 2 * K - 3;   // input rows of the slab
     constexpr int SC = 2 * T2 + 2 * K - 3;   // input columns of the slab
+    constexpr bool DI = !VT<V>::cplx;        // de-interleaved slab rows
+    constexpr int SE = 48;                   // their first odd column
+    constexpr int LR = DI ? SE + SC / 2 : SC;
+    static_assert(!DI || (SC + 1) / 2 <= SE, "slab row");
     constexpr int W = 2 * K - 1;             // x window
-    __shared__ V A[SR * SC];
-    __shared__ V Z[SR * T2];
+    __shared__ V A[PL * SR * LR];
+    __shared__ V Z[PL * SR * T2];
     const int b = xcd_tile(blockIdx.x, gridDim.x);
     const int tz = b % tt.nt2;
-    const int ty = (b / tt.nt2) % tt.nt1;
-    const int band = b / (tt.nt2 * tt.nt1);
+    int rest = b / tt.nt2;
+    const int ty = rest % tt.nt1;
+    rest /= tt.nt1;
+    const int ch = rest % tt.nch;
+    const int band = rest / tt.nch;
     const int tid = threadIdx.x;
     const int tzi = tid % T2, tyi = tid / T2;
     const V* __restrict__ a = in + (i64)band * t.ngin;
     V* __restrict__ o = out + (i64)band * t.ngout;
     const int o1 = ty * T1 + tyi, o2 = tz * T2 + tzi;
+    const int o0s = ch * tt.cq, no0 = min(tt.cq, t.nout[0] - o0s);
     // slab origin (input index of slab row/col 0)
     const int r0 = 2 * ty * T1 - t.lo[1];
     const int s0 = 2 * tz * T2 - t.lo[2];
@@ -54,19 +71,36 @@ __global__ __launch_bounds__(256) void k_restrict_tile(const V* __restrict__ in,
     const int hi0 = 2 * t.nout[0] + 2 * K - 3 - t.lo[0];
     const int hi1 = 2 * t.nout[1] + 2 * K - 3 - t.lo[1];
     const int hi2 = 2 * t.nout[2] + 2 * K - 3 - t.lo[2];
-    const int p0s = -t.lo[0];
-    const int np = 2 * t.nout[0] + 2 * K - 3;   // input planes swept
+    const int p0s = 2 * o0s - t.lo[0];
+    const int np = 2 * no0 + 2 * K - 3;   // input planes swept
     // slab cells of this thread: c = tid + 256 k, with their in-plane
     // references (code 3: a cell no valid output uses, zero without a
-    // load).  The next plane's cells are loaded raw into registers while the
-    // current plane is combined and fixed (zero / phase) when stored to LDS.
+    // load).  The next planes' cells are loaded raw into registers while the
+    // current ones are combined and fixed (zero / phase) when stored to LDS.
     constexpr int NS = (SR * SC + 255) / 256;
-    auto cref = [&](int k) -> PlaneRef {   // recomputed: registers are scarce here
+    auto make_ref = [&](int k) -> PlaneRef {
         const int c = tid + 256 * k;
         const int j1 = r0 + c / SC, j2 = s0 + c % SC;
         const bool ok = c < SR * SC && j1 >= lo1 && j1 < hi1 && j2 >= lo2 && j2 < hi2;
         return ok ? plane_ref(j1, j2, t.gin) : PREF_ZERO;
     };
+    auto make_lds = [&](int k) -> int {
+        const int c = tid + 256 * k, r = c / SC, col = c % SC;
+        return DI ? r * LR + ((col & 1) ? SE : 0) + (col >> 1) : c;
+    };
+    // kept in registers for real data; recomputed for complex data, whose
+    // registers are scarce
+    PlaneRef kref[DI ? NS : 1];
+    int klds[DI ? NS : 1];
+    if (DI) {
+#pragma unroll
+        for (int k = 0; k < NS; k++) {
+            kref[k] = make_ref(k);
+            klds[k] = make_lds(k);
+        }
+    }
+    auto cref = [&](int k) -> PlaneRef { return DI ? kref[k] : make_ref(k); };
+    auto clds = [&](int k) -> int { return DI ? klds[k] : make_lds(k); };
     const i64 plane = (i64)t.gin.n[1] * t.gin.n[2];
     auto pflag = [&](int p0, i64& base) -> int {
         int f = 3;
@@ -74,63 +108,102 @@ __global__ __launch_bounds__(256) void k_restrict_tile(const V* __restrict__ in,
         base = f == 3 ? 0 : (i64)p0 * plane;
         return f;
     };
-    V pre[NS];
-    int pf;
-    {
-        i64 base;
-        pf = pflag(p0s, base);
+    V pre[PL][NS];
+    int pf[PL];
+    auto load = [&](int j) {
+        i64 base[PL];
 #pragma unroll
-        for (int k = 0; k < NS; k++) pre[k] = a[base + pref_off(cref(k))];
-    }
-    const bool own = o1 < t.nout[1] && o2 < t.nout[2];
-    V ring[W];
-    // x-pass at the start of plane step j, over the ring as step j - 1 left
-    // it: output plane o0 is complete when its last tap plane arrived.  Its
-    // store is issued with the next plane's loads.
-    auto xpass = [&](int j) {
-        if (j >= W && ((j - W) & 1) == 0) {
-            V s[K + 1];
+        for (int u = 0; u < PL; u++) pf[u] = pflag(p0s + j + u, base[u]);
 #pragma unroll
-            for (int m = 0; m <= K; m++) s[m] = ring[K - 1 + rst_tap<K>(m)];
-            const V r = rst_combine<V, K>(s);
-            if (own) o[((i64)((j - W) >> 1) * t.nout[1] + o1) * t.nout[2] + o2] = r;
+        for (int k = 0; k < NS; k++) {
+            const int off = pref_off(cref(k));
+#pragma unroll
+            for (int u = 0; u < PL; u++) pre[u][k] = a[base[u] + off];
         }
     };
-    for (int j = 0; j < np; j++) {
-        // one wait per plane step, for loads issued a step earlier
+    load(0);
+    const bool own = o1 < t.nout[1] && o2 < t.nout[2];
+    V* __restrict__ oc = o + ((i64)o0s * t.nout[1] + o1) * t.nout[2] + o2;
+    const i64 oplane = (i64)t.nout[1] * t.nout[2];
+    V ring[W];
+    // x-pass over the ring: an output plane is complete when its last tap
+    // plane, an even one, arrived
+    auto xpass = [&]() -> V {
+        V s[K + 1];
 #pragma unroll
-        for (int k = 0; k < NS; k++) vtouch(pre[k]);
+        for (int m = 0; m <= K; m++) s[m] = ring[K - 1 + rst_tap<K>(m)];
+        return rst_combine<V, K>(s);
+    };
+    // outputs of the step that began at plane j, stored with the next step's
+    // loads; a one-plane step leaves its x-pass to this point too
+    V xr[PL > 1 ? PL / 2 : 1];
+    auto store = [&](int j) {
+        if constexpr (PL == 1) {
+            const int p = j - (W - 1);
+            if (p >= 0 && !(p & 1)) {
+                const V r = xpass();
+                if (own) oc[(p >> 1) * oplane] = r;
+            }
+        } else {
 #pragma unroll
-        for (int k = 0; k < NS; k++)
-            if (tid + 256 * k < SR * SC) A[tid + 256 * k] = ghost_fix(pre[k], pf, cref(k), ph);
-        xpass(j);
-        if (j + 1 < np) {
-            i64 base;
-            pf = pflag(p0s + j + 1, base);
-#pragma unroll
-            for (int k = 0; k < NS; k++) pre[k] = a[base + pref_off(cref(k))];
+            for (int u = 0; u < PL; u += 2) {
+                const int p = j + u - (W - 1);
+                if (p >= 0 && (p >> 1) < no0 && own) oc[(p >> 1) * oplane] = xr[u / 2];
+            }
         }
+    };
+    constexpr int NZ = (PL * SR * T2 + 255) / 256;   // z-pass values per thread
+    for (int j = 0; j < np; j += PL) {
+        // one wait per step, for loads issued a step earlier
+#pragma unroll
+        for (int u = 0; u < PL; u++)
+#pragma unroll
+            for (int k = 0; k < NS; k++) vtouch(pre[u][k]);
+#pragma unroll
+        for (int k = 0; k < NS; k++) {
+            const int c = tid + 256 * k;
+            if (c < SR * SC) {
+                const PlaneRef cr = cref(k);
+                V* d = A + clds(k);
+#pragma unroll
+                for (int u = 0; u < PL; u++) d[u * SR * LR] = ghost_fix(pre[u][k], pf[u], cr, ph);
+            }
+        }
+        if (j) store(j - PL);
+        if (j + PL < np) load(j + PL);
         __syncthreads();
-        for (int c = tid; c < SR * T2; c += 256) {
-            const int r = c / T2, z = c % T2;
+        auto zpass = [&](int c) {
+            const V* row = A + (c / T2) * LR + (DI ? 1 : 2) * (c % T2);   // column 2 z
             V s[K + 1];
 #pragma unroll
-            for (int m = 0; m <= K; m++) s[m] = A[r * SC + 2 * z + K - 1 + rst_tap<K>(m)];
+            for (int m = 0; m <= K; m++) {
+                const int col = K - 1 + rst_tap<K>(m);
+                s[m] = row[!DI ? col : (col & 1) ? SE + (col >> 1) : (col >> 1)];
+            }
             Z[c] = rst_combine<V, K>(s);
+        };
+        if constexpr (DI) {   // every row's reads in flight together
+#pragma unroll
+            for (int k = 0; k < NZ; k++)
+                if (tid + 256 * k < PL * SR * T2) zpass(tid + 256 * k);
+        } else {
+            for (int c = tid; c < PL * SR * T2; c += 256) zpass(c);
         }
         __syncthreads();
-        V y;
-        {
+#pragma unroll
+        for (int u = 0; u < PL; u++) {
             V s[K + 1];
 #pragma unroll
-            for (int m = 0; m <= K; m++) s[m] = Z[(2 * tyi + K - 1 + rst_tap<K>(m)) * T2 + tzi];
-            y = rst_combine<V, K>(s);
-        }
+            for (int m = 0; m <= K; m++)
+                s[m] = Z[(u * SR + 2 * tyi + K - 1 + rst_tap<K>(m)) * T2 + tzi];
+            const V y = rst_combine<V, K>(s);
 #pragma unroll
-        for (int m = 0; m < W - 1; m++) ring[m] = ring[m + 1];
-        ring[W - 1] = y;
+            for (int m = 0; m < W - 1; m++) ring[m] = ring[m + 1];
+            ring[W - 1] = y;
+            if (PL > 1 && u % 2 == 0) xr[u / 2] = xpass();
+        }
     }
-    xpass(np);
+    store(((np - 1) / PL) * PL);
 }
 
 // ----------------------------------------------------------- interpolation
@@ -144,8 +217,11 @@ __global__ __launch_bounds__(256) void k_interp_tile(const V* __restrict__ in, V
     __shared__ V Z[SR * T2];
     const int b = xcd_tile(blockIdx.x, gridDim.x);
     const int tz = b % tt.nt2;
-    const int ty = (b / tt.nt2) % tt.nt1;
-    const int band = b / (tt.nt2 * tt.nt1);
+    int rest = b / tt.nt2;
+    const int ty = rest % tt.nt1;
+    rest /= tt.nt1;
+    const int ch = rest % tt.nch;
+    const int band = rest / tt.nch;
     const int tid = threadIdx.x;
     const int tzi = tid % T2, tyi = tid / T2;
     const V* __restrict__ a = in + (i64)band * t.ngin;
@@ -163,18 +239,21 @@ __global__ __launch_bounds__(256) void k_interp_tile(const V* __restrict__ in, V
     const int c1 = centre(o1, 1), c2 = centre(o2, 2);
     const bool oy = (o1 + t.skip[1][0]) & 1, oz = (o2 + t.skip[2][0]) & 1;
     // z-pass target of this thread's Z entries: fine column z of the tile
-    const int c0f = centre(0, 0);                         // first output's centre
+    const int c0f = centre(0, 0) + ch * tt.cq;            // first centre of the chunk
+    const int c0l = min(c0f + tt.cq - 1, centre(t.nout[0] - 1, 0));   // last one
     const int p0s = c0f - K / 2 + 1;                      // first plane swept
-    const int p0e = centre(t.nout[0] - 1, 0) + K / 2;     // last plane swept
+    const int p0e = c0l + K / 2;                          // last plane swept
     // coarse slab cells of this thread (c = tid + 256 k) with their in-plane
     // references; loaded raw one plane ahead, fixed when stored to LDS
     constexpr int NSI = (SR * SC + 255) / 256;
-    auto cref = [&](int k) -> PlaneRef {
+    PlaneRef cref[NSI];
+#pragma unroll
+    for (int k = 0; k < NSI; k++) {
         const int c = tid + 256 * k;
         const int j1 = r0 + c / SC, j2 = s0 + c % SC;
         const bool ok = c < SR * SC && j1 >= lo1 && j1 < hi1 && j2 >= lo2 && j2 < hi2;
-        return ok ? plane_ref(j1, j2, t.gin) : PREF_ZERO;
-    };
+        cref[k] = ok ? plane_ref(j1, j2, t.gin) : PREF_ZERO;
+    }
     const i64 plane = (i64)t.gin.n[1] * t.gin.n[2];
     auto pflag = [&](int p0, i64& base) -> int {
         const int f = wrap_index(p0, t.gin.n[0], t.gin.per[0]);
@@ -195,7 +274,7 @@ __global__ __launch_bounds__(256) void k_interp_tile(const V* __restrict__ in, V
         i64 base;
         pf = pflag(p0s, base);
 #pragma unroll
-        for (int k = 0; k < NSI; k++) pre[k] = a[base + pref_off(cref(k))];
+        for (int k = 0; k < NSI; k++) pre[k] = a[base + pref_off(cref[k])];
     }
     V ring[K];
     V old[2] = {vzero<V>(), vzero<V>()};   // subtract: outputs' values, loaded a step ahead
@@ -232,13 +311,13 @@ __global__ __launch_bounds__(256) void k_interp_tile(const V* __restrict__ in, V
         }
 #pragma unroll
         for (int k = 0; k < NSI; k++)
-            if (tid + 256 * k < SR * SC) A[tid + 256 * k] = ghost_fix(pre[k], pf, cref(k), ph);
+            if (tid + 256 * k < SR * SC) A[tid + 256 * k] = ghost_fix(pre[k], pf, cref[k], ph);
         opass(p0);
         if (p0 < p0e) {
             i64 base;
             pf = pflag(p0 + 1, base);
 #pragma unroll
-            for (int k = 0; k < NSI; k++) pre[k] = a[base + pref_off(cref(k))];
+            for (int k = 0; k < NSI; k++) pre[k] = a[base + pref_off(cref[k])];
         }
         if (MODE == TR_SUBTRACT && p0 + 1 - p0s >= K) {
 #pragma unroll
@@ -248,7 +327,11 @@ __global__ __launch_bounds__(256) void k_interp_tile(const V* __restrict__ in, V
             }
         }
         __syncthreads();
-        for (int c = tid; c < SR * T2; c += 256) {
+        constexpr int NZ = (SR * T2 + 255) / 256;
+#pragma unroll
+        for (int k = 0; k < NZ; k++) {
+            const int c = tid + 256 * k;
+            if (c >= SR * T2) continue;
             const int r = c / T2, z = c % T2;
             const int fz = tz * T2 + z;
             const int cc = centre(fz, 2) - s0;              // slab column of the centre

@@ -242,6 +242,32 @@ def axpby(y, x, a, b):
     yy.finish()
 
 
+def axpby_shared(y, x, a, b, nin):
+    """y_k = a*y_k + b*x for the nin equal parts y_k of y (float64 device
+    tensors) in one launch."""
+    yy = Arg(y, write=True, name='y', code=_lib.GPAW_F64)
+    xx = Arg(x, name='x', code=_lib.GPAW_F64)
+    n = yy.tensor.numel() // max(nin, 1)
+    if nin and xx.tensor.numel() < n:
+        raise ValueError('axpby_shared: x of shape %s for y of shape %s' % (xx.shape, yy.shape))
+    _lib.check(_lib.lib().gpaw_axpby_shared(yy.ptr, xx.ptr, float(a), float(b), nin, n,
+                                            _arrays.stream()))
+    yy.finish()
+
+
+def renormalize(gd, y, target):
+    """y *= target / np.sum(gd.integrate(y)) on a float64 device tensor of at
+    most 7 functions, without reading the integral back."""
+    yy = Arg(y, write=True, name='y', code=_lib.GPAW_F64)
+    nin = int(np.prod(yy.shape[:-3]))
+    work = _arrays.torch().empty(max(1, nin) * _lib.GPAW_RENORMALIZE_WORK,
+                                 dtype=yy.tensor.dtype, device=yy.tensor.device)
+    _lib.check(_lib.lib().gpaw_renormalize(
+        yy.ptr, nin, int(np.prod(yy.shape[-3:])), float(gd.dv), float(target),
+        work.data_ptr(), _arrays.stream()))
+    yy.finish()
+
+
 def cast(y, x):
     """Precision conversion (float64 <-> float32, complex128 <-> complex64)."""
     yy = Arg(y, write=True)

@@ -332,6 +332,22 @@ int gpaw_dots_noalloc(const double* a, const double* b, long nb, long n,
 int gpaw_axpby(double* y, const double* x, double a, double b, long n,
                void* stream);
 
+/* y_k = a*y_k + b*x for nin functions of n doubles, x shared by them (the
+ * spins' vt_g += vHt_g, gpaw/hamiltonian.py:254-256). */
+int gpaw_axpby_shared(double* y, const double* x, double a, double b, long nin,
+                      long n, void* stream);
+
+/* y *= target / I for nin functions of n doubles, I the sum over them of
+ * scale * sum(y_k): the charge renormalisation of the interpolated density
+ * (gpaw/density.py:230-234) without a readback.  The rounding of gpaw_sum
+ * for each function, the functions added in index order, then gpaw_scale.
+ * work: GPAW_RENORMALIZE_WORK * nin doubles on the device, owned by the
+ * caller. */
+#define GPAW_RENORMALIZE_MAX 7
+#define GPAW_RENORMALIZE_WORK 1024
+int gpaw_renormalize(double* y, long nin, long n, double scale, double target,
+                     double* work, void* stream);
+
 /* y = x - b over n doubles (rho - background, phi -= phi_ave:
  * gpaw/poisson.py:138,216). */
 int gpaw_sub_scalar(double* y, const double* x, double b, long n,
