@@ -5,13 +5,17 @@
 // Transformer holds the restriction / interpolation geometry.  Both are
 // plans only: no grid-sized buffers are allocated except the relax
 // ping-pong scratch and the norm partials, allocated on first use.
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "capi_internal.h"
+#include "stencil_gen.h"
 
 using namespace gpaw;
 
@@ -80,6 +84,54 @@ static int star_range(const Stencil& s)
     return R;
 }
 
+// Reach per axis, and whether the stencil lies along one axis in the order
+// -R..-1, +1..+R (Gradient, gpaw/fd_operators.py:123-144).
+static void stencil_reach(Stencil& s)
+{
+    for (int c = 0; c < s.nc; c++)
+        for (int a = 0; a < 3; a++) s.reach[a] = std::max(s.reach[a], std::abs(s.off[c][a]));
+    s.gen_r = std::max(s.reach[0], std::max(s.reach[1], s.reach[2]));
+    const int R = s.gen_r;
+    if (R < 1 || R > GEN_MAXR || s.nc != 2 * R) return;
+    for (int axis = 0; axis < 3; axis++) {
+        bool line = true;
+        for (int c = 0; c < s.nc && line; c++)
+            for (int a = 0; a < 3; a++)
+                line = line && s.off[c][a] == (a != axis ? 0 : c < R ? c - R : c - R + 1);
+        if (line) s.axis = axis;
+    }
+}
+
+// The device copy of a stencil in one allocation (d_coefs owns it): the
+// coefficients, the terms of k_gen_sweep where it can run, the offsets.
+hipError_t gpaw_stencil_upload(Stencil& s)
+{
+    const bool gen = !s.star_r && s.axis < 0 && s.gen_r >= 1 && s.gen_r <= GEN_MAXR;
+    const size_t nc = s.nc, at_terms = sizeof(double) * nc,
+                 at_off = at_terms + (gen ? sizeof(GenTerm) * nc : 0),
+                 bytes = at_off + sizeof(int) * 3 * nc;
+    std::vector<char> h(bytes);
+    memcpy(h.data(), s.coefs, at_terms);
+    if (gen) {
+        GenTerm* tm = (GenTerm*)(h.data() + at_terms);
+        for (int c = 0; c < s.nc; c++)
+            tm[c] = {s.coefs[c], {(short)s.off[c][0], (short)s.off[c][1], (short)s.off[c][2], 0}};
+    }
+    memcpy(h.data() + at_off, s.off, sizeof(int) * 3 * nc);
+    char* d = nullptr;
+    hipError_t e = hipMalloc((void**)&d, bytes);
+    if (e != hipSuccess) return e;
+    e = hipMemcpy(d, h.data(), bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        hipFree(d);
+        return e;
+    }
+    s.d_coefs = (double*)d;
+    s.d_terms = gen ? (GenTerm*)(d + at_terms) : nullptr;
+    s.d_off = (int*)(d + at_off);
+    return hipSuccess;
+}
+
 extern "C" int gpaw_operator_new(const double* coefs, const long* offsets, int ncoefs,
                                  const long size[3], int range, const long* neighbors, int real,
                                  int cfd, gpaw_operator** out)
@@ -136,13 +188,9 @@ extern "C" int gpaw_operator_new(const double* coefs, const long* offsets, int n
         if (offsets[c] == 0) op->diag = coefs[c];
     s.star_r = star_range(s);
     hipGetDevice(&op->device);
-    if (!s.star_r) {   // device copy of the stencil for the generic kernel
-        hipError_t e = hipMalloc(&s.d_coefs, sizeof(double) * ncoefs);
-        if (e == hipSuccess) e = hipMalloc(&s.d_off, sizeof(int) * 3 * ncoefs);
-        if (e == hipSuccess)
-            e = hipMemcpy(s.d_coefs, s.coefs, sizeof(double) * ncoefs, hipMemcpyHostToDevice);
-        if (e == hipSuccess)
-            e = hipMemcpy(s.d_off, s.off, sizeof(int) * 3 * ncoefs, hipMemcpyHostToDevice);
+    if (!s.star_r) {   // device copy of the stencil for the other kernels
+        stencil_reach(s);
+        hipError_t e = gpaw_stencil_upload(s);
         if (e != hipSuccess) {
             gpaw_operator_free(op);
             return gpaw_check(e, "operator: coefficient upload");
@@ -216,17 +264,10 @@ extern "C" int gpaw_operator_apply_potential(gpaw_operator* op, const void* in, 
     Phases ph;
     gpaw_phases(phases, ph);
     hipStream_t st = (hipStream_t)stream;
-    if (op->st.star_r > 0)   // one pass: out = L in + in * v
-        return gpaw_check(launch_stencil(op->st, dtype, ST_HPSI, in, out, v, op->g, ph, (int)nin,
-                                         0.0, nullptr, nullptr, true, st),
-                          "operator apply_potential");
-    // other stencils: the stencil, then the potential (same arithmetic)
-    hipError_t e = launch_stencil(op->st, dtype, ST_APPLY, in, out, nullptr, op->g, ph, (int)nin,
-                                  0.0, nullptr, nullptr, true, st);
-    if (e == hipSuccess)
-        e = launch_add_potential(out, in, v, nin,
-                                 (long long)op->g.n[0] * op->g.n[1] * op->g.n[2], dtype, st);
-    return gpaw_check(e, "operator apply_potential");
+    // one pass: out = L in + in * v
+    return gpaw_check(launch_stencil(op->st, dtype, ST_HPSI, in, out, v, op->g, ph, (int)nin, 0.0,
+                                     nullptr, nullptr, true, st),
+                      "operator apply_potential");
 }
 
 // Jacobi sweeps on f in place: ping-pong through `scratch`, ending in f.
@@ -267,14 +308,7 @@ extern "C" int gpaw_operator_relax(gpaw_operator* op, int method, double* f, con
     if (rc) return rc;
     if (method == 1) {
         if (!op->st.d_coefs) {   // star stencils upload their table on first use
-            hipError_t e = hipMalloc(&op->st.d_coefs, sizeof(double) * op->st.nc);
-            if (e == hipSuccess) e = hipMalloc(&op->st.d_off, sizeof(int) * 3 * op->st.nc);
-            if (e == hipSuccess)
-                e = hipMemcpy(op->st.d_coefs, op->st.coefs, sizeof(double) * op->st.nc,
-                              hipMemcpyHostToDevice);
-            if (e == hipSuccess)
-                e = hipMemcpy(op->st.d_off, op->st.off, sizeof(int) * 3 * op->st.nc,
-                              hipMemcpyHostToDevice);
+            hipError_t e = gpaw_stencil_upload(op->st);
             if (e != hipSuccess) return gpaw_check(e, "relax: stencil upload");
         }
         return gpaw_op_gauss_seidel(op, f, s, nrelax, op->scratch, (hipStream_t)stream);
@@ -317,7 +351,6 @@ extern "C" void gpaw_operator_free(gpaw_operator* op)
 {
     if (!op) return;
     if (op->st.d_coefs) hipFree(op->st.d_coefs);
-    if (op->st.d_off) hipFree(op->st.d_off);
     if (op->scratch) hipFree(op->scratch);
     if (op->partial) hipFree(op->partial);
     delete op;

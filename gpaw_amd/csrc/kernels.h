@@ -72,6 +72,12 @@ constexpr bool st_norm_ok()
 #define GPAW_MAXC 512
 #define GPAW_MAXR 6
 
+// One term of a stencil on the device, for k_gen_sweep (stencil_gen.h).
+struct GenTerm {
+    double c;
+    short d[4];   // offset per axis; d[3] unused
+};
+
 // A stencil: coefficients in the caller's order (the summation order) and
 // integer offsets.  `star` marks the canonical order of an orthogonal-cell
 // Laplacian, [centre, +1..+R along axis 2, -1..-R along 2, then axis 1,
@@ -82,8 +88,16 @@ struct Stencil {
     int star_r = 0;                 // R of the canonical star order, 0 if not
     double coefs[GPAW_MAXC];
     int off[GPAW_MAXC][3];
-    double* d_coefs = nullptr;      // device copies for the generic kernel
+    double* d_coefs = nullptr;      // device copies for the generic kernel, in
+                                    // one allocation that d_coefs owns
     int* d_off = nullptr;
+    // other stencils (stencil_gen.h): reach per axis and the largest of them;
+    // the axis of a stencil along one axis in the order -R..-1, +1..+R (-1:
+    // none); device terms (null: reach beyond GEN_MAXR, or a star)
+    int reach[3] = {0, 0, 0};
+    int gen_r = 0;
+    int axis = -1;
+    GenTerm* d_terms = nullptr;
 };
 
 // Stencil launch-shape autotuner (stencil.hip): switch on (1) / off (0), or

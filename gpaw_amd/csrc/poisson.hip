@@ -426,14 +426,7 @@ extern "C" int gpaw_poisson_new(int levels, gpaw_operator* const* ops,
     for (int l = 0; l <= levels && !rc && relax_method == 1; l++) {
         gpaw_operator* op = ps->ops[l];
         if (!op->st.d_coefs) {   // Gauss-Seidel reads the stencil table on the device
-            hipError_t e = hipMalloc(&op->st.d_coefs, sizeof(double) * op->st.nc);
-            if (e == hipSuccess) e = hipMalloc(&op->st.d_off, sizeof(int) * 3 * op->st.nc);
-            if (e == hipSuccess)
-                e = hipMemcpy(op->st.d_coefs, op->st.coefs, sizeof(double) * op->st.nc,
-                              hipMemcpyHostToDevice);
-            if (e == hipSuccess)
-                e = hipMemcpy(op->st.d_off, op->st.off, sizeof(int) * 3 * op->st.nc,
-                              hipMemcpyHostToDevice);
+            hipError_t e = gpaw_stencil_upload(op->st);
             rc = gpaw_check(e, "poisson: stencil upload");
         }
     }

@@ -13,8 +13,9 @@
 //    read from HBM once.  In-plane neighbours come from the same plane rows
 //    that the neighbouring lanes / waves of the block load (L1/L2 hits).
 //    Waves are 64 lanes along i2, so every HBM access is a coalesced row.
-//  * k_generic: any stencil (non-orthogonal cells, Mehrstellen, gradients):
-//    one thread per point, coefficients read through the scalar cache.
+//  * k_generic: any stencil, one thread per point, coefficients read through
+//    the scalar cache; kept for passes with partial sums and for grids and
+//    stencils that the kernels of stencil_gen.h do not take.
 // Both fuse the residual (apply - rho) and an FP64 sum of |result|^2 per
 // block (deterministic tree order) for the multigrid convergence test.
 #include <algorithm>
@@ -50,6 +51,16 @@ hipError_t tile_launch_f32(const Stencil&, int, const void*, void*, const void*,
                           const Phases&, double, int, const TileShape&, double*, bool, hipStream_t);
 hipError_t tile_launch_c64(const Stencil&, int, const void*, void*, const void*, const Geom&,
                           const Phases&, double, int, const TileShape&, double*, bool, hipStream_t);
+
+// other stencils, without partial sums (stencil_gen.h)
+hipError_t gen_launch_f64(const Stencil&, int, const void*, void*, const void*, const Geom&,
+                          const Phases&, int, double, hipStream_t, bool*);
+hipError_t gen_launch_c128(const Stencil&, int, const void*, void*, const void*, const Geom&,
+                           const Phases&, int, double, hipStream_t, bool*);
+hipError_t gen_launch_f32(const Stencil&, int, const void*, void*, const void*, const Geom&,
+                          const Phases&, int, double, hipStream_t, bool*);
+hipError_t gen_launch_c64(const Stencil&, int, const void*, void*, const void*, const Geom&,
+                          const Phases&, int, double, hipStream_t, bool*);
 
 struct StarCoefs {
     double c[6 * GPAW_MAXR + 1];
@@ -864,6 +875,20 @@ hipError_t launch_stencil(const Stencil& s, int dtype, int mode, const void* in,
     // sweep come from the tile and box kernels only
     if (partial && (mode == ST_APPLY || mode == ST_JACOBI) && c.kind != K_TILE && c.kind != K_BOX)
         return hipErrorInvalidValue;
+    // stencils without a star form; partial sums (whose layout the callers
+    // size) and a forced generic kernel keep k_generic
+    if (c.kind == K_GENERIC && !s.star_r && !partial && ov != K_GENERIC &&
+        forced_kind() != K_GENERIC) {
+        bool handled = false;
+        hipError_t e = hipSuccess;
+        switch (dtype) {
+        case DT_F64: e = gen_launch_f64(s, mode, in, out, aux, g, ph, nin, w, st, &handled); break;
+        case DT_C128: e = gen_launch_c128(s, mode, in, out, aux, g, ph, nin, w, st, &handled); break;
+        case DT_F32: e = gen_launch_f32(s, mode, in, out, aux, g, ph, nin, w, st, &handled); break;
+        case DT_C64: e = gen_launch_c64(s, mode, in, out, aux, g, ph, nin, w, st, &handled); break;
+        }
+        if (handled || e != hipSuccess) return e;
+    }
     return launch_cfg(c, s, dtype, mode, in, out, aux, g, ph, nin, w, partial, write, st);
 }
 

@@ -1,0 +1,13 @@
+// stencil_gen.h instantiations for double2 grid functions.
+#include "stencil_gen_impl.h"
+
+namespace gpaw {
+
+hipError_t gen_launch_c128(const Stencil& s, int mode, const void* in, void* out, const void* aux,
+                        const Geom& g, const Phases& ph, int nin, double w, hipStream_t st,
+                        bool* handled)
+{
+    return gen_launch<double2>(s, mode, in, out, aux, g, ph, nin, w, st, handled);
+}
+
+}  // namespace gpaw
