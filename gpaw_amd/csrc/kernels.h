@@ -184,6 +184,7 @@ struct Transfer {
     int nout[3];
     int lo[3];           // low padding per axis (maps output to input index)
     int skip[3][2];
+    int negate = 0;      // restriction: out = -T(in)
 };
 
 enum TransferMode {

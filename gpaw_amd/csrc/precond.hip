@@ -1,6 +1,6 @@
 // Multigrid preconditioner of the finite-difference eigensolvers
-// (gpaw/preconditioner.py:13-70) as one stream-ordered sequence of ten
-// launches over all bands at once.
+// (gpaw/preconditioner.py:13-70) as one stream-ordered sequence of launches
+// over all bands at once.
 //
 // The reference evaluates, per call (r = residuals, s = step):
 //   r1 = R0(-r);  d1 = 4s r1;  q1 = L1 d1 - r1
@@ -15,25 +15,133 @@
 // Every value is rounded exactly where the reference's numpy / BLAS steps
 // round it (BLAS axpy evaluated as y + (a x), without a fused multiply-add).
 //
+// Six launches where the levels allow it (pc_scaled, pc_interp): d1 = 4s r1, d2 = 16s r2,
+// d1 - I2(d2) and e0 = I1(d1) are formed inside the stencil passes that read
+// them (precond_sweep.h), so E0, D1 and D2 are never stored; 4.3 instead of
+// 7.4 GB on 256 complex128 bands of 64^3.  A pass that cannot be fused runs
+// its steps one by one.
+//
 // Buffers (caller's workspace, one slice per band, 256-byte aligned):
 //   level 0: E0;  level 1: R1, D1, Q1;  level 2: R2, D2, X2.
 #include "capi_internal.h"
+#include "precond_sweep.h"
 
 namespace gpaw {
 
-// r = -r (if neg); d = c * r, over n doubles (complex data counted as pairs)
-__global__ __launch_bounds__(256) void k_pc_scale(double* __restrict__ r, double* __restrict__ d,
-                                                  double c, i64 n, int neg)
+// d = c * r over n doubles (complex data counted as pairs)
+__global__ __launch_bounds__(256) void k_pc_scale(const double* __restrict__ r,
+                                                  double* __restrict__ d, double c, i64 n)
 {
     const i64 i = (i64)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    double v = r[i];
-    if (neg) {
-        v = -v;
-        r[i] = v;
-    }
-    d[i] = c * v;
+    if (i < n) d[i] = c * r[i];
 }
+
+namespace {
+
+// Runs of the whole i0 axis, split where there are too few tiles (a run of
+// k_pc_interp starts with R + 1 coarse planes, each two barriers).
+bool pc_shape(const Geom& g, int R, int esize, int nin, int nt, TileShape* sh)
+{
+    if (!tile_geometry(g, R, esize, nin, 32, g.n[0], *sh, nt)) return false;
+    long nch = (1024L + sh->nblocks - 1) / sh->nblocks;
+    const long maxch = g.n[0] / 8 > 1 ? g.n[0] / 8 : 1;
+    if (nch > maxch) nch = maxch;
+    return tile_geometry(g, R, esize, nin, 32, (int)((g.n[0] + nch - 1) / nch), *sh, nt);
+}
+
+TileCoefs pc_coefs(const Stencil& s)
+{
+    TileCoefs sc{};
+    for (int c = 0; c < 6 * s.star_r + 1; c++) sc.c[c] = s.coefs[c];
+    return sc;
+}
+
+i64 pc_points(const int n[3]) { return (i64)n[0] * n[1] * n[2]; }
+
+// out = mode(L F, aux b) with F = c b; hipErrorNotSupported (nothing launched)
+// where k_pc_scaled cannot run: it takes range-1 stars whose halo wraps once.
+template <class V>
+hipError_t pc_scaled(const gpaw_operator* L, int mode, const void* b, void* out, int nin,
+                     const Phases& ph, double cb, double w, hipStream_t st)
+{
+    TileShape sh;
+    if (L->st.star_r != 1 || !pc_shape(L->g, 1, (int)sizeof(V), nin, TILE_NT, &sh))
+        return hipErrorNotSupported;
+    const dim3 grid(sh.nblocks), block(32, TILE_NT / 32);
+    const TileCoefs sc = pc_coefs(L->st);
+    const i64 ng = pc_points(L->g.n);
+    if (mode == ST_RESID)
+        return launch_kernel((k_pc_scaled<V, 1, ST_RESID, TILE_NT>), grid, block, 0, st,
+                             (const V*)b, (V*)out, L->g, ph, sc, cb, w, sh, ng);
+    return launch_kernel((k_pc_scaled<V, 1, ST_PCUPD, TILE_NT>), grid, block, 0, st, (const V*)b,
+                         (V*)out, L->g, ph, sc, cb, w, sh, ng);
+}
+
+// out = mode(L F, aux) with F = I e (b null) or c b - I e; hipErrorNotSupported
+// where k_pc_interp cannot run: it takes K = 2, stars of range 1 .. 3 (1 with
+// b), halos that wrap once, and on periodic axes grids twice the coarser one.
+template <class V, int R, bool BASE, int MODE, int TY>
+hipError_t pc_interp_go(const gpaw_operator* L, const Transfer& t, const void* b, const void* e,
+                        void* out, const void* aux, int nin, const Phases& ph, double cb, double w,
+                        hipStream_t st)
+{
+    const Geom& g = L->g;
+    TileShape sh;
+    if (!pc_shape(g, R, (int)sizeof(V), nin, 32 * TY, &sh)) return hipErrorNotSupported;
+    PcCoarse pc;
+    for (int a = 0; a < 3; a++) {
+        pc.nc[a] = t.gin.n[a];
+        pc.skip[a] = t.skip[a][0];
+        pc.lo[a] = t.lo[a];
+    }
+    return launch_kernel((k_pc_interp<V, R, BASE, MODE, TY>), dim3(sh.nblocks), dim3(32, TY), 0, st,
+                         (const V*)b, (const V*)e, (V*)out, (const V*)aux, g, ph, pc,
+                         pc_coefs(L->st), cb, w, sh, pc_points(g.n), pc_points(pc.nc));
+}
+
+template <class V>
+hipError_t pc_interp(const gpaw_operator* L, const Transfer& t, const void* b, const void* e,
+                     void* out, const void* aux, int nin, const Phases& ph, double cb, double w,
+                     hipStream_t st)
+{
+    const Geom& g = L->g;
+    const int R = L->st.star_r;
+    if (t.K != 2 || R < 1 || R > (b ? 1 : 3)) return hipErrorNotSupported;
+    for (int a = 0; a < 3; a++) {
+        if (t.nout[a] != g.n[a] || t.gin.per[a] != g.per[a] || g.n[a] < 2 * R + 2)
+            return hipErrorNotSupported;
+        if (g.per[a] && (t.nout[a] != 2 * t.gin.n[a] || t.skip[a][0] || t.lo[a]))
+            return hipErrorNotSupported;
+    }
+    const i64 points = nin * pc_points(g.n);
+    // complex bands below 2^18 points in all: every launch is a few us there, and
+    // a block's serial planes cost more than the launch saved (1 / 4 / 16 bands
+    // of 32^3: 49.5 / 53 / 55 us fused, 46 / 50 / 58 in steps; real bands gain at
+    // every size measured)
+    if (VT<V>::cplx && points < 1 << 18) return hipErrorNotSupported;
+    // 16 rows per block on large sets where they pad no more rows than 8 do
+    // (complex128, 256 x 64^3: 1075 us a call with 8, 1001 with 16, 1009 with 32
+    // rows; 64 x 32^3: 90 with 8, 82 with 16; real 16 x 48^3: 47 with 8, 50 with 16)
+    const bool tall = points >= 1 << 21 && (g.n[1] + 15) / 16 * 2 == (g.n[1] + 7) / 8;
+    hipError_t r = hipErrorNotSupported;
+#define GPAW_PC_INTERP(RR, B, M)                                                                  \
+    if (tall) r = pc_interp_go<V, RR, B, M, 16>(L, t, b, e, out, aux, nin, ph, cb, w, st);        \
+    if (r == hipErrorNotSupported)                                                                \
+        r = pc_interp_go<V, RR, B, M, 8>(L, t, b, e, out, aux, nin, ph, cb, w, st);
+    if (b) {
+        GPAW_PC_INTERP(1, true, ST_PCUPD)
+    } else if (R == 1) {
+        GPAW_PC_INTERP(1, false, ST_PCFIN)
+    } else if (R == 2) {
+        GPAW_PC_INTERP(2, false, ST_PCFIN)
+    } else {
+        GPAW_PC_INTERP(3, false, ST_PCFIN)
+    }
+#undef GPAW_PC_INTERP
+    return r;
+}
+
+}  // namespace
 
 }  // namespace gpaw
 
@@ -151,10 +259,10 @@ extern "C" int gpaw_preconditioner_apply(gpaw_preconditioner* pc, const void* re
     Phases ph;
     gpaw_phases(phases, ph);
     const int nb = (int)nin;
-    char* w = (char*)work;
+    char* free_ = (char*)work;
     auto take = [&](int l) {
-        void* p = w;
-        w += slice_bytes(pc->ng[l], nin, dtype);
+        void* p = free_;
+        free_ += slice_bytes(pc->ng[l], nin, dtype);
         return p;
     };
     void* E0 = take(0);
@@ -169,34 +277,66 @@ extern "C" int gpaw_preconditioner_apply(gpaw_preconditioner* pc, const void* re
     const double s = pc->step, c1 = 4 * s, c2 = 16 * s;
     gpaw_operator *L0 = pc->kin[0], *L1 = pc->kin[1], *L2 = pc->kin[2];
 
-    hipError_t e = launch_transfer(pc->rst[0]->t, dtype, TR_STORE, residuals, R1, nullptr, ph, nb, st);
-    if (e == hipSuccess) {   // r1 = -R0(r), d1 = 4s r1
-        launch_kernel(k_pc_scale, dim3((unsigned)((n1 + 255) / 256)), dim3(256), 0, st,
-                           (double*)R1, (double*)D1, c1, n1, 1);
-        e = launch_error();
+    hipError_t e;
+    auto scale = [&](const void* r, void* d, double c, i64 n) {
+        return launch_kernel(k_pc_scale, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
+                             (const double*)r, (double*)d, c, n);
+    };
+    auto stencil = [&](const gpaw_operator* L, int mode, const void* in, void* o, const void* aux,
+                       double c) {
+        return launch_stencil(L->st, dtype, mode, in, o, aux, L->g, ph, nb, c, nullptr, nullptr,
+                              true, st);
+    };
+    auto transfer = [&](const Transfer& t, int mode, const void* in, void* o) {
+        return launch_transfer(t, dtype, mode, in, o, nullptr, ph, nb, st);
+    };
+    // the passes in one launch each or, where those kernels cannot run one
+    // (hipErrorNotSupported, nothing launched), in its separate steps
+    const bool real = !dtype_complex(dtype);
+    auto scaled = [&](const gpaw_operator* L, int mode, const void* b, void* o, double c) {
+        return real ? pc_scaled<double>(L, mode, b, o, nb, ph, c, c, st)
+                    : pc_scaled<double2>(L, mode, b, o, nb, ph, c, c, st);
+    };
+    auto interp = [&](const gpaw_operator* L, const Transfer& t, const void* b, const void* x,
+                      void* o, const void* aux, double c, double w) {
+        return real ? pc_interp<double>(L, t, b, x, o, aux, nb, ph, c, w, st)
+                    : pc_interp<double2>(L, t, b, x, o, aux, nb, ph, c, w, st);
+    };
+    bool d1 = false;   // D1 = 4s r1
+    Transfer rneg = pc->rst[0]->t;
+    rneg.negate = 1;
+    e = transfer(rneg, TR_STORE, residuals, R1);   // r1 = -R0(r)
+    if (e == hipSuccess) {   // q1 = L1 d1 - r1, d1 = 4s r1
+        e = scaled(L1, ST_RESID, R1, Q1, c1);
+        if (e == hipErrorNotSupported) {
+            d1 = true;
+            e = scale(R1, D1, c1, n1);
+            if (e == hipSuccess) e = stencil(L1, ST_RESID, D1, Q1, R1, 0.0);
+        }
     }
-    if (e == hipSuccess)   // q1 = L1 d1 - r1
-        e = launch_stencil(L1->st, dtype, ST_RESID, D1, Q1, R1, L1->g, ph, nb, 0.0, nullptr,
-                           nullptr, true, st);
-    if (e == hipSuccess) e = launch_transfer(pc->rst[1]->t, dtype, TR_STORE, Q1, R2, nullptr, ph, nb, st);
-    if (e == hipSuccess) {   // d2 = 16s r2
-        launch_kernel(k_pc_scale, dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0, st,
-                           (double*)R2, (double*)D2, c2, n2, 0);
-        e = launch_error();
+    if (e == hipSuccess) e = transfer(pc->rst[1]->t, TR_STORE, Q1, R2);   // r2 = R1(q1)
+    if (e == hipSuccess) {   // x2 = d2 - 16s (L2 d2 - r2), d2 = 16s r2
+        e = scaled(L2, ST_PCUPD, R2, X2, c2);
+        if (e == hipErrorNotSupported) {
+            e = scale(R2, D2, c2, n2);
+            if (e == hipSuccess) e = stencil(L2, ST_PCUPD, D2, X2, R2, c2);
+        }
     }
-    if (e == hipSuccess)   // d2 - 16s (L2 d2 - r2)
-        e = launch_stencil(L2->st, dtype, ST_PCUPD, D2, X2, R2, L2->g, ph, nb, c2, nullptr,
-                           nullptr, true, st);
-    if (e == hipSuccess)   // d1 -= I2(d2)
-        e = launch_transfer(pc->ip[0]->t, dtype, TR_SUBTRACT, X2, D1, nullptr, ph, nb, st);
-    if (e == hipSuccess)   // d1 - 4s (L1 d1 - r1)
-        e = launch_stencil(L1->st, dtype, ST_PCUPD, D1, Q1, R1, L1->g, ph, nb, c1, nullptr,
-                           nullptr, true, st);
-    if (e == hipSuccess)   // e0 = I1(d1) = -d0
-        e = launch_transfer(pc->ip[1]->t, dtype, TR_STORE, Q1, E0, nullptr, ph, nb, st);
-    if (e == hipSuccess)   // e0 - s (L0 e0 + r)
-        e = launch_stencil(L0->st, dtype, ST_PCFIN, E0, out, residuals, L0->g, ph, nb, s, nullptr,
-                           nullptr, true, st);
+    if (e == hipSuccess) {   // q = d1 - 4s (L1 d1 - r1), d1 = 4s r1 - I2(x2)
+        e = interp(L1, pc->ip[0]->t, R1, X2, Q1, R1, c1, c1);
+        if (e == hipErrorNotSupported) {
+            e = d1 ? hipSuccess : scale(R1, D1, c1, n1);
+            if (e == hipSuccess) e = transfer(pc->ip[0]->t, TR_SUBTRACT, X2, D1);
+            if (e == hipSuccess) e = stencil(L1, ST_PCUPD, D1, Q1, R1, c1);
+        }
+    }
+    if (e == hipSuccess) {   // e0 - s (L0 e0 + r), e0 = I1(q) = -d0
+        e = interp(L0, pc->ip[1]->t, nullptr, Q1, out, residuals, 0.0, s);
+        if (e == hipErrorNotSupported) {
+            e = transfer(pc->ip[1]->t, TR_STORE, Q1, E0);
+            if (e == hipSuccess) e = stencil(L0, ST_PCFIN, E0, out, residuals, s);
+        }
+    }
     return gpaw_check(e, "preconditioner apply");
 }
 

@@ -17,6 +17,7 @@ TrArgs make_trargs(const Transfer& tr)
 {
     TrArgs t;
     t.gin = tr.gin;
+    t.negate = tr.negate;
     for (int a = 0; a < 3; a++) {
         t.nout[a] = tr.nout[a];
         t.lo[a] = tr.lo[a];

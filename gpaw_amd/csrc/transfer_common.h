@@ -44,8 +44,15 @@ struct TrArgs {
     int nout[3];
     int lo[3];
     int skip[3][2];
+    int negate;
     i64 ngin, ngout;
 };
+
+template <class V>
+__device__ __forceinline__ V neg_if(V v, int neg)
+{
+    return neg ? vmul(v, (typename VT<V>::R)-1) : v;
+}
 
 // restriction taps of one axis: s[0] centre, s[2j-1] = +(2j-1), s[2j] = -(2j-1)
 template <class V, int K>

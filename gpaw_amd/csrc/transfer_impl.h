@@ -29,7 +29,7 @@ __global__ __launch_bounds__(256) void k_restrict(const V* __restrict__ in, V* _
     const int o0 = (int)(idx / ((i64)t.nout[1] * t.nout[2]));
     const V* __restrict__ a = in + (i64)blockIdx.y * t.ngin;
     const i64 o = (i64)blockIdx.y * t.ngout + idx;
-    out[o] = restrict_point<V, K>(a, o0, o1, o2, t, ph);
+    out[o] = neg_if(restrict_point<V, K>(a, o0, o1, o2, t, ph), t.negate);
     if (zero_out) zero_out[o] = vzero<V>();
 }
 

@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void k_restrict_tile(const V* __restrict__ in,
         V s[K + 1];
 #pragma unroll
         for (int m = 0; m <= K; m++) s[m] = ring[K - 1 + rst_tap<K>(m)];
-        return rst_combine<V, K>(s);
+        return neg_if(rst_combine<V, K>(s), t.negate);
     };
     // outputs of the step that began at plane j, stored with the next step's
     // loads; a one-plane step leaves its x-pass to this point too

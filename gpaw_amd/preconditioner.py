@@ -4,7 +4,7 @@ Same constructor, allocate() and __call__(residuals, kpt) as the reference
 class (gpaw/preconditioner.py:13-70): two coarser grids with nn=1 kinetic
 operators and nn=1 transformers, one damped Jacobi-like step per level.
 The whole sequence for all bands runs inside libgpaw_amd.so
-(gpaw_preconditioner_apply): ten launches per call instead of the
+(gpaw_preconditioner_apply): six to ten launches per call instead of the
 reference's per-block operator calls and numpy temporaries.
 
 As in the reference, the returned array is the preconditioner's own

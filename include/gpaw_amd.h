@@ -209,7 +209,7 @@ void gpaw_poisson_free(gpaw_poisson* ps);
  * Replaces the Python class Preconditioner (gpaw/preconditioner.py:13-70),
  * whose __call__ drives _gpaw.Operator / _gpaw.Transformer objects and
  * numpy updates band-block by band-block; here the whole sequence runs on
- * the device for all nin bands in ten launches.  kin0 is the fine-grid
+ * the device for all nin bands in six to ten launches.  kin0 is the fine-grid
  * kinetic operator, kin1 / kin2 the nn=1 Laplacians (scale -0.5) of the two
  * coarser grids, restrictor0/1 and interpolator2/1 the nn=1 transformers
  * 0->1, 1->2, 2->1, 1->0 (gpaw/preconditioner.py:14-31).  All are borrowed

@@ -93,3 +93,48 @@ def test_preconditioner_reuses_buffers_across_band_counts():
         res = rng.standard_normal((nb,) + N) + 1j * rng.standard_normal((nb,) + N)
         got = pc(torch.from_numpy(res).cuda(), _Kpt(ph)).cpu().numpy()
         assert np.array_equal(got, ref(res, ph)), nb
+
+
+FUSED = [
+    # N, pbc, dtype, bands, nn0: tiles of 8 and 16 rows, partial tiles, runs
+    # that start on either parity, halos across every kind of boundary
+    ((36, 28, 44), True, complex, 8, 3),
+    ((28, 36, 52), (True, False, True), complex, 8, 3),
+    ((44, 28, 40), (False, True, False), complex, 7, 2),
+    ((40, 36, 36), False, complex, 8, 1),
+    ((32, 32, 36), True, complex, 60, 3),
+    ((36, 36, 68), False, float, 30, 3),
+    ((36, 28, 44), True, float, 3, 3),
+    ((28, 28, 36), (False, True, True), float, 2, 2),
+    ((20, 24, 20), False, float, 1, 1),
+]
+
+
+@pytest.mark.parametrize('N,pbc,dtype,nb,nn0', FUSED)
+def test_fused_passes(N, pbc, dtype, nb, nn0):
+    """The passes over scaled and interpolated fields: the first and last band
+    against the oracle, and every band against the same band alone (which for
+    complex data runs the passes step by step)."""
+    print('case precond fused', N, pbc, dtype.__name__, nb, nn0, flush=True)
+    torch = _torch()
+    from gpaw_amd.grid_descriptor import GridDescriptor
+    from gpaw_amd.fd_operators import Laplace
+    from gpaw_amd.preconditioner import Preconditioner
+    cell = np.array(N) * 0.2
+    og, gd = O.Grid(N, cell, pbc), GridDescriptor(N, cell, pbc)
+    ref = O.Preconditioner(og, O.laplace(og, -0.5, nn0, dtype), dtype)
+    pc = Preconditioner(gd, Laplace(gd, -0.5, nn0, dtype), dtype, block=nb)
+    rng = np.random.default_rng(sum(N) + nb)
+    shape = (nb,) + tuple(og.n_c)
+    res = rng.standard_normal(shape)
+    ph = kpt = None
+    if dtype == complex:
+        res = res + 1j * rng.standard_normal(shape)
+        ph = og.phase_cd(np.where(gd.pbc_c, (0.15, -0.3, 0.4), 0.0))
+        kpt = _Kpt(ph)
+    x = torch.from_numpy(res).cuda()
+    got = pc(x, kpt).clone()
+    ends = sorted({0, nb - 1})
+    assert np.array_equal(got[ends].cpu().numpy(), ref(res[ends], ph))
+    for n in range(nb):
+        assert torch.equal(pc(x[n:n + 1], kpt)[0], got[n])
