@@ -26,7 +26,9 @@ SOURCES = ['stencil.hip', 'stencil_tile_f64.hip', 'stencil_tile_c128.hip',
            'precond.hip', 'batch.hip', 'batch_f64.hip', 'batch_c128.hip',
            'batch_f32.hip', 'batch_c64.hip', 'jacobi_fused.hip',
            'resid_restrict.hip', 'jacobi_corr.hip', 'stencil_gen_f64.hip',
-           'stencil_gen_c128.hip', 'stencil_gen_f32.hip', 'stencil_gen_c64.hip']
+           'stencil_gen_c128.hip', 'stencil_gen_f32.hip', 'stencil_gen_c64.hip',
+           'stencil_pair_f64.hip', 'stencil_pair_c128.hip', 'stencil_pair_f32.hip',
+           'stencil_pair_c64.hip']
 
 FLAGS = ['-O3', '-std=c++17', '-fPIC', '--offload-arch=' + ARCH,
          '-ffp-contract=off', '-Xclang', '-target-feature', '-Xclang',

@@ -59,12 +59,16 @@ TileCoefs pc_coefs(const Stencil& s)
 i64 pc_points(const int n[3]) { return (i64)n[0] * n[1] * n[2]; }
 
 // out = mode(L F, aux b) with F = c b; hipErrorNotSupported (nothing launched)
-// where k_pc_scaled cannot run: it takes range-1 stars whose halo wraps once.
+// where k_pc_scaled does not run: it takes range-1 stars whose halo wraps once,
+// complex data from 2^15 points in all (below, one tile's serial planes take
+// longer than the two short launches: 8 bands of 13 x 11 x 17, a call of 48
+// instead of 44 us).
 template <class V>
 hipError_t pc_scaled(const gpaw_operator* L, int mode, const void* b, void* out, int nin,
                      const Phases& ph, double cb, double w, hipStream_t st)
 {
     TileShape sh;
+    if (VT<V>::cplx && nin * pc_points(L->g.n) < 1 << 15) return hipErrorNotSupported;
     if (L->st.star_r != 1 || !pc_shape(L->g, 1, (int)sizeof(V), nin, TILE_NT, &sh))
         return hipErrorNotSupported;
     const dim3 grid(sh.nblocks), block(32, TILE_NT / 32);
@@ -116,9 +120,13 @@ hipError_t pc_interp(const gpaw_operator* L, const Transfer& t, const void* b, c
     const i64 points = nin * pc_points(g.n);
     // complex bands below 2^18 points in all: every launch is a few us there, and
     // a block's serial planes cost more than the launch saved (1 / 4 / 16 bands
-    // of 32^3: 49.5 / 53 / 55 us fused, 46 / 50 / 58 in steps; real bands gain at
-    // every size measured)
-    if (VT<V>::cplx && points < 1 << 18) return hipErrorNotSupported;
+    // of 32^3: 49.5 / 53 / 55 us fused, 46 / 50 / 58 in steps).  Real bands gain
+    // there (a call is bound by the host), but lose on few tiles of many planes
+    // (3 bands of 79 x 63 x 71, 72 tiles: 47 against 44.5 us; 16 of 48^3, 192
+    // tiles: 47 against 52.6).
+    const i64 tiles = (i64)((g.n[1] + 7) / 8) * ((g.n[2] + 31) / 32) * nin;
+    if (VT<V>::cplx ? points < 1 << 18 : points >= 1 << 18 && tiles < 128)
+        return hipErrorNotSupported;
     // 16 rows per block on large sets where they pad no more rows than 8 do
     // (complex128, 256 x 64^3: 1075 us a call with 8, 1001 with 16, 1009 with 32
     // rows; 64 x 32^3: 90 with 8, 82 with 16; real 16 x 48^3: 47 with 8, 50 with 16)

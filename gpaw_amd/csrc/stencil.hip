@@ -30,6 +30,7 @@
 
 #include "kernels.h"
 #include "stencil_box.h"
+#include "stencil_pair.h"
 #include "stencil_tile.h"
 
 namespace gpaw {
@@ -51,6 +52,15 @@ hipError_t tile_launch_f32(const Stencil&, int, const void*, void*, const void*,
                           const Phases&, double, int, const TileShape&, double*, bool, hipStream_t);
 hipError_t tile_launch_c64(const Stencil&, int, const void*, void*, const void*, const Geom&,
                           const Phases&, double, int, const TileShape&, double*, bool, hipStream_t);
+
+hipError_t pair_launch_f64(const Stencil&, int, const void*, void*, const void*, const Geom&,
+                           const Phases&, double, int, const TileShape&, hipStream_t);
+hipError_t pair_launch_c128(const Stencil&, int, const void*, void*, const void*, const Geom&,
+                            const Phases&, double, int, const TileShape&, hipStream_t);
+hipError_t pair_launch_f32(const Stencil&, int, const void*, void*, const void*, const Geom&,
+                           const Phases&, double, int, const TileShape&, hipStream_t);
+hipError_t pair_launch_c64(const Stencil&, int, const void*, void*, const void*, const Geom&,
+                           const Phases&, double, int, const TileShape&, hipStream_t);
 
 // other stencils, without partial sums (stencil_gen.h)
 hipError_t gen_launch_f64(const Stencil&, int, const void*, void*, const void*, const Geom&,
@@ -350,7 +360,7 @@ hipError_t dispatch_mode(bool star, const Stencil& s, int mode, const void* in, 
 // data on grids that sit in the caches, the LDS tile kernel on other large
 // grids, the register-queue kernel on other star stencils, the generic one
 // otherwise.
-enum { K_GENERIC = 0, K_QUEUE = 1, K_TILE = 2, K_BOX = 3 };
+enum { K_GENERIC = 0, K_QUEUE = 1, K_TILE = 2, K_BOX = 3, K_PAIR = 4 };
 
 static int forced_kind()
 {
@@ -401,7 +411,7 @@ int stencil_kernel_set(int kind)
 
 static const char* kind_name(int k)
 {
-    return k == K_TILE ? "tile" : k == K_BOX ? "box" : k == K_QUEUE ? "queue" : "generic";
+    return k == K_TILE ? "tile" : k == K_PAIR ? "pair" : k == K_BOX ? "box" : k == K_QUEUE ? "queue" : "generic";
 }
 
 // Box kernel shapes (stencil_box.h): 32 x 8 columns, Q planes per block.
@@ -548,6 +558,119 @@ bool tile_shape(const Geom& g, int R, int esize, int nin, int& TZ, TileShape& sh
     return (long)sh.nblocks * nt >= 256L * TILE_NT;
 }
 
+// One launch configuration: the kernel kind and, for tiles, the shape.
+struct LaunchCfg {
+    int kind;
+    int TZ;
+    TileShape sh;
+};
+
+// Tiles of TZ columns and runs of q planes of the pair kernel (compiled for
+// applies, and with the potential in FP64); false if it cannot run the launch.
+static bool pair_geometry(const Stencil& s, const Geom& g, int dtype, int mode, int nin, int TZ,
+                          int q, TileShape& sh)
+{
+    const int R = s.star_r, esize = dtype_size(dtype);
+    if (R < 1 || R > 3 || q < 1 || nin < 1) return false;
+    if (mode != ST_APPLY && !(mode == ST_HPSI && (dtype == DT_F64 || dtype == DT_C128)))
+        return false;
+    if (TZ != 32 && TZ != 48 && TZ != 64 && !(TZ == 96 && esize < 16)) return false;
+    sh.nt = TZ * PAIR_TY;
+    sh.ntz = (g.n[2] + TZ - 1) / TZ;
+    sh.nty = (g.n[1] + PAIR_TY - 1) / PAIR_TY;
+    // every coordinate a tile touches lies within one period of the grid
+    if (sh.ntz * TZ + R > 2 * g.n[2] || sh.nty * PAIR_TY + R > 2 * g.n[1] || g.n[0] < R ||
+        g.n[1] < R || g.n[2] < R)
+        return false;
+    if ((long)g.n[1] * g.n[2] >= PLANE_REF_MAX) return false;
+    sh.q = q < g.n[0] ? q : g.n[0];
+    sh.nchunk = (g.n[0] + sh.q - 1) / sh.q;
+    const long nb = (long)sh.ntz * sh.nty * nin * sh.nchunk;
+    if (nb > 0x7fffffffL) return false;
+    sh.nblocks = (int)nb;
+    return true;
+}
+
+// Default shape of the pair kernel: the width with the fewest lanes over the
+// row, the widest of those (a whole row is contiguous memory; 47 and 95
+// columns: 48 and 96, not 2 or 3 tiles of 32), and the run length whose blocks
+// fill the chip's slots best: rounds of resident blocks, half a one for the
+// last, times steps and the R + 2 planes each run starts with
+// (float64, 95 columns, 1056 tiles, 512 slots: 262 us in runs of 40 planes,
+// 273 in runs of 80).
+static bool pair_shape(const Stencil& s, const Geom& g, int dtype, int mode, int nin, int& TZ,
+                       TileShape& sh)
+{
+    TileShape c;
+    TZ = 0;
+    for (int tz : {96, 64, 48, 32})
+        if (pair_geometry(s, g, dtype, mode, nin, tz, g.n[0], c) &&
+            (!TZ || c.ntz * tz < sh.ntz * TZ)) {
+            TZ = tz;
+            sh = c;
+        }
+    if (!TZ) return false;
+    const int R = s.star_r;
+    const long lds = (long)(R + 2) * (TZ + 2 * R) * (PAIR_TY + 2 * R) * dtype_size(dtype);
+    const long slots = 256 * std::min(160 * 1024 / lds, 2048L / sh.nt);
+    double best = 0.0;
+    const long tiles = sh.nblocks;
+    for (int nch = 1; nch == 1 || g.n[0] / nch >= 8; nch++) {
+        const int q = ((g.n[0] + nch - 1) / nch + 1) & ~1;
+        const long blocks = tiles * ((g.n[0] + q - 1) / q);
+        const double cost = std::max(1.0, (double)blocks / slots + 0.5) * (q / 2 + 2);
+        if (nch == 1 || cost < 0.98 * best) {
+            best = cost;
+            if (!pair_geometry(s, g, dtype, mode, nin, TZ, q, c)) return false;
+            sh = c;
+        }
+    }
+    return true;
+}
+
+// The kernel and shape of an apply (or kinetic + potential pass) of range <= 3
+// that is too large for the real-data box default, by storage type and range.
+// Measured on sets of 0.1 .. 2 GB (us; tile = k_star_tile with 256 or 1024
+// threads, box = k_star_box with 8 planes):
+//   float64    96 x 79x87x95   apply  pair 279  box 277  tile 290
+//                              + v         325      310       348
+//              256 x 64^3      apply       244      256       262
+//              128 x 63^3      + v         156      163       172
+//   complex64  60 x 56x60x51               60        54   58 / 60
+//              64 x 48^3                   46        40   43 / 53
+//   float32    256 x 64^3                 150       166       178
+//   complex128 R = 3: 256 x 64^3          468             470 / 449
+//              256 x 47^3                 220       263   247 / 283
+//              100 x 28x36x44              48        51    49 / 97
+//              12 x 96x80x72               71        61    61 / 82
+//              100 x 30x46x42  + v         63        60    56 / 73
+//              R = 2, 1: 60 x 60x50x70     93, 72  139, 109  125, 112 / 120, 92
+// 1024-thread tiles have the smallest halo but need planes that fill their
+// 32 x 32 columns.  The other modes and range 4 keep the tile kernel.
+static void large_cfg(const Stencil& s, const Geom& g, int dtype, int mode, int nin, LaunchCfg& c)
+{
+    const int R = s.star_r;
+    if (R < 1 || R > 3 || (mode != ST_APPLY && mode != ST_HPSI)) return;
+    LaunchCfg p{K_PAIR, 0, TileShape{}};
+    const bool row = g.n[2] <= 64;   // one tile per row
+    if (dtype == DT_C64 || (dtype == DT_F64 && mode == ST_HPSI && !row)) {
+        p.kind = K_BOX;
+        p.TZ = BOX_TZ;
+        if (box_geometry(g, R, nin, 8, p.sh)) c = p;
+        return;
+    }
+    if (dtype == DT_C128 && R == 3) {
+        const double lanes = (double)((g.n[1] + 31) / 32 * 32) * ((g.n[2] + 31) / 32 * 32);
+        if (g.n[1] * (double)g.n[2] >= 0.9 * lanes) return;   // 1024-thread tiles
+        if (mode == ST_HPSI || !row) {
+            p.kind = K_TILE;
+            if (tile_shape(g, R, dtype_size(dtype), nin, p.TZ, p.sh, TILE_NT)) c = p;
+            return;
+        }
+    }
+    if (pair_shape(s, g, dtype, mode, nin, p.TZ, p.sh)) c = p;
+}
+
 // `dtype` and `mode` decide whether the box kernel applies; partial-sum
 // layouts are asked for with DT_F64 / ST_RESID (norms are taken of real
 // data only, and float and double grids get the same box and tile shapes)
@@ -588,13 +711,6 @@ int stencil_partials(const Stencil& s, const Geom& g, int nin)
     return (int)((ng + 255) / 256) * nin;
 }
 
-// One launch configuration: the kernel kind and, for tiles, the shape.
-struct LaunchCfg {
-    int kind;
-    int TZ;
-    TileShape sh;
-};
-
 static hipError_t launch_cfg(const LaunchCfg& c, const Stencil& s, int dtype, int mode,
                              const void* in, void* out, const void* aux, const Geom& g,
                              const Phases& ph, int nin, double w, double* partial, bool write,
@@ -602,6 +718,15 @@ static hipError_t launch_cfg(const LaunchCfg& c, const Stencil& s, int dtype, in
 {
     if (c.kind == K_BOX)
         return box_launch(s, dtype, mode, in, out, aux, g, ph, w, c.sh, partial, write, st);
+    if (c.kind == K_PAIR) {
+        switch (dtype) {
+        case DT_F64: return pair_launch_f64(s, mode, in, out, aux, g, ph, w, c.TZ, c.sh, st);
+        case DT_C128: return pair_launch_c128(s, mode, in, out, aux, g, ph, w, c.TZ, c.sh, st);
+        case DT_F32: return pair_launch_f32(s, mode, in, out, aux, g, ph, w, c.TZ, c.sh, st);
+        case DT_C64: return pair_launch_c64(s, mode, in, out, aux, g, ph, w, c.TZ, c.sh, st);
+        }
+        return hipErrorInvalidValue;
+    }
     if (c.kind == K_TILE) {
         switch (dtype) {
         case DT_F64: return tile_launch_f64(s, mode, in, out, aux, g, ph, w, c.TZ, c.sh, partial, write, st);
@@ -735,6 +860,12 @@ TuneVal tune(const TuneKey& key, const LaunchCfg& heuristic, const Stencil& s, i
             LaunchCfg c{K_BOX, BOX_TZ, TileShape{}};
             if (box_geometry(g, s.star_r, nin, q, c.sh)) cand.push_back(c);
         }
+    for (int TZ : {96, 64, 48, 32})
+        for (int q : {8, 16, 32, 64, 1 << 20}) {
+            LaunchCfg c{K_PAIR, TZ, TileShape{}};
+            if (!pair_geometry(s, g, dtype, mode, nin, TZ, q, c.sh)) continue;
+            if (q == 1 << 20 || q < g.n[0]) cand.push_back(c);
+        }
     TuneVal best{heuristic, -1.0f, 0};
     hipEvent_t e0, e1;
     if (hipEventCreate(&e0) != hipSuccess) return best;
@@ -821,6 +952,7 @@ hipError_t launch_stencil(const Stencil& s, int dtype, int mode, const void* in,
         TileShape b8;
         if (box_geometry(g, s.star_r, nin, 8, b8)) c.sh = b8;
     }
+    if (!partial && c.kind == K_TILE && forced_kind() < 0) large_cfg(s, g, dtype, mode, nin, c);
     const int ov = g_kind_override.load();
     if (!partial && ov >= 0 && ov != c.kind) {
         // the requested family when it can run this launch, else the default
