@@ -38,13 +38,19 @@ __global__ __launch_bounds__(256) void k_pc_scale(const double* __restrict__ r,
 
 namespace {
 
-// Runs of the whole i0 axis, split where there are too few tiles (a run of
-// k_pc_interp starts with R + 1 coarse planes, each two barriers).
-bool pc_shape(const Geom& g, int R, int esize, int nin, int nt, TileShape* sh)
+// Runs of the whole i0 axis, split towards 1024 blocks where there are too few
+// tiles, each of at least `run` planes: a small set waits on a block's serial
+// planes, but a run reads 2 R more and one of k_pc_interp starts with R + 1
+// coarse planes of two barriers each.  2 planes for k_pc_scaled, 4 for
+// k_pc_interp with b and 8 without: real 3 bands of 79 x 63 x 71, a call in
+// 40.7 us, with 8 planes in all three 50.4, 4 / 8 / 8 44.7, 2 / 2 / 8 42.5;
+// complex128 24 x 64^3 145, 149, 147, 150; 16 x 32^3 54, 56, 54, 56; 6 or 4
+// planes without b: 59 or 54.5, real 8 x 64^3 48.6 or 47.3 instead of 45.
+bool pc_shape(const Geom& g, int R, int esize, int nin, int nt, int run, TileShape* sh)
 {
     if (!tile_geometry(g, R, esize, nin, 32, g.n[0], *sh, nt)) return false;
     long nch = (1024L + sh->nblocks - 1) / sh->nblocks;
-    const long maxch = g.n[0] / 8 > 1 ? g.n[0] / 8 : 1;
+    const long maxch = g.n[0] / run > 1 ? g.n[0] / run : 1;
     if (nch > maxch) nch = maxch;
     return tile_geometry(g, R, esize, nin, 32, (int)((g.n[0] + nch - 1) / nch), *sh, nt);
 }
@@ -61,15 +67,15 @@ i64 pc_points(const int n[3]) { return (i64)n[0] * n[1] * n[2]; }
 // out = mode(L F, aux b) with F = c b; hipErrorNotSupported (nothing launched)
 // where k_pc_scaled does not run: it takes range-1 stars whose halo wraps once,
 // complex data from 2^15 points in all (below, one tile's serial planes take
-// longer than the two short launches: 8 bands of 13 x 11 x 17, a call of 48
-// instead of 44 us).
+// longer than the two short launches: 8 bands of 13 x 11 x 17, a call of 50
+// instead of 46 us).
 template <class V>
 hipError_t pc_scaled(const gpaw_operator* L, int mode, const void* b, void* out, int nin,
                      const Phases& ph, double cb, double w, hipStream_t st)
 {
     TileShape sh;
     if (VT<V>::cplx && nin * pc_points(L->g.n) < 1 << 15) return hipErrorNotSupported;
-    if (L->st.star_r != 1 || !pc_shape(L->g, 1, (int)sizeof(V), nin, TILE_NT, &sh))
+    if (L->st.star_r != 1 || !pc_shape(L->g, 1, (int)sizeof(V), nin, TILE_NT, 2, &sh))
         return hipErrorNotSupported;
     const dim3 grid(sh.nblocks), block(32, TILE_NT / 32);
     const TileCoefs sc = pc_coefs(L->st);
@@ -91,7 +97,7 @@ hipError_t pc_interp_go(const gpaw_operator* L, const Transfer& t, const void* b
 {
     const Geom& g = L->g;
     TileShape sh;
-    if (!pc_shape(g, R, (int)sizeof(V), nin, 32 * TY, &sh)) return hipErrorNotSupported;
+    if (!pc_shape(g, R, (int)sizeof(V), nin, 32 * TY, BASE ? 4 : 8, &sh)) return hipErrorNotSupported;
     PcCoarse pc;
     for (int a = 0; a < 3; a++) {
         pc.nc[a] = t.gin.n[a];
@@ -119,14 +125,11 @@ hipError_t pc_interp(const gpaw_operator* L, const Transfer& t, const void* b, c
     }
     const i64 points = nin * pc_points(g.n);
     // complex bands below 2^18 points in all: every launch is a few us there, and
-    // a block's serial planes cost more than the launch saved (1 / 4 / 16 bands
-    // of 32^3: 49.5 / 53 / 55 us fused, 46 / 50 / 58 in steps).  Real bands gain
-    // there (a call is bound by the host), but lose on few tiles of many planes
-    // (3 bands of 79 x 63 x 71, 72 tiles: 47 against 44.5 us; 16 of 48^3, 192
-    // tiles: 47 against 52.6).
-    const i64 tiles = (i64)((g.n[1] + 7) / 8) * ((g.n[2] + 31) / 32) * nin;
-    if (VT<V>::cplx ? points < 1 << 18 : points >= 1 << 18 && tiles < 128)
-        return hipErrorNotSupported;
+    // a block's serial planes cost what the launch saved (1 / 4 / 16 bands of
+    // 32^3: 49 / 51 / 54 us fused, 47 / 50 / 58 in steps); real bands gain at
+    // every size (3 bands of 79 x 63 x 71: 38 us instead of 41, one of 96^3: 33
+    // instead of 37)
+    if (VT<V>::cplx && points < 1 << 18) return hipErrorNotSupported;
     // 16 rows per block on large sets where they pad no more rows than 8 do
     // (complex128, 256 x 64^3: 1075 us a call with 8, 1001 with 16, 1009 with 32
     // rows; 64 x 32^3: 90 with 8, 82 with 16; real 16 x 48^3: 47 with 8, 50 with 16)
