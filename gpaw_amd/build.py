@@ -22,7 +22,7 @@ SOURCES = ['stencil.hip', 'stencil_tile_f64.hip', 'stencil_tile_c128.hip',
            'stencil_box_c128.hip', 'stencil_box_f32.hip', 'stencil_box_c64.hip', 'transfer.hip',
            'transfer_f64.hip', 'transfer_c128.hip', 'transfer_f32.hip',
            'transfer_c64.hip',
-           'misc.hip', 'capi.hip', 'poisson.hip', 'coarse.hip', 'mixed.hip', 'gs.hip',
+           'misc.hip', 'capi.hip', 'poisson.hip', 'coarse.hip', 'cg_step.hip', 'mixed.hip', 'gs.hip',
            'precond.hip', 'batch.hip', 'batch_f64.hip', 'batch_c128.hip',
            'batch_f32.hip', 'batch_c64.hip', 'jacobi_fused.hip',
            'resid_restrict.hip', 'jacobi_corr.hip', 'stencil_gen_f64.hip',

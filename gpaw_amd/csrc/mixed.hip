@@ -35,6 +35,7 @@
 #include <cstdlib>
 #include <cstring>
 
+#include "cg_step.h"
 #include "poisson_internal.h"
 
 using namespace gpaw;
@@ -63,16 +64,16 @@ struct MixedState {
     std::vector<std::vector<double>> wpre, wpost;
     VLevels v[2];                       // [0] FP32, [1] FP64 inner V-cycle
     bool ready[2] = {false, false};
-    double *p = nullptr, *q = nullptr;  // FP64 search direction, L p
+    // FP64 search direction (two arrays: a step writes the one it does not
+    // read; a chunk begins and ends with p[0]) and L p
+    double *p[2] = {nullptr, nullptr}, *q = nullptr;
     double* S = nullptr;                // device scalars
     double* h_S = nullptr;              // pinned readback
     double* partial = nullptr;
     // graphs per inner precision
     hipGraphExec_t g_vcycle[2] = {nullptr, nullptr};   // one V-cycle from zero
     hipGraphExec_t g_vwarm[2] = {nullptr, nullptr};    // one V-cycle from the last result
-    hipGraphExec_t g_a[2] = {nullptr, nullptr};        // PCG: q = Lp, alpha, update, |d|^2
-    hipGraphExec_t g_b[2] = {nullptr, nullptr};        // PCG: z = V(d), beta, p = z + beta p
-    // k PCG steps (b then a) per launch, k = 1 .. MIXED_CHUNK_MAX; [1]: the
+    // k PCG steps (emit_step) per launch, k = 1 .. MIXED_CHUNK_MAX; [1]: the
     // same followed by the true residual's norm (chunks expected to converge)
     std::vector<hipGraphExec_t> g_ba[2][2];
     // PCG steps the last converged solve took, per inner precision, and the
@@ -137,15 +138,16 @@ __device__ __forceinline__ double sum_partials(const double* __restrict__ p, int
     return block_sum<256>(t, red);
 }
 
-// alpha = dz / pq ; phi -= alpha p ; d -= alpha q ; dlow = d (the inner
-// V-cycle's right-hand side in its own precision; nullptr when the inner
-// V-cycle reads d itself) ; partials of |d|^2 into `partial`.  dz (the ndz
-// partials at dzp) and pq (the npq partials at pqp, or S[PQ] when npq = 0)
-// are summed by every block itself; block 0 keeps dz in S[DZ] (the next
-// step's old dz) and alpha in S[ALPHA].
+// alpha = dz / pq ; d -= alpha q ; dlow = d (the inner V-cycle's right-hand
+// side in its own precision; nullptr when the inner V-cycle reads d itself) ;
+// partials of |d|^2 into `partial`.  dz (the ndz partials at dzp) and pq (the
+// npq partials at pqp, or S[PQ] when npq = 0) are summed by every block
+// itself; block 0 keeps dz in S[DZ] (the next step's old dz) and alpha in
+// S[ALPHA].  phi -= alpha p is left to the next direction step, which reads p
+// anyway (k_cg_dir), or to k_phi_step at the end of a chunk.
+// Bound by memory: 112 MB on 159^3.
 template <class T>
-__global__ __launch_bounds__(256) void k_pcg_update(double* __restrict__ phi, double* __restrict__ d,
-                                                    const double* __restrict__ p,
+__global__ __launch_bounds__(256) void k_pcg_update(double* __restrict__ d,
                                                     const double* __restrict__ q,
                                                     T* __restrict__ dlow, double* __restrict__ S,
                                                     i64 n, double* __restrict__ partial,
@@ -159,7 +161,6 @@ __global__ __launch_bounds__(256) void k_pcg_update(double* __restrict__ phi, do
     const double alpha = pq != 0.0 ? dz / pq : 0.0;
     double s = 0.0;
     for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < n; i += (i64)gridDim.x * 256) {
-        phi[i] = phi[i] - alpha * p[i];
         const double di = d[i] - alpha * q[i];
         d[i] = di;
         if (dlow) dlow[i] = (T)di;
@@ -170,6 +171,21 @@ __global__ __launch_bounds__(256) void k_pcg_update(double* __restrict__ phi, do
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         S[S_ALPHA] = alpha;
         S[S_DZ] = dz;
+    }
+}
+
+// phi -= alpha p, the last step of a chunk; p_out (not nullptr): p_out = p,
+// where the next chunk looks for it
+__global__ __launch_bounds__(256) void k_phi_step(double* __restrict__ phi,
+                                                  const double* __restrict__ p,
+                                                  double* __restrict__ p_out,
+                                                  const double* __restrict__ S, i64 n)
+{
+    const double alpha = S[S_ALPHA];
+    for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < n; i += (i64)gridDim.x * 256) {
+        const double v = p[i];
+        phi[i] = phi[i] - alpha * v;
+        if (p_out) p_out[i] = v;
     }
 }
 
@@ -197,12 +213,15 @@ __global__ __launch_bounds__(256) void k_dot_dz_zq(const double* __restrict__ d,
 
 // p = z + beta p, beta = -alpha (z.q) / (d_old.z_old) (Polak-Ribiere), z.q
 // summed by every block from the nzq partials at zqp, d_old.z_old = S[DZ]
-// (kept by the previous update); first, or S[DZ] = 0 (a restart): p = z.
+// (kept by the previous update); S[DZ] = 0 (a restart): p = z.  Before that
+// the pending phi -= alpha p (phi not nullptr).
 // hist: block 0 also sums the previous step's |d|^2 partials (ndd at ddp)
 // into *hist, so the host sees |d| after every step of a chunk.
+// For operators without k_cg_dir, which does this in the operator's launch.
 template <class T>
 __global__ __launch_bounds__(256) void k_p_update(double* __restrict__ p, const T* __restrict__ z,
-                                                  double* __restrict__ S, i64 n, int first,
+                                                  double* __restrict__ phi,
+                                                  const double* __restrict__ S, i64 n,
                                                   const double* __restrict__ zqp, int nzq,
                                                   const double* __restrict__ ddp, int ndd,
                                                   double* __restrict__ hist)
@@ -212,12 +231,15 @@ __global__ __launch_bounds__(256) void k_p_update(double* __restrict__ p, const 
         const double v = sum_partials(ddp, ndd, red);
         if (threadIdx.x == 0) *hist = v;
     }
-    const double dzo = S[S_DZ];
-    const bool f = first || dzo == 0.0;   // uniform over the grid
+    const double dzo = S[S_DZ], alpha = S[S_ALPHA];
+    const bool f = dzo == 0.0;   // uniform over the grid
     const double zq = f ? 0.0 : sum_partials(zqp, nzq, red);
-    const double beta = f ? 0.0 : -S[S_ALPHA] * zq / dzo;
-    for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < n; i += (i64)gridDim.x * 256)
-        p[i] = f ? (double)z[i] : (double)z[i] + beta * p[i];
+    const double beta = f ? 0.0 : -alpha * zq / dzo;
+    for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < n; i += (i64)gridDim.x * 256) {
+        const double v = p[i];
+        if (phi) phi[i] = phi[i] - alpha * v;
+        p[i] = f ? (double)z[i] : (double)z[i] + beta * v;
+    }
 }
 
 // The first Jacobi sweep from phi = 0: every stencil term is zero, so the
@@ -551,7 +573,8 @@ int setup(gpaw_poisson* ps, int pr)
         for (int l = 1; l <= ps->L; l++)
             mixed_level_schedule(ps, l, m->pre[l], m->post[l], m->wpre[l], m->wpost[l]);
         const size_t n0 = sizeof(double) * ps->npts[0];
-        int rc = gpaw_check(hipMalloc((void**)&m->p, n0), "mixed: p");
+        int rc = gpaw_check(hipMalloc((void**)&m->p[0], n0), "mixed: p");
+        if (!rc) rc = gpaw_check(hipMalloc((void**)&m->p[1], n0), "mixed: p");
         if (!rc) rc = gpaw_check(hipMalloc((void**)&m->q, n0), "mixed: q");
         if (!rc) rc = gpaw_check(hipMalloc((void**)&m->S, sizeof(double) * S_N), "mixed: scalars");
         if (!rc)
@@ -565,13 +588,14 @@ int setup(gpaw_poisson* ps, int pr)
     MixedState* m = ps->mixed;
     if (m->ready[pr]) return GPAW_OK;
     int rc = pr ? setup_v64(ps, m) : setup_v32(ps, m);
+    for (int t = 0; t < 2; t++) m->g_ba[pr][t].assign(MIXED_CHUNK_MAX, nullptr);
     if (!rc) m->ready[pr] = true;
     return rc;
 }
 
 void destroy_graphs(MixedState* m, int pr)
 {
-    for (hipGraphExec_t* g : {&m->g_vcycle[pr], &m->g_vwarm[pr], &m->g_a[pr], &m->g_b[pr]}) {
+    for (hipGraphExec_t* g : {&m->g_vcycle[pr], &m->g_vwarm[pr]}) {
         if (*g) hipGraphExecDestroy(*g);
         *g = nullptr;
     }
@@ -582,87 +606,89 @@ void destroy_graphs(MixedState* m, int pr)
         }
 }
 
-// PCG step part a: q = L p, alpha, phi += alpha p, d -= alpha q, |d|^2.
-// |d|^2 (S[DD]) is only read by the host after a launch, so only the last
-// step of a launch sums its partials (`last`).
-hipError_t emit_a(gpaw_poisson* ps, MixedState* m, int pr, hipStream_t st, bool last = true)
+// PCG step i of a chunk: z = V(d), beta (flexible), p = z + beta p, q = L p,
+// alpha, d -= alpha q, |d|^2, each step's phi -= alpha p done by the next one
+// (emit_end: the last).  |d|^2 (S[DD]) is only read by the host after a launch,
+// so only the last step of a launch sums its partials into it (`last`); `hist`:
+// where the previous step's |d|^2 goes (nullptr: not summed).
+template <class T>
+hipError_t emit_step(gpaw_poisson* ps, MixedState* m, int pr, int i, bool last, hipStream_t st,
+                     double* hist)
 {
     const i64 n = ps->npts[0];
+    const int nb = (int)gridn(n).x;
     gpaw_operator* op = ps->ops[0];
     Phases ph;
     gpaw_phases(nullptr, ph);
-    hipError_t e;
-    const double* pqp = nullptr;
-    int npq = 0;
-    if (stencil_dot_ok(op->st, DT_F64, op->g, 1)) {   // q = L p with the partials of p.q
-        int np = 0;
-        e = launch_stencil(op->st, DT_F64, ST_APPLY, m->p, m->q, nullptr, op->g, ph, 1, 0.0,
-                           op->partial, &np, true, st);
-        if (e != hipSuccess) return e;
-        pqp = op->partial;   // summed inside the update
-        npq = np;
-    } else {
-        e = launch_stencil(op->st, DT_F64, ST_APPLY, m->p, m->q, nullptr, op->g, ph, 1, 0.0,
-                           nullptr, nullptr, true, st);
-        if (e != hipSuccess) return e;
-        launch_kernel(k_dot, gridn(n), dim3(256), 0, st, m->p, m->q, n, m->partial + PART_PQ);
-        launch_kernel(k_red1, dim3(1), dim3(256), 0, st, m->partial + PART_PQ,
-                      (int)gridn(n).x, m->S, (int)S_PQ);
-    }
-    // dz: the d.z partials of the step's k_dot_dz_zq
-    if (pr == 0)
-        launch_kernel(k_pcg_update<float>, gridn(n), dim3(256), 0, st, ps->phiA[0], ps->res[0],
-                      m->p, m->q, (float*)m->v[0].rho[0], m->S, n, m->partial + PART_DD, pqp,
-                      npq, (const double*)m->partial, (int)gridn(n).x);
-    else
-        launch_kernel(k_pcg_update<double>, gridn(n), dim3(256), 0, st, ps->phiA[0], ps->res[0],
-                      m->p, m->q, (double*)nullptr, m->S, n, m->partial + PART_DD, pqp, npq,
-                      (const double*)m->partial, (int)gridn(n).x);
-    if (last)
-        launch_kernel(k_red1, dim3(1), dim3(256), 0, st, m->partial + PART_DD, (int)gridn(n).x,
-                      m->S, (int)S_DD);
-    return launch_error();
-}
-
-// z, beta (flexible), p = z + beta p after the inner V-cycle; first: p = z
-template <class T>
-void emit_dz_p(gpaw_poisson* ps, MixedState* m, int pr, int first, hipStream_t st,
-               double* hist = nullptr)
-{
-    const i64 n = ps->npts[0];
-    launch_kernel(k_dot_dz_zq<T>, gridn(n), dim3(256), 0, st, ps->res[0],
-                  (const T*)z_of(m, pr), m->q, n, m->partial);
-    launch_kernel(k_p_update<T>, gridn(n), dim3(256), 0, st, m->p, (const T*)z_of(m, pr),
-                  m->S, n, first, (const double*)m->partial + gridn(n).x,
-                  (int)gridn(n).x, (const double*)m->partial + PART_DD, (int)gridn(n).x, hist);
-}
-
-// PCG step part b: z = V(d), beta (flexible), p = z + beta p; `hist`: where
-// the previous step's |d|^2 goes (nullptr: not summed)
-hipError_t emit_b(gpaw_poisson* ps, MixedState* m, int pr, hipStream_t st, double* hist = nullptr)
-{
     hipError_t e = emit_top(ps, m, pr, true, st);
     if (e != hipSuccess) return e;
-    if (pr == 0)
-        emit_dz_p<float>(ps, m, pr, 0, st, hist);
-    else
-        emit_dz_p<double>(ps, m, pr, 0, st, hist);
+    const T* z = (const T*)z_of(m, pr);
+    launch_kernel(k_dot_dz_zq<T>, gridn(n), dim3(256), 0, st, ps->res[0], z, m->q, n, m->partial);
+    const double* pqp = op->partial;   // the partials of p.q, summed inside the update
+    int npq = 0;
+    double* phi = i > 0 ? ps->phiA[0] : nullptr;
+    if (cg_dir_ok(op->st, op->g, &npq)) {
+        const CgStep s = {m->p[i & 1], m->p[~i & 1], m->q, phi, m->S, S_ALPHA, S_DZ,
+                          m->partial + nb, nb, m->partial + PART_DD, nb, hist, op->partial};
+        e = launch_cg_dir(op->st, op->g, s, z, m->v[pr].dt, st);
+        if (e != hipSuccess) return e;
+    } else {
+        launch_kernel(k_p_update<T>, gridn(n), dim3(256), 0, st, m->p[0], z, phi, m->S, n,
+                      (const double*)m->partial + nb, nb, (const double*)m->partial + PART_DD, nb,
+                      hist);
+        const bool dot = stencil_dot_ok(op->st, DT_F64, op->g, 1);
+        npq = 0;
+        e = launch_stencil(op->st, DT_F64, ST_APPLY, m->p[0], m->q, nullptr, op->g, ph, 1, 0.0,
+                           dot ? op->partial : nullptr, dot ? &npq : nullptr, true, st);
+        if (e != hipSuccess) return e;
+        if (!dot) {
+            launch_kernel(k_dot, gridn(n), dim3(256), 0, st, m->p[0], m->q, n,
+                          m->partial + PART_PQ);
+            launch_kernel(k_red1, dim3(1), dim3(256), 0, st, m->partial + PART_PQ, nb, m->S,
+                          (int)S_PQ);
+        }
+    }
+    // dz: the d.z partials of the step's k_dot_dz_zq
+    launch_kernel(k_pcg_update<T>, gridn(n), dim3(256), 0, st, ps->res[0], m->q,
+                  pr == 0 ? (T*)m->v[0].rho[0] : (T*)nullptr, m->S, n, m->partial + PART_DD, pqp,
+                  npq, (const double*)m->partial, nb);
+    if (last)
+        launch_kernel(k_red1, dim3(1), dim3(256), 0, st, m->partial + PART_DD, nb, m->S,
+                      (int)S_DD);
     return launch_error();
+}
+
+// the end of a chunk of k steps: phi -= alpha p of its last step, p in p[0]
+hipError_t emit_end(gpaw_poisson* ps, MixedState* m, int k, hipStream_t st)
+{
+    const i64 n = ps->npts[0];
+    int np = 0;
+    const bool odd = cg_dir_ok(ps->ops[0]->st, ps->ops[0]->g, &np) && (k & 1);
+    launch_kernel(k_phi_step, gridn(n), dim3(256), 0, st, ps->phiA[0], m->p[odd],
+                  odd ? m->p[0] : (double*)nullptr, m->S, n);
+    return launch_error();
+}
+
+hipError_t emit_steps(gpaw_poisson* ps, MixedState* m, int pr, int k, hipStream_t st)
+{
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < k && e == hipSuccess; i++) {
+        double* hist = i > 0 ? m->S + S_HIST + i - 1 : nullptr;
+        e = pr == 0 ? emit_step<float>(ps, m, pr, i, i == k - 1, st, hist)
+                    : emit_step<double>(ps, m, pr, i, i == k - 1, st, hist);
+    }
+    return e == hipSuccess ? emit_end(ps, m, k, st) : e;
 }
 
 int capture_all(gpaw_poisson* ps, int pr)
 {
     MixedState* m = ps->mixed;
-    if (m->g_b[pr]) return GPAW_OK;   // the last one built: all four exist
+    if (m->g_vwarm[pr]) return GPAW_OK;   // the last one built: both exist
     int rc = capture_graph(&m->g_vcycle[pr],
                            [&](hipStream_t st) { return emit_top(ps, m, pr, true, st); });
     if (!rc)
         rc = capture_graph(&m->g_vwarm[pr],
                            [&](hipStream_t st) { return emit_top(ps, m, pr, false, st); });
-    if (!rc) rc = capture_graph(&m->g_a[pr], [&](hipStream_t st) { return emit_a(ps, m, pr, st); });
-    if (!rc) rc = capture_graph(&m->g_b[pr], [&](hipStream_t st) { return emit_b(ps, m, pr, st); });
-    if (!rc)
-        for (int t = 0; t < 2; t++) m->g_ba[pr][t].assign(MIXED_CHUNK_MAX, nullptr);
     if (rc) destroy_graphs(m, pr);   // retried from scratch on the next call
     return rc;
 }
@@ -681,18 +707,14 @@ hipError_t emit_true_norm(gpaw_poisson* ps, MixedState* m, int slot, hipStream_t
     return e;
 }
 
-// k PCG steps (b, a) in one graph; `fin`: then the true residual's norm
+// k PCG steps in one graph; `fin`: then the true residual's norm
 // into S[DT] (a chunk expected to reach the tolerance)
 int run_ba(gpaw_poisson* ps, MixedState* m, int pr, int k, bool fin, hipStream_t st)
 {
     hipGraphExec_t& g = m->g_ba[pr][fin ? 1 : 0][k - 1];
     if (!g) {
         int rc = capture_graph(&g, [&](hipStream_t s) -> hipError_t {
-            hipError_t e = hipSuccess;
-            for (int i = 0; i < k && e == hipSuccess; i++) {
-                e = emit_b(ps, m, pr, s, i > 0 ? m->S + S_HIST + i - 1 : nullptr);
-                if (e == hipSuccess) e = emit_a(ps, m, pr, s, i == k - 1);
-            }
+            hipError_t e = emit_steps(ps, m, pr, k, s);
             if (e == hipSuccess && fin) e = emit_true_norm(ps, m, S_DT, s);
             return e;
         });
@@ -786,7 +808,7 @@ void gpaw_mixed_free(MixedState* m)
         for (void* p : m->v[pr].owned) hipFree(p);
         if (m->v[pr].own_coarse && m->v[pr].d_coarse) hipFree(m->v[pr].d_coarse);
     }
-    for (double* p : {m->p, m->q, m->S, m->partial})
+    for (double* p : {m->p[0], m->p[1], m->q, m->S, m->partial})
         if (p) hipFree(p);
     if (m->h_S) hipHostFree(m->h_S);
     delete m;
@@ -844,11 +866,10 @@ extern "C" int gpaw_poisson_solve_mixed(gpaw_poisson* ps, double* phi, const dou
         // one eager pass of the graph bodies on the plan's own buffers (all
         // reloaded below), so that the graphs record tuned launch shapes
         m->tuned[pr] = 1;
-        hipError_t e = emit_top(ps, m, pr, true, st);
-        if (e == hipSuccess) e = emit_a(ps, m, pr, st);
+        hipError_t e = emit_steps(ps, m, pr, 1, st);
         rc = gpaw_check(e, "mixed: tune");
     }
-    if (!rc) rc = capture_all(ps, pr);
+    if (!rc && !pcg) rc = capture_all(ps, pr);   // CG steps have graphs of their own
     if (rc) return rc;
     const i64 n = ps->npts[0];
     hipError_t e = rho ? launch_copy(ps->rho[0], rho, DT_F64, n, st) : hipSuccess;
