@@ -218,6 +218,10 @@ hipError_t launch_axpby(double* y, const double* x, double a, double b, long lon
                         hipStream_t st);   // y = a*y + b*x
 hipError_t launch_axpby_shared(double* y, const double* x, double a, double b, int nin,
                                long long n, hipStream_t st);   // y_k = a*y_k + b*x
+// y = x - mean, mean = scale * sum(x) / dv / n; integral (device or pinned host
+// memory, or nullptr) = scale * sum(x); partial holds SUM_PARTIALS doubles
+hipError_t launch_sub_mean(double* y, const double* x, long long n, double scale, double dv,
+                           double* partial, double* integral, hipStream_t st);
 hipError_t launch_sub_scalar(double* y, const double* x, double b, long long n,
                              hipStream_t st);  // y = x - b
 hipError_t launch_fill(void* y, int dtype, long long n, hipStream_t st);

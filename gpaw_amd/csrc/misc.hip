@@ -89,6 +89,25 @@ __global__ __launch_bounds__(256) void k_sub_scalar(double* __restrict__ y,
     if (i < n) y[i] = x[i] - b;
 }
 
+// y = x - mean, mean = scale * sum(x) / dv / n with sum(x) in the np partials
+// k_sum left: every block sums them itself in the order of k_reduce_partials, so
+// neither a reduction launch nor a readback stands between the sum and its use.
+// integral (not nullptr, may be host memory): scale * sum(x).
+__global__ __launch_bounds__(256) void k_sub_mean(double* y, const double* x, i64 n,
+                                                  const double* __restrict__ partial, int np,
+                                                  double scale, double dv,
+                                                  double* __restrict__ integral)
+{
+    __shared__ double red[256];
+    double s = 0.0;
+    for (int i = threadIdx.x; i < np; i += 256) s += partial[i];
+    const double q = block_sum<256>(s, red) * scale;
+    if (integral && blockIdx.x == 0 && threadIdx.x == 0) *integral = q;
+    const double mean = q / dv / (double)n;
+    const i64 step = (i64)gridDim.x * 256;
+    for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < n; i += step) y[i] = x[i] - mean;
+}
+
 template <class T>
 __global__ __launch_bounds__(256) void k_fill(T* __restrict__ y, i64 n)
 {
@@ -253,6 +272,20 @@ hipError_t launch_axpby(double* y, const double* x, double a, double b, long lon
 {
     if (n <= 0) return hipSuccess;
     launch_kernel(k_axpby, grid1(n), dim3(256), 0, st, y, x, a, b, (i64)n);
+    return launch_error();
+}
+
+hipError_t launch_sub_mean(double* y, const double* x, long long n, double scale, double dv,
+                           double* partial, double* integral, hipStream_t st)
+{
+    if (n <= 0) return hipSuccess;
+    int np = 0;
+    hipError_t e = launch_sum(x, n, partial, &np, st);
+    if (e != hipSuccess) return e;
+    i64 nb = (n + 1023) / 1024;   // 4 points a thread; at most 8 blocks per CU
+    if (nb > 2048) nb = 2048;
+    launch_kernel(k_sub_mean, dim3((unsigned)nb), dim3(256), 0, st, y, x, (i64)n,
+                  (const double*)partial, np, scale, dv, integral);
     return launch_error();
 }
 

@@ -129,6 +129,37 @@ __global__ __launch_bounds__(256) void k_red1(const double* __restrict__ p, int 
     if (threadIdx.x == 0) S[slot] = s;
 }
 
+// the device scalars into pinned host memory: a kernel's store in place of a
+// copy back, whose launch and gaps took about 15 us
+__global__ __launch_bounds__(64) void k_publish(const double* __restrict__ S, double* __restrict__ h)
+{
+    if (threadIdx.x < S_N) h[threadIdx.x] = S[threadIdx.x];
+}
+
+// phi = src (less its mean, scale * sum(src) / dv / n, when `mean`) if the
+// chunk that ended with the true residual converged: the host's own test, made
+// here so that the store need not wait for it.
+__global__ __launch_bounds__(256) void k_store_if(double* __restrict__ phi,
+                                                  const double* __restrict__ src, i64 n,
+                                                  const double* __restrict__ S, double tol2,
+                                                  const double* __restrict__ partial, int np,
+                                                  double scale, double dv, int mean)
+{
+    __shared__ double red[256];
+    const double dd = S[S_DD], dt = S[S_DT];
+    if (!(dd - dd == 0.0) || !(dt <= tol2 * S[S_RR])) return;   // uniform over the grid
+    if (mean) {
+        double t = 0.0;
+        for (int i = threadIdx.x; i < np; i += 256) t += partial[i];
+        const double m = block_sum<256>(t, red) * scale / dv / (double)n;
+        for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < n; i += (i64)gridDim.x * 256)
+            phi[i] = src[i] - m;
+    } else {
+        for (i64 i = (i64)blockIdx.x * 256 + threadIdx.x; i < n; i += (i64)gridDim.x * 256)
+            phi[i] = src[i];
+    }
+}
+
 // Sum of n partials in k_red1's order (every block of a launch gets the
 // same value).
 __device__ __forceinline__ double sum_partials(const double* __restrict__ p, int n, double* red)
@@ -770,16 +801,33 @@ bool mixed_log()
 // S[DZ] = 0: the next direction update restarts the recursion (p = z)
 int mark_restart(MixedState* m, hipStream_t st)
 {
-    return gpaw_check(hipMemsetAsync(m->S + S_DZ, 0, sizeof(double), st), "mixed: restart");
+    return gpaw_check(launch_fill(m->S + S_DZ, DT_F64, 1, st), "mixed: restart");
 }
 
 int read_scalar(MixedState* m, int slot, hipStream_t st, double* v)
 {
-    hipError_t e = hipMemcpyAsync(m->h_S, m->S, sizeof(double) * S_N, hipMemcpyDeviceToHost, st);
+    launch_kernel(k_publish, dim3(1), dim3(64), 0, st, (const double*)m->S, m->h_S);
+    hipError_t e = launch_error();
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return gpaw_check(e, "mixed: readback");
     *v = m->h_S[slot];
     return GPAW_OK;
+}
+
+// phi stored if the chunk just launched (one with the true residual) converges
+int store_if(gpaw_poisson* ps, MixedState* m, double* phi, double tol2, hipStream_t st)
+{
+    const i64 n = ps->npts[0];
+    int np = 0;
+    hipError_t e = hipSuccess;
+    if (ps->remove_mean) e = launch_sum(ps->phiA[0], n, ps->d_sum, &np, st);
+    if (e == hipSuccess) {
+        launch_kernel(k_store_if, dim3((unsigned)std::min<i64>((n + 1023) / 1024, 2048)),
+                      dim3(256), 0, st, phi, (const double*)ps->phiA[0], n, (const double*)m->S,
+                      tol2, (const double*)ps->d_sum, np, ps->dv, ps->dv, (int)ps->remove_mean);
+        e = launch_error();
+    }
+    return gpaw_check(e, "mixed: store");
 }
 
 // d = L phi - rho (FP64, stored in res[0]) with |d|^2 into S[slot]; the
@@ -884,6 +932,7 @@ extern "C" int gpaw_poisson_solve_mixed(gpaw_poisson* ps, double* phi, const dou
     if (e != hipSuccess) return gpaw_check(e, "mixed: load");
     double rr = 0.0, dd = 0.0, target = 0.0;
     int it = 0;
+    bool stored = false;   // phi was stored by the chunk itself
     if (pcg) {
         // d = L phi - rho with |d|^2 into S[D0] and a restart marker, then
         // the first chunk with no readback in between (on a zero residual
@@ -908,6 +957,7 @@ extern "C" int gpaw_poisson_solve_mixed(gpaw_poisson* ps, double* phi, const dou
             k = std::min(k, maxiter - it);
             if (k < 1) break;
             rc = run_ba(ps, m, pr, k, fin, st);
+            if (!rc && fin) rc = store_if(ps, m, phi, rel_tol * rel_tol, st);
             if (!rc) rc = read_scalar(m, S_DD, st, &dd);
             if (rc) break;
             if (first) {   // |rho|^2 and the starting |d|^2 came back too
@@ -939,6 +989,7 @@ extern "C" int gpaw_poisson_solve_mixed(gpaw_poisson* ps, double* phi, const dou
                 have_true = true;
             }
             if (have_true && (!std::isfinite(dt) || dt <= target)) {
+                stored = fin;
                 dd = dt;
                 break;
             }
@@ -1012,7 +1063,10 @@ extern "C" int gpaw_poisson_solve_mixed(gpaw_poisson* ps, double* phi, const dou
         return gpaw_fail(GPAW_EDEVICE, "mixed-precision Poisson solver broke down (residual "
                                        "norm %g after %d iterations); phi not updated",
                          dd, it);
-    rc = gpaw_check(launch_copy(phi, ps->phiA[0], DT_F64, n, st), "mixed: store");
+    if (!stored)
+        rc = gpaw_check(dd <= target ? gpaw_poisson_store(ps, phi, ps->phiA[0], st)
+                                     : launch_copy(phi, ps->phiA[0], DT_F64, n, st),
+                        "mixed: store");
     if (rc) return rc;
     if (!(dd <= target))
         return gpaw_fail(GPAW_ENOCONV, "mixed-precision Poisson solver did not reach %g in %d "

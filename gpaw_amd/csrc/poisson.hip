@@ -15,8 +15,8 @@
 // Transformer calls and numpy updates.  The sequence is captured once into
 // a hipGraph and replayed; when level 0 does an odd number of sweeps per
 // cycle the phi_0 buffers swap roles every cycle, so two graphs (one per
-// starting buffer) are captured and alternated.  The host reads the 8-byte
-// error after each cycle to apply the reference's stopping rule exactly.
+// starting buffer) are captured and alternated.  The host reads the errors
+// of a chunk of cycles to apply the reference's stopping rule exactly.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -191,7 +191,7 @@ hipError_t emit_level(gpaw_poisson* ps, int l, double*& cur0, double*& alt0, hip
             e = np == ps->np0 ? hipSuccess : hipErrorInvalidValue;
         else
             e = launch_reduce_partials(op->partial, np, ps->dv,
-                                       ps->err_dst ? ps->err_dst : ps->d_err, st);
+                                       ps->err_dst ? ps->err_dst : ps->h_err, st);
     }
     cur0 = cur;
     alt0 = alt;
@@ -222,7 +222,7 @@ int capture(gpaw_poisson* ps)
     return GPAW_OK;
 }
 
-// k V-cycles; the error after cycle i goes to d_errs[i].
+// k V-cycles; the error after cycle i goes to h_errs[i].
 // Jacobi: from phiA[0]; cycle i reads S_i and leaves its result in
 // S_{i+1} = snap[i] (S_0 = phiA[0]) without writing S_i, its other sweeps
 // going to phiB[0] and tmp2; then S_k is copied to phiA[0] for the next
@@ -273,13 +273,13 @@ hipError_t emit_chunk(gpaw_poisson* ps, int k, int state, hipStream_t st)
         // the k norms: row i of the partials, in the order of one reduction
         // launch per cycle
         if (e == hipSuccess)
-            e = launch_reduce_rows(ps->d_chunk_partials, k, ps->np0, ps->dv, ps->d_errs, st);
+            e = launch_reduce_rows(ps->d_chunk_partials, k, ps->np0, ps->dv, ps->h_errs, st);
         if (e == hipSuccess) e = launch_copy(ps->phiA[0], ps->snap[k - 1], DT_F64, ps->npts[0], st);
         return e;
     }
     for (int i = 0; i < k && e == hipSuccess; i++) {
         e = launch_copy(ps->snap[i], state ? ps->phiB[0] : ps->phiA[0], DT_F64, ps->npts[0], st);
-        ps->err_dst = ps->d_errs + i;
+        ps->err_dst = ps->h_errs + i;
         if (e == hipSuccess) e = emit_cycle(ps, state, st);
         ps->err_dst = nullptr;
         state ^= ps->swaps;
@@ -298,8 +298,6 @@ int ensure_chunks(gpaw_poisson* ps)
         rc = alloc(&ps->tmp2, ps->npts[0]);
         if (!rc) rc = alloc(&ps->d_chunk_partials, (long long)GPAW_CHUNK_MAX * ps->np0);
     }
-    if (!rc) rc = alloc(&ps->d_errs, GPAW_CHUNK_MAX);
-    if (!rc) rc = alloc(&ps->d_sum, 1024);
     if (!rc)
         rc = gpaw_check(hipHostMalloc((void**)&ps->h_errs, sizeof(double) * GPAW_CHUNK_MAX),
                         "poisson: pinned errors");
@@ -312,10 +310,6 @@ int ensure_chunks(gpaw_poisson* ps)
         ps->tmp2 = nullptr;
         if (ps->d_chunk_partials) hipFree(ps->d_chunk_partials);
         ps->d_chunk_partials = nullptr;
-        if (ps->d_errs) hipFree(ps->d_errs);
-        ps->d_errs = nullptr;
-        if (ps->d_sum) hipFree(ps->d_sum);
-        ps->d_sum = nullptr;
     }
     return rc;
 }
@@ -345,8 +339,7 @@ int run_cycle(gpaw_poisson* ps, int state, hipStream_t st)
 
 int read_error(gpaw_poisson* ps, hipStream_t st, double* err)
 {
-    hipError_t e = hipMemcpyAsync(ps->h_err, ps->d_err, sizeof(double), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    hipError_t e = hipStreamSynchronize(st);
     if (e != hipSuccess) return gpaw_check(e, "poisson: error readback");
     *err = ps->h_err[0];
     return GPAW_OK;
@@ -430,7 +423,10 @@ extern "C" int gpaw_poisson_new(int levels, gpaw_operator* const* ops,
             rc = gpaw_check(e, "poisson: stencil upload");
         }
     }
-    if (!rc) rc = alloc(&ps->d_err, 1);
+    if (!rc) rc = alloc(&ps->d_sum, SUM_PARTIALS);
+    if (!rc)
+        rc = gpaw_check(hipEventCreateWithFlags(&ps->charge_ev, hipEventDisableTiming),
+                        "poisson: event");
     if (!rc) rc = gpaw_check(hipHostMalloc((void**)&ps->h_err, sizeof(double)), "poisson: pinned");
     if (rc) {
         gpaw_poisson_free(ps);
@@ -569,8 +565,16 @@ extern "C" int gpaw_poisson_vcycles(gpaw_poisson* ps, double* phi, const double*
     return rc;
 }
 
+// What a solve whose V-cycles started before the charge was known still has
+// to read: its charge, and whether that is neutral.
+struct ChargeCheck {
+    double maxcharge;
+    double* charge;
+    int* neutral;
+};
+
 static int solve_loaded(gpaw_poisson* ps, double* phi, double eps, int maxiter, int* niter,
-                        double* error, hipStream_t st);
+                        double* error, const ChargeCheck* check, hipStream_t st);
 
 extern "C" int gpaw_poisson_solve_neutral(gpaw_poisson* ps, double* phi, const double* rho,
                                           double eps, int maxiter, int* niter, double* error,
@@ -580,7 +584,28 @@ extern "C" int gpaw_poisson_solve_neutral(gpaw_poisson* ps, double* phi, const d
     hipStream_t st = (hipStream_t)stream;
     int rc = load_inputs(ps, phi, rho, st);
     if (rc) return rc;
-    return solve_loaded(ps, phi, eps, maxiter, niter, error, st);
+    return solve_loaded(ps, phi, eps, maxiter, niter, error, nullptr, st);
+}
+
+// The charge dv * sum(rho) of gd.integrate into h_err[0] (same kernels and
+// summation order as gpaw_sum) and rho minus its mean, as gpaw/poisson.py:130-138
+// computes it, into the plan's level-0 rho; nothing is waited for.
+static int launch_neutralize(gpaw_poisson* ps, const double* rho, hipStream_t st)
+{
+    ps->rho_loaded = false;
+    int rc = pretune(ps, st);   // works on the plan's arrays: first
+    if (rc) return rc;
+    return gpaw_check(launch_sub_mean(ps->rho[0], rho, ps->npts[0], ps->dv, ps->dv, ps->d_sum,
+                                      ps->h_err, st), "poisson: charge");
+}
+
+// the charge once the launches above are done
+static void read_charge(gpaw_poisson* ps, const ChargeCheck& c)
+{
+    const double q = ps->h_err[0];
+    *c.charge = q;
+    *c.neutral = std::fabs(q) <= c.maxcharge;   // charged: the caller's branches
+    ps->was_neutral = *c.neutral != 0;
 }
 
 extern "C" int gpaw_poisson_neutralize(gpaw_poisson* ps, const double* rho, double maxcharge,
@@ -589,32 +614,11 @@ extern "C" int gpaw_poisson_neutralize(gpaw_poisson* ps, const double* rho, doub
     if (!ps || !rho || !charge || !neutral) return gpaw_fail(GPAW_EINVAL, "poisson: bad argument");
     hipStream_t st = (hipStream_t)stream;
     *neutral = 0;
-    ps->rho_loaded = false;
-    int rc = ensure_chunks(ps);
+    int rc = launch_neutralize(ps, rho, st);
+    if (!rc) rc = gpaw_check(hipStreamSynchronize(st), "poisson: charge");
     if (rc) return rc;
-    // the charge integral dv * sum(rho) of gd.integrate, the same kernels
-    // and summation order as gpaw_sum
-    const long long n = ps->npts[0];
-    int np = 0;
-    hipError_t e = launch_sum(rho, n, ps->d_sum, &np, st);
-    if (e == hipSuccess) e = launch_reduce_partials(ps->d_sum, np, ps->dv, ps->d_err, st);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(ps->h_err, ps->d_err, sizeof(double), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) return gpaw_check(e, "poisson: charge");
-    const double q = ps->h_err[0];
-    *charge = q;
-    if (!(std::fabs(q) <= maxcharge)) return GPAW_OK;   // charged: the caller's branches
-    // neutral: rho minus its mean, as gpaw/poisson.py:130-138 computes it,
-    // written straight into the plan's level-0 rho (the eager pre-tuning
-    // V-cycle, which works on the plan's arrays, runs first)
-    rc = pretune(ps, st);
-    if (rc) return rc;
-    const double background = q / ps->dv / (double)n;
-    e = launch_sub_scalar(ps->rho[0], rho, background, n, st);
-    if (e != hipSuccess) return gpaw_check(e, "poisson: load");
-    ps->rho_loaded = true;
-    *neutral = 1;
+    read_charge(ps, {maxcharge, charge, neutral});
+    ps->rho_loaded = *neutral != 0;
     return GPAW_OK;
 }
 
@@ -624,17 +628,44 @@ extern "C" int gpaw_poisson_solve(gpaw_poisson* ps, double* phi, const double* r
 {
     if (!ps || !phi || !rho || !charge || !neutral || maxiter < 1)
         return gpaw_fail(GPAW_EINVAL, "poisson: bad argument");
-    int rc = gpaw_poisson_neutralize(ps, rho, maxcharge, charge, neutral, stream);
-    if (rc || !*neutral) return rc;
-    ps->rho_loaded = false;
     hipStream_t st = (hipStream_t)stream;
+    // After a neutral density (as in every step of an SCF loop) the first
+    // V-cycles are launched before the charge is read: waiting for it first left
+    // the GPU idle for about 40 us.  On a charged one they are thrown away: phi is
+    // written only once the charge is known.
+    const ChargeCheck check = {maxcharge, charge, neutral};
+    const bool early = ps->was_neutral;
+    int rc;
+    if (early) {
+        *neutral = 0;
+        rc = launch_neutralize(ps, rho, st);
+        if (!rc) rc = gpaw_check(hipEventRecord(ps->charge_ev, st), "poisson: charge");
+    } else {
+        rc = gpaw_poisson_neutralize(ps, rho, maxcharge, charge, neutral, stream);
+        if (!rc && !*neutral) return GPAW_OK;
+    }
+    if (rc) return rc;
+    ps->rho_loaded = false;
     rc = gpaw_check(launch_copy(ps->phiA[0], phi, DT_F64, ps->npts[0], st), "poisson: load");
     if (rc) return rc;
-    return solve_loaded(ps, phi, eps, maxiter, niter, error, st);
+    return solve_loaded(ps, phi, eps, maxiter, niter, error, early ? &check : nullptr, st);
+}
+
+extern "C" int gpaw_poisson_remove_mean(gpaw_poisson* ps, int on)
+{
+    if (!ps) return gpaw_fail(GPAW_EINVAL, "poisson: bad argument");
+    ps->remove_mean = on != 0;
+    return GPAW_OK;
+}
+
+hipError_t gpaw_poisson_store(gpaw_poisson* ps, double* phi, const double* result, hipStream_t st)
+{
+    if (!ps->remove_mean) return launch_copy(phi, result, DT_F64, ps->npts[0], st);
+    return launch_sub_mean(phi, result, ps->npts[0], ps->dv, ps->dv, ps->d_sum, nullptr, st);
 }
 
 static int solve_loaded(gpaw_poisson* ps, double* phi, double eps, int maxiter, int* niter,
-                        double* error, hipStream_t st)
+                        double* error, const ChargeCheck* check, hipStream_t st)
 {
     int rc = ensure_chunks(ps);
     if (rc) return rc;
@@ -655,13 +686,25 @@ static int solve_loaded(gpaw_poisson* ps, double* phi, double eps, int maxiter, 
     int n = 0;         // V-cycles accepted so far
     double err = 0.0;
     double prev = -1.0, rate = -1.0;
+    const bool hinted = ps->hint > 0 && ps->hint_eps == eps && ps->hint <= GPAW_CHUNK_MAX;
     int k = (ps->hint > 0 && ps->hint_eps == eps) ? std::min(ps->hint, GPAW_CHUNK_MAX) : 2;
+    bool expect = hinted;      // the chunk is expected to end at the stopping cycle
+    bool stored = false;       // the chunk's last phi was stored before its errors were read
     for (;;) {
         if (k > maxiter - n) k = maxiter - n;
         rc = run_chunk(ps, k, state, st);
         if (rc) return rc;
-        hipError_t e = hipMemcpyAsync(ps->h_errs, ps->d_errs, sizeof(double) * k,
-                                      hipMemcpyDeviceToHost, st);
+        hipError_t e = hipSuccess;
+        if (check) {           // the charge came back while the chunk was launched
+            e = hipEventSynchronize(ps->charge_ev);
+            if (e != hipSuccess) return gpaw_check(e, "poisson: charge");
+            read_charge(ps, *check);
+            if (!*check->neutral)
+                return gpaw_check(hipStreamSynchronize(st), "poisson: charge");
+            check = nullptr;
+        }
+        stored = jac && expect;
+        if (stored) e = gpaw_poisson_store(ps, phi, ps->snap[k - 1], st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e != hipSuccess) return gpaw_check(e, "poisson: error readback");
         int stop = -1;
@@ -677,6 +720,7 @@ static int solve_loaded(gpaw_poisson* ps, double* phi, double eps, int maxiter, 
         }
         if (stop >= 0 && jac) {
             result = ps->snap[stop];
+            stored = stored && stop == k - 1 && n < maxiter;
             break;
         }
         if (stop >= 0) {
@@ -691,13 +735,20 @@ static int solve_loaded(gpaw_poisson* ps, double* phi, double eps, int maxiter, 
         if (!jac) state ^= ps->swaps & (k & 1);
         // cycles still needed at the observed rate
         k = GPAW_CHUNK_MAX;
+        expect = false;
         if (rate > 0 && rate < 1 && err > eps) {
             const double m = std::ceil(std::log(eps / err) / std::log(rate));
-            if (m >= 1 && m < GPAW_CHUNK_MAX) k = (int)m;
+            if (m >= 1 && m < GPAW_CHUNK_MAX) {
+                k = (int)m;
+                expect = true;
+            }
         }
     }
     if (!result) result = state ? ps->phiB[0] : ps->phiA[0];
-    rc = gpaw_check(launch_copy(phi, result, DT_F64, ps->npts[0], st), "poisson: store");
+    // a solve that did not converge leaves phi with its mean
+    if (!stored)
+        rc = gpaw_check(n == maxiter ? launch_copy(phi, result, DT_F64, ps->npts[0], st)
+                                     : gpaw_poisson_store(ps, phi, result, st), "poisson: store");
     if (niter) *niter = n;
     if (error) *error = err;
     if (rc) return rc;
@@ -717,15 +768,14 @@ extern "C" void gpaw_poisson_free(gpaw_poisson* ps)
     for (auto v : {&ps->phiA, &ps->phiB, &ps->rho, &ps->res})
         for (double* p : *v)
             if (p) hipFree(p);
-    if (ps->d_err) hipFree(ps->d_err);
     for (hipGraphExec_t g : ps->chunk)
         if (g) hipGraphExecDestroy(g);
     for (double* p : ps->snap)
         if (p) hipFree(p);
     if (ps->tmp2) hipFree(ps->tmp2);
     if (ps->d_chunk_partials) hipFree(ps->d_chunk_partials);
-    if (ps->d_errs) hipFree(ps->d_errs);
     if (ps->d_sum) hipFree(ps->d_sum);
+    if (ps->charge_ev) hipEventDestroy(ps->charge_ev);
     if (ps->h_errs) hipHostFree(ps->h_errs);
     if (ps->d_coarse) hipFree(ps->d_coarse);
     if (ps->d_coarse_nb) hipFree(ps->d_coarse_nb);

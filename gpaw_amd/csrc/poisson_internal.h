@@ -20,7 +20,9 @@ struct gpaw_poisson {
     std::vector<double> w;
     std::vector<double*> phiA, phiB, rho, res;
     std::vector<long long> npts;
-    double* d_err = nullptr;
+    // pinned host memory that kernels write and the host reads after a wait: the
+    // error of a single cycle or the charge, and the errors of a chunk.  A copy
+    // back from device memory would cost a launch and its gaps, about 15 us
     double* h_err = nullptr;
     double* err_dst = nullptr;  // where the level-0 norm of the next emitted cycle goes
     // when set: the level-0 norm partials of the next emitted cycle go here
@@ -42,8 +44,13 @@ struct gpaw_poisson {
         double* t[2] = {nullptr, nullptr};
         int done = 0, total = 0;
     } rot;
-    double* d_errs = nullptr;
-    double* d_sum = nullptr;   // 1024 partial sums of the charge integral
+    double* d_sum = nullptr;   // partial sums of the charge and mean integrals
+    hipEvent_t charge_ev = nullptr;   // after the charge integral
+    // the last density was neutral: the next solve starts its V-cycles before
+    // it has read the charge back
+    bool was_neutral = false;
+    // solutions leave with their mean removed (gpaw_poisson_remove_mean)
+    bool remove_mean = false;
     // rho[0] holds a density gpaw_poisson_neutralize wrote (a solve may
     // then take rho = nullptr)
     bool rho_loaded = false;
@@ -77,3 +84,5 @@ struct gpaw_poisson {
 };
 
 void gpaw_mixed_free(MixedState* m);
+// phi = result, its mean removed where the plan says so
+hipError_t gpaw_poisson_store(gpaw_poisson* ps, double* phi, const double* result, hipStream_t st);

@@ -5,8 +5,8 @@ the finest grid, 7-point operators and K=2 transformers below it), smoothing
 counts (2/1 on level 0, 4/4 below, 8 on the coarsest), Jacobi weights
 (2/3, then 1), stopping rule (dv * sum r^2 <= eps, at most maxiter V-cycles)
 and charged-system branches.  The V-cycle itself runs in libgpaw_amd.so as
-one captured hipGraph per cycle (gpaw_poisson_solve_neutral); Python only
-prepares the neutral density and reads back one number per cycle.
+captured hipGraphs (gpaw_poisson_solve), with one host round trip for the
+errors of a whole solve of a familiar density.
 """
 import ctypes
 from math import pi, sqrt
@@ -123,6 +123,8 @@ class PoissonSolver:
             L, opa, ra, ia, pre, post, w, self.relax_method, float(self.dv),
             ctypes.byref(h)))
         self._plan = h
+        # phi's mean is removed on periodic grids
+        _lib.check(_lib.lib().gpaw_poisson_remove_mean(h, int(np.all(self.gd.pbc_c))))
 
     def __del__(self):
         p = getattr(self, '_plan', None)
@@ -221,16 +223,8 @@ class PoissonSolver:
                 'Poisson solver did not converge in %d iterations!' %
                 self.maxiter)
         _lib.check(rc)
-        return self._finish_neutral(P, niter.value), q.value
-
-    def _finish_neutral(self, P, niter):
-        """The end of solve_neutral: phi's mean removed on periodic grids."""
-        if np.all(self.gd.pbc_c):
-            phi_ave = self.gd.integrate(P.tensor) / self.gd.dv
-            phi_ave /= np.prod(self.gd.get_size_of_global_array())
-            ops.sub_scalar(P.tensor, P.tensor, phi_ave)
         P.finish()
-        return niter
+        return niter.value, q.value
 
     def _args(self, phi, rho):
         """phi (written) and rho as device arguments; both must be float64
@@ -260,10 +254,6 @@ class PoissonSolver:
                 'Poisson solver did not converge in %d iterations!' %
                 self.maxiter)
         _lib.check(rc)
-        if np.all(self.gd.pbc_c):
-            phi_ave = self.gd.integrate(P.tensor) / self.gd.dv
-            phi_ave /= np.prod(self.gd.get_size_of_global_array())
-            ops.sub_scalar(P.tensor, P.tensor, phi_ave)
         P.finish()
         return niter.value
 
@@ -379,7 +369,8 @@ class MixedPoissonSolver(PoissonSolver):
                 'mixed-precision Poisson solver did not converge in %d '
                 'iterations' % self.maxiter)
         _lib.check(rc)
-        return self._finish_neutral(P, niter.value)
+        P.finish()
+        return niter.value
 
     def smoothing_weights(self, level=0):
         """(pre, post) Jacobi weights of level `level` in the inner V-cycle,

@@ -143,10 +143,18 @@ int gpaw_poisson_neutralize(gpaw_poisson* ps, const double* rho, double maxcharg
                             double* charge, int* neutral, void* stream);
 
 /* gpaw_poisson_neutralize, then for a neutral density solve_neutral as
- * above (*neutral = 1); a charged one returns with *neutral = 0. */
+ * above (*neutral = 1); a charged one returns with *neutral = 0 and phi as it
+ * was.  After a neutral density the V-cycles are launched before the charge is
+ * read back. */
 int gpaw_poisson_solve(gpaw_poisson* ps, double* phi, const double* rho, double eps,
                        int maxiter, double maxcharge, double* charge, int* neutral,
                        int* niter, double* error, void* stream);
+
+/* on != 0: the solves above and gpaw_poisson_solve_mixed leave a converged
+ * phi with its mean removed, as solve_neutral does on periodic grids
+ * (gpaw/poisson.py:210-217): phi -= (dv * sum(phi)) / dv / npts.  Off in a new
+ * plan. */
+int gpaw_poisson_remove_mean(gpaw_poisson* ps, int on);
 
 /* Exactly ncycles V-cycles; errors[i] (host) gets dv*sum(r^2) after
  * cycle i.  Used for fixed-cycle comparisons. */
