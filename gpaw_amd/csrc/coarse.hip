@@ -1,10 +1,8 @@
 // Fused coarse-level V-cycle (gfx950): the smallest levels of the multigrid
-// hierarchy are smoothed, restricted and corrected by ONE workgroup of 1024
-// threads in one launch, with a workgroup barrier between passes instead of
-// a kernel boundary.  On these grids (11^3 and below for a 95^3 problem) a
-// separate launch per pass costs more than the pass itself.  When the level
-// arrays fit, they live in LDS: only the first level's right-hand side is
-// read from HBM and its solution written back.
+// hierarchy are smoothed, restricted and corrected by ONE workgroup in one
+// launch, with a workgroup barrier between passes instead of a kernel
+// boundary.  On these grids (11^3 and below for a 95^3 problem) a separate
+// launch per pass costs more than the pass itself.
 //
 // The passes and their arithmetic are those of iterate2
 // (gpaw/poisson.py:245-270) on 7-point operators (Laplace nn=1) with K=2
@@ -14,6 +12,17 @@
 //   residual  r = sum_c coef_c phi[g+off_c] - rho       (c/bmgs/fd.c:41-44)
 //   restrict / interpolate   transfer_common.h
 // so the fused path is bit-identical to launching the passes one by one.
+//
+// Bound by latency: about 20 passes on one compute unit, each a round of LDS
+// reads, a chain of some 15 dependent FP64 operations and a barrier.  So
+// nothing else is left on that chain.  The plan comes as a kernel argument
+// (read from memory behind a pointer, with neighbour tables behind a second
+// one, the first pass waited for three round trips), each thread keeps its
+// points' right-hand sides and neighbour indices in registers for all passes of
+// a level, and only the phi pair of every level lives in LDS (the residual
+// takes the array the last sweep read).  The block has no more waves than the
+// first level needs.  11^3 + 5^3 (16 sweeps): 17.6 us before, 13.0 now;
+// 6 x 6 x 8 + 3 x 3 x 4: 13.0 and 7.6; 9^3 alone (8 sweeps): 6.6 and 5.0.
 #include "kernels.h"
 #include "coarse.h"
 #include "transfer_common.h"
@@ -22,90 +31,74 @@ namespace gpaw {
 
 namespace {
 
-__device__ __forceinline__ void split(int idx, const Geom& g, int& i0, int& i1, int& i2)
+// index of (j0, j1, j2), each at most one period outside, in a level's array:
+// wrapped on periodic axes; outside a zero boundary the array's element n, its
+// zero slot, which holds 0.0 for the whole kernel
+__device__ __forceinline__ int slot_of(int j0, int j1, int j2, const CoarseLevel& L, int n)
 {
-    i2 = idx % g.n[2];
-    const int t = idx / g.n[2];
-    i1 = t % g.n[1];
-    i0 = t / g.n[1];
+    const int j[3] = {j0, j1, j2};
+    int w[3];
+    bool out = false;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        w[a] = j[a];
+        if (w[a] < 0 || w[a] >= L.n[a]) {
+            if (!L.per[a]) out = true;
+            w[a] = w[a] < 0 ? w[a] + L.n[a] : w[a] - L.n[a];
+        }
+    }
+    return out ? n : (w[0] * L.n[1] + w[1]) * L.n[2] + w[2];
 }
 
-// level arrays: phi A/B, rho, residual
-enum { PA = 0, PB = 1, RHO = 2, RES = 3 };
-
-// A level has at most 2048 points (two per thread).  Each thread's points
-// and their six neighbours (z+, z-, y+, y-, x+, x-: the summation order of
-// the 7-point operator, centre first) come from the plan's table; a
-// neighbour outside a zero boundary is -1 in the table.  ZS (the LDS
-// layout): such a neighbour reads the level's zero slot instead, element n
-// of its phi arrays, which holds 0.0 for the whole kernel.
+// A thread's K points of one level: flat index (-1: none), the six neighbours
+// in summation order (z+, z-, y+, y-, x+, x-), right-hand side and phi.
+template <int K>
 struct Pts {
-    int idx[2];       // flat index, -1 when the thread has no such point
-    int nb[2][6];
+    int idx[K];
+    int i[K][3];
+    int nb[K][6];
+    double rho[K], phi[K];
 };
 
-template <bool ZS>
-__device__ __forceinline__ void level_points(const CoarseLevel& L, const short* __restrict__ tab,
-                                             Pts& p)
+__device__ __forceinline__ int points(const CoarseLevel& L) { return L.n[0] * L.n[1] * L.n[2]; }
+
+template <int K>
+__device__ __forceinline__ void level_points(const CoarseLevel& L, Pts<K>& p)
 {
-    const int n = L.g.n[0] * L.g.n[1] * L.g.n[2];
+    const int n = points(L);
 #pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int idx = threadIdx.x + 1024 * k;
+    for (int k = 0; k < K; k++) {
+        const int idx = threadIdx.x + blockDim.x * k;
         p.idx[k] = idx < n ? idx : -1;
-        const short* t = tab + L.nb_off + 6 * (idx < n ? idx : 0);
+        const int i2 = idx % L.n[2], t = idx / L.n[2], i1 = t % L.n[1], i0 = t / L.n[1];
+        p.i[k][0] = i0;
+        p.i[k][1] = i1;
+        p.i[k][2] = i2;
+        p.rho[k] = p.phi[k] = 0.0;
 #pragma unroll
-        for (int m = 0; m < 6; m++) p.nb[k][m] = (ZS && t[m] < 0) ? n : t[m];
+        for (int m = 0; m < 6; m++) p.nb[k][m] = n;
+        if (idx < n) {
+            p.nb[k][0] = slot_of(i0, i1, i2 + 1, L, n);
+            p.nb[k][1] = slot_of(i0, i1, i2 - 1, L, n);
+            p.nb[k][2] = slot_of(i0, i1 + 1, i2, L, n);
+            p.nb[k][3] = slot_of(i0, i1 - 1, i2, L, n);
+            p.nb[k][4] = slot_of(i0 + 1, i1, i2, L, n);
+            p.nb[k][5] = slot_of(i0 - 1, i1, i2, L, n);
+        }
     }
 }
 
-// x + the six neighbour terms in summation order (the coarse levels are
-// real, phases 1, so a neighbour is a plain load or zero).  A zero
-// neighbour contributes 0.0 * c either way: the same bits with or without
-// the zero slot.
-template <bool ZS>
-__device__ __forceinline__ double nb_sum(const double* __restrict__ a, const int* nb,
-                                         const double* c, double x)
+// x + the six neighbour terms in summation order.  A zero neighbour adds
+// 0.0 * c as the standalone kernels do.
+__device__ __forceinline__ double nb_sum(const double* a, const int* nb, const double* c, double x)
 {
-    // every load issued unconditionally (without the zero slot: index 0 for
-    // a zero neighbour, whose value is then replaced by 0): no branch
-    // between the loads
     double v[6];
 #pragma unroll
-    for (int m = 0; m < 6; m++) v[m] = a[(ZS || nb[m] >= 0) ? nb[m] : 0];
+    for (int m = 0; m < 6; m++) v[m] = a[nb[m]];
 #pragma unroll
-    for (int m = 0; m < 6; m++) x = x + ((ZS || nb[m] >= 0) ? v[m] : 0.0) * c[m + 1];
+    for (int m = 0; m < 6; m++) x = x + v[m] * c[m + 1];
     return x;
 }
-
-// The four arrays of one level.  In LDS mode they are derived from the
-// kernel's shared array, so the compiler addresses them as LDS (ds_read /
-// ds_write); from a pointer table in memory it could only use flat
-// accesses, which take the vector-memory path even for LDS.
-struct LevelArrays {
-    double* a[4];
-};
-
-template <bool LDS>
-__device__ __forceinline__ LevelArrays level_arrays(const CoarseLevel& L, double* smem)
-{
-    LevelArrays r;
-    if (LDS) {   // n + 1 elements each: element n of phi A / B is the zero slot
-        const int n = L.g.n[0] * L.g.n[1] * L.g.n[2];
-#pragma unroll
-        for (int k = 0; k < 4; k++) r.a[k] = smem + L.off + k * (n + 1);
-    } else {
-        r.a[PA] = L.phiA;
-        r.a[PB] = L.phiB;
-        r.a[RHO] = L.rho;
-        r.a[RES] = L.res;
-    }
-    return r;
-}
-
-#ifndef GPAW_COARSE_DIV_RN
-#define GPAW_COARSE_DIV_RN 1
-#endif
 
 // a / d rounded to nearest, from r = 1 / d rounded to nearest: the product
 // q = a r is within an ulp of a / d, its remainder a - q d is exact in one
@@ -121,341 +114,223 @@ __device__ __forceinline__ double div_rn(double a, double d, double r)
     return e == 0.0 ? q : __builtin_fma(e, r, q);
 }
 
-template <bool ZS>
-__device__ __forceinline__ void jacobi_sweeps(const CoarseLevel& L, const Pts& p,
-                                              const LevelArrays& A, int k, int& cur)
+// `sweeps` Jacobi sweeps between the level's arrays, from src; src is the
+// array that holds the result, dst the other one
+template <int K>
+__device__ __forceinline__ void jacobi_sweeps(const CoarseLevel& L, Pts<K>& p, int sweeps,
+                                              double*& src, double*& dst)
 {
-    const double* __restrict__ rho = A.a[RHO];
     double c[7];
 #pragma unroll
     for (int m = 0; m < 7; m++) c[m] = L.c[m];
-    const double w = L.w;
-    const double rc0 = 1.0 / c[0];
-    for (int it = 0; it < k; it++) {
-        const double* __restrict__ src = cur == PA ? A.a[PA] : A.a[PB];
-        double* __restrict__ dst = cur == PA ? A.a[PB] : A.a[PA];
+    const double w = L.w, rc0 = 1.0 / c[0];
+    for (int it = 0; it < sweeps; it++) {
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const int idx = p.idx[q];
+        for (int k = 0; k < K; k++) {
+            const int idx = p.idx[k];
             if (idx < 0) continue;
-            const double x = nb_sum<ZS>(src, p.nb[q], c, 0.0);
-            if (GPAW_COARSE_DIV_RN)
-                dst[idx] = (1.0 - w) * src[idx] + div_rn(w * (rho[idx] - x), c[0], rc0);
-            else
-                dst[idx] = (1.0 - w) * src[idx] + w * (rho[idx] - x) / c[0];
-        }
-        __syncthreads();
-        cur ^= 1;
-    }
-}
-
-}  // namespace
-
-// TB: storage type of the first level's right-hand side and solution in HBM
-// (double, or float when the fused kernel is the FP64 coarse solve of an
-// FP32 V-cycle; then the arrays must live in LDS and are converted there).
-// LDS: the level arrays live in the kernel's shared memory (plan->lds).
-template <class TB, bool LDS>
-__global__ __launch_bounds__(1024) void k_coarse_vcycle(const CoarsePlan* __restrict__ Pg)
-{
-    extern __shared__ double smem[];
-    // the plan is read from an LDS copy: its fields are read at every phase,
-    // and from global memory each such read would miss the scalar cache
-    // (the kernel runs once per V-cycle, between much larger kernels)
-    __shared__ CoarsePlan Ps;
-    {
-        static_assert(sizeof(CoarsePlan) % 4 == 0, "plan copied in 4-byte words");
-        const int* src = (const int*)Pg;
-        int* dst = (int*)&Ps;
-        for (int i = threadIdx.x; i < (int)(sizeof(CoarsePlan) / 4); i += blockDim.x)
-            dst[i] = src[i];
-        __syncthreads();
-    }
-    const CoarsePlan* P = &Ps;
-    // neighbour tables: copied next to the level arrays in LDS mode
-    const short* tab = P->nbtab;
-    if (LDS) {
-        int* dst = (int*)(smem + P->lds_doubles);
-        const int* src = (const int*)P->nbtab;
-        for (int i = threadIdx.x; i < P->nb_words; i += blockDim.x) dst[i] = src[i];
-        tab = (const short*)dst;
-        // the zero slots (LDS starts undefined)
-        for (int l = threadIdx.x; l < P->nlev; l += blockDim.x) {
-            const CoarseLevel& L = P->lev[l];
-            const int n = L.g.n[0] * L.g.n[1] * L.g.n[2];
-            smem[L.off + n] = 0.0;
-            smem[L.off + (n + 1) + n] = 0.0;
-        }
-        // made visible by the barrier after the first level's load below
-    }
-    Phases ph;
-    for (int a = 0; a < 3; a++)
-        for (int d = 0; d < 2; d++) {
-            ph.re[a][d] = 1.0;
-            ph.im[a][d] = 0.0;
-        }
-    const int nl = P->nlev;
-    if (LDS) {   // right-hand side of the first coarse level, phi = 0
-        const CoarseLevel& G = P->lev[0];
-        const LevelArrays A = level_arrays<LDS>(G, smem);
-        const int n = G.g.n[0] * G.g.n[1] * G.g.n[2];
-        const TB* __restrict__ grho = (const TB*)G.rho;
-        for (int idx = threadIdx.x; idx < n; idx += blockDim.x) {
-            A.a[RHO][idx] = (double)grho[idx];
-            A.a[PA][idx] = 0.0;
-        }
-        __syncthreads();
-    }
-    // down: pre-smooth, residual, restrict (phi of the next level zeroed)
-    for (int l = 0; l < nl - 1; l++) {
-        const CoarseLevel& L = P->lev[l];
-        const LevelArrays A = level_arrays<LDS>(L, smem);
-        Pts pts;
-        level_points<LDS>(L, tab, pts);
-        int cur = PA;
-        jacobi_sweeps<LDS>(L, pts, A, L.pre, cur);
-        const double* __restrict__ phi = cur == PA ? A.a[PA] : A.a[PB];
-        const double* __restrict__ rho = A.a[RHO];
-        double* __restrict__ res = A.a[RES];
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const int idx = pts.idx[q];
-            if (idx < 0) continue;
-            double c[7];
-#pragma unroll
-            for (int m = 0; m < 7; m++) c[m] = L.c[m];
-            res[idx] = nb_sum<LDS>(phi, pts.nb[q], c, 0.0 + phi[idx] * c[0]) - rho[idx];
-        }
-        __syncthreads();
-        const CoarseLevel& N = P->lev[l + 1];
-        const LevelArrays NA = level_arrays<LDS>(N, smem);
-        const int m = N.g.n[0] * N.g.n[1] * N.g.n[2];
-        for (int idx = threadIdx.x; idx < m; idx += blockDim.x) {
-            int o0, o1, o2;
-            split(idx, N.g, o0, o1, o2);
-            NA.a[RHO][idx] = restrict_point<double, 2>(res, o0, o1, o2, L.rst, ph);
-            NA.a[PA][idx] = 0.0;
-        }
-        __syncthreads();
-    }
-    {   // bottom: post-smooth only
-        const CoarseLevel& L = P->lev[nl - 1];
-        const LevelArrays A = level_arrays<LDS>(L, smem);
-        Pts pts;
-        level_points<LDS>(L, tab, pts);
-        int cur = PA;
-        jacobi_sweeps<LDS>(L, pts, A, L.post, cur);
-    }
-    // up: correct from the coarser level, post-smooth
-    for (int l = nl - 2; l >= 0; l--) {
-        const CoarseLevel& L = P->lev[l];
-        const CoarseLevel& N = P->lev[l + 1];
-        const LevelArrays A = level_arrays<LDS>(L, smem);
-        const LevelArrays NA = level_arrays<LDS>(N, smem);
-        int cur = (L.pre & 1) ? PB : PA;
-        const int kc = (l + 1 < nl - 1 ? N.pre : 0) + N.post;
-        const double* __restrict__ coarse = (kc & 1) ? NA.a[PB] : NA.a[PA];
-        double* __restrict__ phi = cur == PA ? A.a[PA] : A.a[PB];
-        // one coarse cell (2 x 2 x 2 fine points) per thread, as k_interp2
-        const int nc0 = interp2_cells(L.itp, 0), nc1 = interp2_cells(L.itp, 1),
-                  nc2 = interp2_cells(L.itp, 2);
-        for (int idx = threadIdx.x; idx < nc0 * nc1 * nc2; idx += blockDim.x) {
-            const int k2 = idx % nc2, k1 = (idx / nc2) % nc1, k0 = idx / (nc2 * nc1);
-            interp2_cell<double, TR_SUBTRACT>(coarse, phi, L.itp, k0, k1, k2, ph);
-        }
-        __syncthreads();
-        Pts pts;
-        level_points<LDS>(L, tab, pts);
-        jacobi_sweeps<LDS>(L, pts, A, L.post, cur);
-    }
-    if (LDS) {   // hand the first level's solution back where the caller expects it
-        const CoarseLevel& G = P->lev[0];
-        const LevelArrays A = level_arrays<LDS>(G, smem);
-        const int k = (nl > 1 ? G.pre : 0) + G.post;
-        const double* src = (k & 1) ? A.a[PB] : A.a[PA];
-        TB* dst = (TB*)((k & 1) ? G.phiB : G.phiA);
-        const int n = G.g.n[0] * G.g.n[1] * G.g.n[2];
-        for (int idx = threadIdx.x; idx < n; idx += blockDim.x) dst[idx] = (TB)src[idx];
-    }
-}
-
-// The single-coarse-level case (the hierarchy's last level alone, as for a
-// 159^3 problem, whose 19^3 level is too large for one workgroup and 9^3
-// is the last): post-smoothing sweeps only, in a compact kernel whose
-// parameters arrive as kernel arguments.  The generic kernel first copies
-// its plan and neighbour table in, two dependent round trips; here the
-// neighbour indices are computed per point.  Same sweep arithmetic as
-// jacobi_sweeps.
-namespace {
-
-// flat index of (j0, j1, j2), wrapped on periodic axes, -1 outside a zero
-// boundary (the neighbour table's rule)
-__device__ __forceinline__ int one_nb(int j0, int j1, int j2, const Geom& g)
-{
-    const int j[3] = {j0, j1, j2};
-    int w[3];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        w[a] = j[a];
-        if (w[a] < 0 || w[a] >= g.n[a]) {
-            if (!g.per[a]) return -1;
-            w[a] = w[a] < 0 ? w[a] + g.n[a] : w[a] - g.n[a];
-        }
-    }
-    return (w[0] * g.n[1] + w[1]) * g.n[2] + w[2];
-}
-
-template <class TB>
-__global__ __launch_bounds__(1024) void k_coarse_one(CoarseOne p)
-{
-    extern __shared__ double smem[];
-    const int n = p.g.n[0] * p.g.n[1] * p.g.n[2];
-    // phi A / B with their zero slots (element n), then rho
-    double* A = smem;
-    double* B = smem + (n + 1);
-    double* rho = smem + 2 * (n + 1);
-    if (threadIdx.x == 0) {
-        A[n] = 0.0;
-        B[n] = 0.0;
-    }
-    Pts q;
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int idx = threadIdx.x + 1024 * k;
-        q.idx[k] = idx < n ? idx : -1;
-        int i0 = 0, i1 = 0, i2 = 0;
-        if (idx < n) split(idx, p.g, i0, i1, i2);
-        q.nb[k][0] = one_nb(i0, i1, i2 + 1, p.g);
-        q.nb[k][1] = one_nb(i0, i1, i2 - 1, p.g);
-        q.nb[k][2] = one_nb(i0, i1 + 1, i2, p.g);
-        q.nb[k][3] = one_nb(i0, i1 - 1, i2, p.g);
-        q.nb[k][4] = one_nb(i0 + 1, i1, i2, p.g);
-        q.nb[k][5] = one_nb(i0 - 1, i1, i2, p.g);
-#pragma unroll
-        for (int m = 0; m < 6; m++)
-            if (q.nb[k][m] < 0) q.nb[k][m] = n;
-        if (idx < n) {
-            rho[idx] = (double)((const TB*)p.rho)[idx];
-            A[idx] = 0.0;
-        }
-    }
-    __syncthreads();
-    double c[7];
-#pragma unroll
-    for (int m = 0; m < 7; m++) c[m] = p.c[m];
-    const double w = p.w;
-    const double rc0 = 1.0 / c[0];
-    double* src = A;
-    double* dst = B;
-    for (int it = 0; it < p.sweeps; it++) {
-#pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const int idx = q.idx[k];
-            if (idx < 0) continue;
-            const double x = nb_sum<true>(src, q.nb[k], c, 0.0);
-            if (GPAW_COARSE_DIV_RN)
-                dst[idx] = (1.0 - w) * src[idx] + div_rn(w * (rho[idx] - x), c[0], rc0);
-            else
-                dst[idx] = (1.0 - w) * src[idx] + w * (rho[idx] - x) / c[0];
+            const double x = nb_sum(src, p.nb[k], c, 0.0);
+            p.phi[k] = (1.0 - w) * p.phi[k] + div_rn(w * (p.rho[k] - x), c[0], rc0);
+            dst[idx] = p.phi[k];
         }
         __syncthreads();
         double* t = src;
         src = dst;
         dst = t;
     }
+}
+
+// one restriction pass of K = 2: 0.5 * (centre + 0.5 * (plus + minus))
+__device__ __forceinline__ double rst_pass(double c, double p, double m)
+{
+    return (c + (p + m) * 0.5) * 0.5;
+}
+
+// the restriction of `res`, an array of level L, at point i of the next one
+__device__ __forceinline__ double restrict_at(const double* res, const CoarseLevel& L, const int* i)
+{
+    const int n = points(L);
+    const int c0 = 1 + 2 * i[0] - L.rlo[0], c1 = 1 + 2 * i[1] - L.rlo[1],
+              c2 = 1 + 2 * i[2] - L.rlo[2];
+    double v[3][3][3];   // centre, plus, minus per axis
 #pragma unroll
-    for (int k = 0; k < 2; k++)
-        if (q.idx[k] >= 0) ((TB*)p.out)[q.idx[k]] = (TB)src[q.idx[k]];
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int b = 0; b < 3; b++)
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+                v[a][b][c] = res[slot_of(c0 + (a == 2 ? -1 : a), c1 + (b == 2 ? -1 : b),
+                                         c2 + (c == 2 ? -1 : c), L, n)];
+    double y[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        double z[3];
+#pragma unroll
+        for (int b = 0; b < 3; b++) z[b] = rst_pass(v[a][b][0], v[a][b][1], v[a][b][2]);
+        y[a] = rst_pass(z[0], z[1], z[2]);
+    }
+    return rst_pass(y[0], y[1], y[2]);
+}
+
+// the interpolation of `e`, an array of level N, at point i of the finer level L
+__device__ __forceinline__ double interp_at(const double* e, const CoarseLevel& L,
+                                            const CoarseLevel& N, const int* i)
+{
+    const int n = points(N);
+    const int q0 = i[0] + L.iskip[0], q1 = i[1] + L.iskip[1], q2 = i[2] + L.iskip[2];
+    const int l0 = (q0 >> 1) - L.ilo[0], l1 = (q1 >> 1) - L.ilo[1], l2 = (q2 >> 1) - L.ilo[2];
+    double v[2][2][2];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) v[a][b][c] = e[slot_of(l0 + a, l1 + b, l2 + c, N, n)];
+    return interp2_combine<double>([&](int a, int b, int c) { return v[a][b][c]; }, q0 & 1, q1 & 1,
+                                   q2 & 1);
+}
+
+// level l down: pre-smooth, residual into the other array
+template <int K>
+__device__ __forceinline__ void descend(const CoarseLevel& L, Pts<K>& p, double*& cur,
+                                        double*& alt)
+{
+    jacobi_sweeps(L, p, L.pre, cur, alt);
+    double c[7];
+#pragma unroll
+    for (int m = 0; m < 7; m++) c[m] = L.c[m];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int idx = p.idx[k];
+        if (idx >= 0) alt[idx] = nb_sum(cur, p.nb[k], c, 0.0 + p.phi[k] * c[0]) - p.rho[k];
+    }
+    __syncthreads();
+}
+
+// level l up: correct from e on the coarser level N, post-smooth
+template <int K>
+__device__ __forceinline__ void ascend(const CoarseLevel& L, const CoarseLevel& N,
+                                       Pts<K>& p, const double* e, double*& cur, double*& alt)
+{
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int idx = p.idx[k];
+        if (idx >= 0) {
+            p.phi[k] = p.phi[k] - interp_at(e, L, N, p.i[k]);
+            cur[idx] = p.phi[k];
+        }
+    }
+    __syncthreads();
+    jacobi_sweeps(L, p, L.post, cur, alt);
+}
+
+// PPT: points per thread of the first level; the others have one
+template <class TB, int NL, int PPT>
+__global__ __launch_bounds__(1024) void k_coarse_vcycle(const CoarsePlan P)
+{
+    extern __shared__ double smem[];
+    // per level: the array the last pass wrote, and the other one
+    double *cur[NL], *alt[NL];
+    Pts<PPT> p0;
+    Pts<1> p[NL];   // p[0] is not used
+#pragma unroll
+    for (int l = 0; l < NL; l++) {
+        const int n = points(P.lev[l]);
+        cur[l] = smem + P.lev[l].off;
+        alt[l] = cur[l] + n + 1;
+        if (threadIdx.x == 0) {   // the zero slots
+            cur[l][n] = 0.0;
+            alt[l][n] = 0.0;
+        }
+    }
+    // the first level's right-hand side, on the way while indices are formed
+    const int n0 = points(P.lev[0]);
+    double rho0[PPT];
+#pragma unroll
+    for (int k = 0; k < PPT; k++) {
+        const int idx = threadIdx.x + blockDim.x * k;
+        rho0[k] = (double)((const TB*)P.rho)[idx < n0 ? idx : 0];
+    }
+    // every level starts from phi = 0
+    level_points(P.lev[0], p0);
+#pragma unroll
+    for (int k = 0; k < PPT; k++) {
+        if (p0.idx[k] >= 0) cur[0][p0.idx[k]] = 0.0;
+        p0.rho[k] = rho0[k];
+    }
+#pragma unroll
+    for (int l = 1; l < NL; l++) {
+        level_points(P.lev[l], p[l]);
+        if (p[l].idx[0] >= 0) cur[l][p[l].idx[0]] = 0.0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int l = 0; l < NL - 1; l++) {
+        if (l == 0)
+            descend(P.lev[0], p0, cur[0], alt[0]);
+        else
+            descend(P.lev[l], p[l], cur[l], alt[l]);
+        if (p[l + 1].idx[0] >= 0) p[l + 1].rho[0] = restrict_at(alt[l], P.lev[l], p[l + 1].i[0]);
+    }
+    // bottom: post-smooth only
+    if (NL == 1)
+        jacobi_sweeps(P.lev[0], p0, P.lev[0].post, cur[0], alt[0]);
+    else
+        jacobi_sweeps(P.lev[NL - 1], p[NL - 1], P.lev[NL - 1].post, cur[NL - 1], alt[NL - 1]);
+#pragma unroll
+    for (int l = NL - 2; l >= 0; l--) {
+        if (l == 0)
+            ascend(P.lev[0], P.lev[1], p0, cur[1], cur[0], alt[0]);
+        else
+            ascend(P.lev[l], P.lev[l + 1], p[l], cur[l + 1], cur[l], alt[l]);
+    }
+#pragma unroll
+    for (int k = 0; k < PPT; k++)   // each thread's own points
+        if (p0.idx[k] >= 0) ((TB*)P.out)[p0.idx[k]] = (TB)p0.phi[k];
+}
+
+template <class TB, int NL>
+hipError_t coarse_nl(const CoarsePlan& P, int nt, bool two, size_t lds, hipStream_t st)
+{
+    return two ? launch_kernel(k_coarse_vcycle<TB, NL, 2>, dim3(1), dim3(nt), lds, st, P)
+               : launch_kernel(k_coarse_vcycle<TB, NL, 1>, dim3(1), dim3(nt), lds, st, P);
+}
+
+template <class TB>
+hipError_t coarse_go(const CoarsePlan& P, hipStream_t st)
+{
+    int first = 0, rest = 1, doubles = 0;
+    for (int l = 0; l < P.nlev; l++) {
+        const int n = P.lev[l].n[0] * P.lev[l].n[1] * P.lev[l].n[2];
+        if (n < 1 || n > (l ? 1024 : GPAW_COARSE_POINTS) || P.lev[l].off != doubles)
+            return hipErrorInvalidValue;
+        if (l == 0) first = n;
+        if (l > 0 && n > rest) rest = n;
+        doubles += 2 * (n + 1);
+    }
+    // no more waves at the barriers than there are points for; beyond 1024
+    // points two for some threads (11^3: 13.0 us with 16 waves, 13.9 with 11)
+    const bool two = first > 1024;
+    const int nt = two ? 1024 : ((first > rest ? first : rest) + 63) / 64 * 64;
+    const size_t lds = sizeof(double) * doubles;
+    if (lds > 64 * 1024) return hipErrorInvalidValue;
+    switch (P.nlev) {
+    case 1: return coarse_nl<TB, 1>(P, nt, two, lds, st);
+    case 2: return coarse_nl<TB, 2>(P, nt, two, lds, st);
+    case 3: return coarse_nl<TB, 3>(P, nt, two, lds, st);
+    case 4: return coarse_nl<TB, 4>(P, nt, two, lds, st);
+    }
+    return hipErrorInvalidValue;
 }
 
 }  // namespace
 
-// the single-level kernel's arguments from a one-level plan
-static bool coarse_one_args(const CoarsePlan& h, CoarseOne& a)
+hipError_t launch_coarse_vcycle(const CoarsePlan& plan, int dtype, hipStream_t st)
 {
-    if (h.nlev != 1) return false;
-    const CoarseLevel& L = h.lev[0];
-    const long n = (long)L.g.n[0] * L.g.n[1] * L.g.n[2];
-    if (n < 1 || n > 2048) return false;
-    a.g = L.g;
-    for (int m = 0; m < 7; m++) a.c[m] = L.c[m];
-    a.w = L.w;
-    a.sweeps = L.post;
-    a.rho = L.rho;
-    a.out = (L.post & 1) ? L.phiB : L.phiA;
-    return true;
-}
-
-static int nb_host(int j0, int j1, int j2, const Geom& g)
-{
-    const int j[3] = {j0, j1, j2};
-    int w[3];
-    for (int a = 0; a < 3; a++) {
-        w[a] = j[a];
-        if (w[a] < 0 || w[a] >= g.n[a]) {
-            if (!g.per[a]) return -1;
-            w[a] = w[a] < 0 ? w[a] + g.n[a] : w[a] - g.n[a];
-        }
-    }
-    return (w[0] * g.n[1] + w[1]) * g.n[2] + w[2];
-}
-
-void coarse_neighbour_table(const Geom& g, short* tab)
-{
-    for (int i0 = 0; i0 < g.n[0]; i0++)
-        for (int i1 = 0; i1 < g.n[1]; i1++)
-            for (int i2 = 0; i2 < g.n[2]; i2++) {
-                short* t = tab + 6 * ((i0 * g.n[1] + i1) * g.n[2] + i2);
-                t[0] = (short)nb_host(i0, i1, i2 + 1, g);
-                t[1] = (short)nb_host(i0, i1, i2 - 1, g);
-                t[2] = (short)nb_host(i0, i1 + 1, i2, g);
-                t[3] = (short)nb_host(i0, i1 - 1, i2, g);
-                t[4] = (short)nb_host(i0 + 1, i1, i2, g);
-                t[5] = (short)nb_host(i0 - 1, i1, i2, g);
-            }
-}
-
-hipError_t coarse_set_lds_limit(int bytes)
-{
-    hipError_t e = hipFuncSetAttribute((const void*)k_coarse_vcycle<double, true>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute((const void*)k_coarse_vcycle<float, true>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    return e;
-}
-
-// lds_bytes > 0: the plan keeps its level arrays in LDS (plan->lds)
-hipError_t launch_coarse_vcycle(const CoarsePlan* d_plan, const CoarsePlan& h_plan, int lds_bytes,
-                                hipStream_t st)
-{
-    CoarseOne one;
-    if (coarse_one_args(h_plan, one)) {
-        const int n = one.g.n[0] * one.g.n[1] * one.g.n[2];
-        launch_kernel(k_coarse_one<double>, dim3(1), dim3(1024),
-                      3 * (n + 1) * (int)sizeof(double), st, one);
-        return launch_error();
-    }
-    if (lds_bytes > 0)
-        launch_kernel(k_coarse_vcycle<double, true>, dim3(1), dim3(1024), lds_bytes, st, d_plan);
-    else
-        launch_kernel(k_coarse_vcycle<double, false>, dim3(1), dim3(1024), 0, st, d_plan);
-    return launch_error();
-}
-
-hipError_t launch_coarse_vcycle_f32(const CoarsePlan* d_plan, const CoarsePlan& h_plan,
-                                    int lds_bytes, hipStream_t st)
-{
-    CoarseOne one;
-    if (coarse_one_args(h_plan, one)) {
-        const int n = one.g.n[0] * one.g.n[1] * one.g.n[2];
-        launch_kernel(k_coarse_one<float>, dim3(1), dim3(1024),
-                      3 * (n + 1) * (int)sizeof(double), st, one);
-        return launch_error();
-    }
-    if (lds_bytes <= 0) return hipErrorInvalidValue;   // float levels need LDS mode
-    launch_kernel(k_coarse_vcycle<float, true>, dim3(1), dim3(1024), lds_bytes, st, d_plan);
-    return launch_error();
+    hipError_t e = dtype == DT_F32   ? coarse_go<float>(plan, st)
+                   : dtype == DT_F64 ? coarse_go<double>(plan, st)
+                                     : hipErrorInvalidValue;
+    return e == hipSuccess ? launch_error() : e;
 }
 
 }  // namespace gpaw

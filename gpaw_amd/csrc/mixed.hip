@@ -48,9 +48,7 @@ struct VLevels {
     int dt = DT_F32;
     std::vector<void*> phiA, phiB, rho, res;
     std::vector<void*> owned;
-    CoarsePlan* d_coarse = nullptr;     // fused coarse levels (FP64 inside)
-    CoarsePlan h_coarse{};              // its host copy
-    bool own_coarse = false;
+    CoarsePlan coarse;                  // fused coarse levels (FP64 inside)
     int lc = -1;                        // first fused coarse level (-1: none)
 };
 
@@ -348,8 +346,7 @@ hipError_t emit_v(gpaw_poisson* ps, MixedState* m, VLevels& V, int l, bool zero0
     if (l == V.lc) {   // the fused coarse kernel leaves it where single sweeps would
         const int kc = (l < m->L ? m->pre[l] : 0) + m->post[l];
         res = (kc % 2) ? V.phiB[l] : V.phiA[l];
-        return V.dt == DT_F32 ? launch_coarse_vcycle_f32(V.d_coarse, V.h_coarse, ps->coarse_lds, st)
-                              : launch_coarse_vcycle(V.d_coarse, V.h_coarse, ps->coarse_lds, st);
+        return launch_coarse_vcycle(V.coarse, V.dt, st);
     }
     gpaw_operator* op = ps->ops[l];
     void* cur = V.phiA[l];
@@ -469,20 +466,12 @@ int setup_v32(gpaw_poisson* ps, MixedState* m)
         V.rho.push_back(r);
         V.res.push_back(x);
     }
-    // the fused FP64 coarse solve needs its arrays in LDS (FP32 boundary)
-    if (!rc && ps->lc > 0 && ps->h_coarse.lds) {
-        CoarsePlan P = ps->h_coarse;
-        P.lev[0].rho = (double*)V.rho[ps->lc];
-        P.lev[0].phiA = (double*)V.phiA[ps->lc];
-        P.lev[0].phiB = (double*)V.phiB[ps->lc];
-        V.h_coarse = P;
-        rc = gpaw_check(hipMalloc((void**)&V.d_coarse, sizeof P), "mixed: coarse plan");
-        if (!rc) {
-            V.own_coarse = true;
-            rc = gpaw_check(hipMemcpy(V.d_coarse, &P, sizeof P, hipMemcpyHostToDevice),
-                            "mixed: coarse plan");
-        }
-        if (!rc) V.lc = ps->lc;
+    if (!rc && ps->lc > 0) {
+        const bool odd = (ps->coarse.lev[0].pre + ps->coarse.lev[0].post) % 2;
+        V.coarse = ps->coarse;
+        V.coarse.rho = V.rho[ps->lc];
+        V.coarse.out = odd ? V.phiB[ps->lc] : V.phiA[ps->lc];
+        V.lc = ps->lc;
     }
     return rc;
 }
@@ -511,8 +500,7 @@ int setup_v64(gpaw_poisson* ps, MixedState* m)
         V.res.push_back(ps->res[l]);
     }
     if (ps->lc > 0) {
-        V.d_coarse = ps->d_coarse;
-        V.h_coarse = ps->h_coarse;
+        V.coarse = ps->coarse;
         V.lc = ps->lc;
     }
     return GPAW_OK;
@@ -854,7 +842,6 @@ void gpaw_mixed_free(MixedState* m)
     for (int pr = 0; pr < 2; pr++) {
         destroy_graphs(m, pr);
         for (void* p : m->v[pr].owned) hipFree(p);
-        if (m->v[pr].own_coarse && m->v[pr].d_coarse) hipFree(m->v[pr].d_coarse);
     }
     for (double* p : {m->p[0], m->p[1], m->q, m->S, m->partial})
         if (p) hipFree(p);

@@ -28,7 +28,7 @@
 using namespace gpaw;
 
 
-static int setup_coarse(gpaw_poisson* ps);
+static void setup_coarse(gpaw_poisson* ps);
 
 namespace {
 
@@ -136,7 +136,7 @@ hipError_t emit_level(gpaw_poisson* ps, int l, double*& cur0, double*& alt0, hip
         // the fused coarse kernel leaves its result where single sweeps would
         const int k = (l < ps->L ? ps->pre[l] : 0) + ps->post[l];
         cur0 = (ps->method == 2 && k % 2) ? ps->phiB[l] : ps->phiA[l];
-        return launch_coarse_vcycle(ps->d_coarse, ps->h_coarse, ps->coarse_lds, st);
+        return launch_coarse_vcycle(ps->coarse, DT_F64, st);
     }
     double* cur = l == 0 ? cur0 : ps->phiA[l];
     double* alt = l == 0 ? alt0 : ps->phiB[l];
@@ -415,7 +415,7 @@ extern "C" int gpaw_poisson_new(int levels, gpaw_operator* const* ops,
         ps->res.push_back(x);
     }
     if (!rc) rc = gpaw_op_ensure_partials(ps->ops[0]);
-    if (!rc && relax_method == 2) rc = setup_coarse(ps);
+    if (!rc && relax_method == 2) setup_coarse(ps);
     for (int l = 0; l <= levels && !rc && relax_method == 1; l++) {
         gpaw_operator* op = ps->ops[l];
         if (!op->st.d_coefs) {   // Gauss-Seidel reads the stencil table on the device
@@ -438,83 +438,49 @@ extern "C" int gpaw_poisson_new(int levels, gpaw_operator* const* ops,
 
 // Levels from lc down are run by one fused kernel when they are small and
 // all 7-point stars with K=2 transfers (the Poisson hierarchy below level 0).
-static int setup_coarse(gpaw_poisson* ps)
+static void setup_coarse(gpaw_poisson* ps)
 {
-    // the fused kernel holds at most 2048 points per level (two per thread)
+    // GPAW_AMD_COARSE_MAX: points of the first fused level, at most
     const char* env = getenv("GPAW_AMD_COARSE_MAX");
     long long limit = env ? atoll(env) : 2000;
-    if (limit > 2048) limit = 2048;
-    int lc = -1;
-    for (int l = 1; l <= ps->L; l++)
-        if (ps->npts[l] <= limit) {
-            lc = l;
-            break;
-        }
-    if (lc < 0 || ps->L - lc + 1 > GPAW_MAX_LEVELS) return GPAW_OK;
+    if (limit > GPAW_COARSE_POINTS) limit = GPAW_COARSE_POINTS;
+    int lc = ps->L + 1;
+    while (lc > 1 && ps->L - lc + 1 < GPAW_COARSE_LEVELS && ps->npts[lc - 1] <= limit &&
+           (lc > ps->L || ps->npts[lc] <= 1024))
+        lc--;
+    if (lc > ps->L) return;
     CoarsePlan P;
-    memset(&P, 0, sizeof P);
     P.nlev = ps->L - lc + 1;
+    int off = 0;
     for (int l = lc; l <= ps->L; l++) {
         const gpaw_operator* op = ps->ops[l];
-        if (op->st.star_r != 1) return GPAW_OK;
-        if (l < ps->L && (ps->rst[l]->t.K != 2 || ps->itp[l]->t.K != 2)) return GPAW_OK;
+        if (op->st.star_r != 1) return;
         CoarseLevel& C = P.lev[l - lc];
-        C.g = op->g;
+        for (int a = 0; a < 3; a++) {
+            C.n[a] = op->g.n[a];
+            C.per[a] = op->g.per[a];
+            C.rlo[a] = C.ilo[a] = C.iskip[a] = 0;
+        }
         for (int c = 0; c < 7; c++) C.c[c] = op->st.coefs[c];
         C.w = ps->w[l];
         C.pre = l < ps->L ? ps->pre[l] : 0;
         C.post = ps->post[l];
-        C.phiA = ps->phiA[l];
-        C.phiB = ps->phiB[l];
-        C.rho = ps->rho[l];
-        C.res = ps->res[l];
-        if (l < ps->L) {
-            C.rst = make_trargs(ps->rst[l]->t);
-            C.itp = make_trargs(ps->itp[l]->t);
+        C.off = off;
+        off += 2 * ((int)ps->npts[l] + 1);
+        if (l == ps->L) break;
+        const TrArgs r = make_trargs(ps->rst[l]->t), i = make_trargs(ps->itp[l]->t);
+        if (ps->rst[l]->t.K != 2 || ps->itp[l]->t.K != 2) return;
+        for (int a = 0; a < 3; a++) {
+            C.rlo[a] = r.lo[a];
+            C.ilo[a] = i.lo[a];
+            C.iskip[a] = i.skip[a][0];
         }
     }
-    // neighbour tables (6 shorts per point), built here once
-    std::vector<short> tab;
-    for (int l = lc; l <= ps->L; l++) {
-        P.lev[l - lc].nb_off = (int)tab.size();
-        tab.resize(tab.size() + 6 * ps->npts[l]);
-        coarse_neighbour_table(P.lev[l - lc].g, tab.data() + P.lev[l - lc].nb_off);
-    }
-    if (tab.size() % 2) tab.push_back(0);   // whole 4-byte words
-    P.nb_words = (int)(tab.size() / 2);
-    {
-        hipError_t e = hipMalloc((void**)&ps->d_coarse_nb, sizeof(short) * tab.size());
-        if (e == hipSuccess)
-            e = hipMemcpy(ps->d_coarse_nb, tab.data(), sizeof(short) * tab.size(),
-                          hipMemcpyHostToDevice);
-        if (e != hipSuccess) return gpaw_check(e, "poisson: coarse neighbour tables");
-        P.nbtab = ps->d_coarse_nb;
-    }
-    // keep the coarse arrays (4 per level, each with one more element: the
-    // zero slot of the phi arrays) and the tables in LDS when they fit
-    long long nd = 0;
-    for (int l = lc; l <= ps->L; l++) {
-        P.lev[l - lc].off = (int)nd;
-        nd += 4 * (ps->npts[l] + 1);
-    }
-    if (nd * 8 + 4LL * P.nb_words <= 128 * 1024) {
-        P.lds = 1;
-        P.lds_doubles = (int)nd;
-        ps->coarse_lds = (int)(nd * 8 + 4LL * P.nb_words);
-        if (ps->coarse_lds > 64 * 1024) {
-            hipError_t e = coarse_set_lds_limit(ps->coarse_lds);
-            if (e != hipSuccess) {
-                P.lds = 0;
-                ps->coarse_lds = 0;
-            }
-        }
-    }
-    ps->h_coarse = P;
-    hipError_t e = hipMalloc((void**)&ps->d_coarse, sizeof(CoarsePlan));
-    if (e == hipSuccess) e = hipMemcpy(ps->d_coarse, &P, sizeof P, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return gpaw_check(e, "poisson: coarse plan");
+    const int k = P.lev[0].pre + P.lev[0].post;   // where single sweeps leave phi
+    P.rho = ps->rho[lc];
+    P.out = k % 2 ? ps->phiB[lc] : ps->phiA[lc];
+    ps->coarse = P;
     ps->lc = lc;
-    return GPAW_OK;
 }
 
 // With the launch-shape tuner on, one V-cycle is first run eagerly on the
@@ -777,8 +743,6 @@ extern "C" void gpaw_poisson_free(gpaw_poisson* ps)
     if (ps->d_sum) hipFree(ps->d_sum);
     if (ps->charge_ev) hipEventDestroy(ps->charge_ev);
     if (ps->h_errs) hipHostFree(ps->h_errs);
-    if (ps->d_coarse) hipFree(ps->d_coarse);
-    if (ps->d_coarse_nb) hipFree(ps->d_coarse_nb);
     if (ps->mixed) gpaw_mixed_free(ps->mixed);
     if (ps->h_err) hipHostFree(ps->h_err);
     delete ps;

@@ -64,9 +64,7 @@ struct gpaw_poisson {
     double hint_eps = 0.0;
     int swaps = 0;             // 1 if level 0 does an odd number of sweeps per cycle
     int lc = -1;               // first level run by the fused coarse kernel (-1: none)
-    gpaw::CoarsePlan* d_coarse = nullptr;
-    short* d_coarse_nb = nullptr;     // neighbour tables of the fused coarse levels
-    int coarse_lds = 0;        // dynamic LDS bytes of the fused kernel
+    gpaw::CoarsePlan coarse;   // its plan
     bool fuse_jacobi = true;   // fused Jacobi sweeps on levels > 0 (GPAW_AMD_FUSED_JACOBI=0: off)
     // coarse-grid correction applied by the first fused post-smoothing launch
     // (GPAW_AMD_FOLD_CORRECTION=0: a separate interpolate-and-subtract launch)
@@ -79,7 +77,6 @@ struct gpaw_poisson {
     bool fuse_norm = true;
     double* norm_in = nullptr;   // partials row for the next emitted cycle's first sweep
     bool skip_norm = false;      // the next emitted cycle takes no norm pass
-    gpaw::CoarsePlan h_coarse; // host copy of the coarse plan
     MixedState* mixed = nullptr;
 };
 
