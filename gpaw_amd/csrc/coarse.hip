@@ -21,8 +21,8 @@
 // points' right-hand sides and neighbour indices in registers for all passes of
 // a level, and only the phi pair of every level lives in LDS (the residual
 // takes the array the last sweep read).  The block has no more waves than the
-// first level needs.  11^3 + 5^3 (16 sweeps): 17.6 us before, 13.0 now;
-// 6 x 6 x 8 + 3 x 3 x 4: 13.0 and 7.6; 9^3 alone (8 sweeps): 6.6 and 5.0.
+// first level needs.  11^3 + 5^3 (16 sweeps): 17.6 us before, 12.7 now;
+// 6 x 6 x 8 + 3 x 3 x 4: 13.0 and 7.8; 9^3 alone (8 sweeps): 6.6 and 5.0.
 #include "kernels.h"
 #include "coarse.h"
 #include "transfer_common.h"

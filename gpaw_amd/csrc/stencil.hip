@@ -500,6 +500,11 @@ hipError_t launch_jacobi_two_from_zero(const Stencil& s, int dtype, const void* 
     if (!jacobi_two_from_zero_ok(s, dtype, g)) return hipErrorInvalidValue;
     TileShape sh;
     box_geometry(g, s.star_r, 1, box_default_q(g, s.star_r, 1), sh);
+    // 8 planes where launch_stencil takes them too (159^3: 18.6 -> 15.5 us)
+    TileShape b8;
+    if (dtype == DT_F32 && (long)g.n[0] * g.n[1] * g.n[2] >= (1L << 19) &&
+        box_geometry(g, s.star_r, 1, 8, b8))
+        sh = b8;
     return dtype == DT_F64 ? box_fz_f64(s, rho, out, g, w0, w1, sh, st)
                            : box_fz_f32(s, rho, out, g, w0, w1, sh, st);
 }
