@@ -22,7 +22,8 @@
 // gpaw/fd_operators.py:123-144).  One thread per in-plane point and Q planes,
 // every load issued at once, no LDS: the neighbours along axes 0 and 1 come
 // from the thread's own column of Q + 2 R points, along axis 2 through the L1.
-// HBM bound: 2 x 127^3 float64, R = 3, 43 -> 12.5 us (16.5 us along axis 2).
+// HBM bound: 2 x 127^3 float64, R = 3, 43 -> 12.5 us (16.5 us along axis 2, where
+// k_axis2 takes over for rows that fit a block).
 #pragma once
 #include "kernels.h"
 
@@ -265,6 +266,62 @@ __global__ __launch_bounds__(256) void k_axis(const V* __restrict__ in, V* __res
             x = vmac(x, y, (RT)sc.c[m]);
         }
         o[(s0 + u) * st] = x;
+    }
+}
+
+// The same along axis 2 for rows of up to AXIS2_PTS points: a block takes whole
+// rows, up to AXIS2_PTS points in all, which are contiguous in memory; they go
+// to LDS once, with R ghosts on either side of each row, and a point reads its
+// 2 R neighbours there instead of through the L1 (2 x 127^3 float64, R = 3:
+// 16.5 -> 12.5 us).
+constexpr int AXIS2_PTS = 1024;
+
+template <class V, int R>
+__global__ __launch_bounds__(256) void k_axis2(const V* __restrict__ in, V* __restrict__ out,
+                                               Geom g, Phases ph, AxisCoefs sc, int nr, int rows,
+                                               unsigned magic)
+{
+    typedef typename VT<V>::R RT;
+    constexpr int PT = AXIS2_PTS / 256;
+    extern __shared__ __align__(16) char axis2_lds[];
+    V* __restrict__ L = (V*)axis2_lds;
+    const int n = g.n[2], LW = n + 2 * R;
+    const int row0 = blockIdx.x * nr, mine = min(nr, rows - row0), pts = mine * n;
+    const V* __restrict__ a = in + (i64)row0 * n;
+    V* __restrict__ o = out + (i64)row0 * n;
+    V v[PT];
+    int at[PT];
+#pragma unroll
+    for (int k = 0; k < PT; k++) {
+        const int el = threadIdx.x + 256 * k;
+        v[k] = a[el < pts ? el : 0];
+        const int r = __umulhi((unsigned)el, magic);   // el / n
+        at[k] = el < pts ? r * LW + R + el - r * n : -1;
+    }
+    // ghosts: cell c of a row is at -R + c, or for c >= R at n + c - R
+    for (int h = threadIdx.x; h < mine * 2 * R; h += 256) {
+        const int r = h / (2 * R), c = h % (2 * R), pos = c < R ? c - R : n + c - R;
+        int p = pos;
+        const int f = wrap_index(p, n, g.per[2]);
+        V x = vzero<V>();
+        if (f != 3) {
+            x = a[r * n + p];
+            if (VT<V>::cplx && f) x = pside<true>(x, ph, 2, f);
+        }
+        L[r * LW + R + pos] = x;
+    }
+#pragma unroll
+    for (int k = 0; k < PT; k++)
+        if (at[k] >= 0) L[at[k]] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PT; k++) {
+        if (at[k] < 0) continue;
+        const V* __restrict__ c = L + at[k];
+        V x = vzero<V>();
+#pragma unroll
+        for (int m = 0; m < 2 * R; m++) x = vmac(x, c[m < R ? m - R : m - R + 1], (RT)sc.c[m]);
+        o[threadIdx.x + 256 * k] = x;
     }
 }
 

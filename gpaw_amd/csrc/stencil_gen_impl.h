@@ -102,6 +102,19 @@ hipError_t axis_go(const Stencil& s, const void* in, void* out, const Geom& g, c
 }
 
 template <class V, int R>
+hipError_t axis2_go(const Stencil& s, const void* in, void* out, const Geom& g, const Phases& ph,
+                    int nin, hipStream_t st)
+{
+    AxisCoefs sc;
+    for (int c = 0; c < 2 * R; c++) sc.c[c] = s.coefs[c];
+    const int n = g.n[2], rows = g.n[0] * g.n[1] * nin, nr = AXIS2_PTS / n;
+    const size_t lds = (size_t)nr * (n + 2 * R) * sizeof(V);
+    const unsigned magic = (unsigned)(((1ULL << 32) + n - 1) / n);   // exact below 2^32 / n
+    return launch_kernel((k_axis2<V, R>), dim3((unsigned)((rows + nr - 1) / nr)), dim3(256), lds,
+                         st, (const V*)in, (V*)out, g, ph, sc, nr, rows, magic);
+}
+
+template <class V, int R>
 hipError_t axis_launch(const Stencil& s, const void* in, void* out, const Geom& g,
                        const Phases& ph, int nin, hipStream_t st)
 {
@@ -110,7 +123,12 @@ hipError_t axis_launch(const Stencil& s, const void* in, void* out, const Geom& 
     switch (s.axis) {
     case 0: return axis_go<V, R, 0, 4>(s, in, out, g, ph, nin, st);
     case 1: return axis_go<V, R, 1, 4>(s, in, out, g, ph, nin, st);
-    case 2: return axis_go<V, R, 2, 4>(s, in, out, g, ph, nin, st);
+    case 2:
+        // whole rows of 16 .. 1024 points in LDS: shorter ones would be mostly
+        // ghosts, longer ones do not fit (127: 12.5 against 16.5 us)
+        if (g.n[2] >= 16 && g.n[2] <= AXIS2_PTS && (long)g.n[0] * g.n[1] * nin < 0x7fffffffL)
+            return axis2_go<V, R>(s, in, out, g, ph, nin, st);
+        return axis_go<V, R, 2, 4>(s, in, out, g, ph, nin, st);
     }
     return hipErrorInvalidValue;
 }

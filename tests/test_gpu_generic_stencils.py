@@ -122,3 +122,38 @@ def test_non_finite_values_stay_local():
         ops.stencil_kernel(prev)
     assert torch.equal(torch.isfinite(got), torch.isfinite(want))
     assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(want))
+
+
+@pytest.mark.parametrize('dtype', ['float64', 'complex128', 'float32', 'complex64'])
+@pytest.mark.parametrize('n, pbc, nn', [
+    ((5, 6, 15), True, 3), ((5, 6, 16), True, 3),        # shortest rows of the LDS kernel
+    ((6, 5, 17), False, 4), ((40, 13, 16), False, 1),    # 64 rows a block, partial last block
+    ((4, 5, 255), False, 2), ((4, 5, 342), True, 3),     # 4 and 2 rows a block
+    ((5, 5, 513), True, 4),                              # one row a block
+    ((4, 3, 1024), True, 3), ((4, 3, 1025), True, 3),    # a full block; too long for one
+])
+def test_gradient_along_rows(n, pbc, nn, dtype):
+    """Axis 2: whole rows in LDS, where they fit, against the generic kernel."""
+    import torch
+
+    from gpaw_amd import ops
+    from gpaw_amd.fd_operators import Gradient
+    from gpaw_amd.grid_descriptor import GridDescriptor
+    print('case gradient rows', n, pbc, nn, dtype, flush=True)
+    m = n if pbc else tuple(x + 1 for x in n)
+    gd = GridDescriptor(m, CELLS['ortho'](m), pbc)
+    cplx = dtype.startswith('complex')
+    ph = gd.phase_cd((0.15, -0.3, 0.4)) if cplx and pbc else None
+    op = Gradient(gd, 2, n=nn, dtype=complex if cplx else float)
+    g = torch.Generator(device='cuda').manual_seed(7)
+    for nb in (1, 3):
+        a = torch.randn((nb,) + tuple(gd.n_c), dtype=getattr(torch, dtype), device='cuda',
+                        generator=g)
+        got, want = torch.full_like(a, 3.0), torch.full_like(a, 5.0)
+        op.apply(a, got, ph)
+        prev = ops.stencil_kernel('generic')
+        try:
+            op.apply(a, want, ph)
+        finally:
+            ops.stencil_kernel(prev)
+        assert torch.equal(got, want)
