@@ -601,7 +601,9 @@ int setup(gpaw_poisson* ps, int pr)
         if (!rc)
             rc = gpaw_check(hipMalloc((void**)&m->partial, sizeof(double) * 4 * NB),
                             "mixed: partials");
+        // on the null stream, which the caller's stream need not wait for
         if (!rc) rc = gpaw_check(hipMemset(m->S, 0, sizeof(double) * S_N), "mixed: scalars");
+        if (!rc) rc = gpaw_check(hipStreamSynchronize(nullptr), "mixed: scalars");
         if (rc) return rc;
     }
     MixedState* m = ps->mixed;

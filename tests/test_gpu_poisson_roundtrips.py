@@ -111,3 +111,26 @@ def test_mean_is_removed_as_integrate_and_subtract(torch, mixed):
         mean /= np.prod(solver.gd.get_size_of_global_array())
         ops.sub_scalar(raw, raw, mean)
         assert torch.equal(phi, raw)
+
+
+@pytest.mark.parametrize('mixed', [False, True])
+def test_first_solve_beside_a_busy_null_stream(torch, mixed):
+    """A solver's first solve sets its state up; on a stream that does not wait
+    for the null stream nothing of that may be left queued there."""
+    want = None
+    side = torch.cuda.Stream()
+    a = torch.ones((4096, 4096), dtype=torch.float64, device='cuda')
+    for busy in (False, True):
+        solver = make((True,) * 3, mixed)
+        rho = density(torch, solver, 8, 0)
+        torch.cuda.synchronize()
+        if busy:
+            for _ in range(20):
+                b = a @ a           # tens of milliseconds on the null stream
+        with torch.cuda.stream(side):
+            got = run(torch, solver, rho)
+        torch.cuda.synchronize()
+        assert got[0] > 0
+        if want is not None:
+            assert got[0] == want[0] and np.array_equal(got[1], want[1])
+        want = got
