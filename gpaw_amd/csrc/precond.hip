@@ -46,13 +46,14 @@ namespace {
 // 40.7 us, with 8 planes in all three 50.4, 4 / 8 / 8 44.7, 2 / 2 / 8 42.5;
 // complex128 24 x 64^3 145, 149, 147, 150; 16 x 32^3 54, 56, 54, 56; 6 or 4
 // planes without b: 59 or 54.5, real 8 x 64^3 48.6 or 47.3 instead of 45.
-bool pc_shape(const Geom& g, int R, int esize, int nin, int nt, int run, TileShape* sh)
+bool pc_shape(const Geom& g, int R, int esize, int nin, int nt, int run, TileShape* sh,
+              int TZ = 32)
 {
-    if (!tile_geometry(g, R, esize, nin, 32, g.n[0], *sh, nt)) return false;
+    if (!tile_geometry(g, R, esize, nin, TZ, g.n[0], *sh, nt)) return false;
     long nch = (1024L + sh->nblocks - 1) / sh->nblocks;
     const long maxch = g.n[0] / run > 1 ? g.n[0] / run : 1;
     if (nch > maxch) nch = maxch;
-    return tile_geometry(g, R, esize, nin, 32, (int)((g.n[0] + nch - 1) / nch), *sh, nt);
+    return tile_geometry(g, R, esize, nin, TZ, (int)((g.n[0] + nch - 1) / nch), *sh, nt);
 }
 
 TileCoefs pc_coefs(const Stencil& s)
@@ -69,22 +70,36 @@ i64 pc_points(const int n[3]) { return (i64)n[0] * n[1] * n[2]; }
 // complex data from 2^15 points in all (below, one tile's serial planes take
 // longer than the two short launches: 8 bands of 13 x 11 x 17, a call of 50
 // instead of 46 us).
+template <class V, int TZ>
+hipError_t pc_scaled_go(const gpaw_operator* L, int mode, const void* b, void* out,
+                        const Phases& ph, double cb, double w, const TileShape& sh, hipStream_t st)
+{
+    const dim3 grid(sh.nblocks), block(TZ, TILE_NT / TZ);
+    const TileCoefs sc = pc_coefs(L->st);
+    const i64 ng = pc_points(L->g.n);
+    if (mode == ST_RESID)
+        return launch_kernel((k_pc_scaled<V, 1, ST_RESID, TILE_NT, TZ>), grid, block, 0, st,
+                             (const V*)b, (V*)out, L->g, ph, sc, cb, w, sh, ng);
+    return launch_kernel((k_pc_scaled<V, 1, ST_PCUPD, TILE_NT, TZ>), grid, block, 0, st,
+                         (const V*)b, (V*)out, L->g, ph, sc, cb, w, sh, ng);
+}
+
 template <class V>
 hipError_t pc_scaled(const gpaw_operator* L, int mode, const void* b, void* out, int nin,
                      const Phases& ph, double cb, double w, hipStream_t st)
 {
     TileShape sh;
     if (VT<V>::cplx && nin * pc_points(L->g.n) < 1 << 15) return hipErrorNotSupported;
-    if (L->st.star_r != 1 || !pc_shape(L->g, 1, (int)sizeof(V), nin, TILE_NT, 2, &sh))
-        return hipErrorNotSupported;
-    const dim3 grid(sh.nblocks), block(32, TILE_NT / 32);
-    const TileCoefs sc = pc_coefs(L->st);
-    const i64 ng = pc_points(L->g.n);
-    if (mode == ST_RESID)
-        return launch_kernel((k_pc_scaled<V, 1, ST_RESID, TILE_NT>), grid, block, 0, st,
-                             (const V*)b, (V*)out, L->g, ph, sc, cb, w, sh, ng);
-    return launch_kernel((k_pc_scaled<V, 1, ST_PCUPD, TILE_NT>), grid, block, 0, st, (const V*)b,
-                         (V*)out, L->g, ph, sc, cb, w, sh, ng);
+    if (L->st.star_r != 1) return hipErrorNotSupported;
+    // rows of up to 16 points (level 2 of a 64^3 grid) in tiles of 16 x 16: a tile
+    // of 32 would wrap twice, and the two separate launches took 21 us on 256
+    // complex128 bands of 16^3, now 10 (a call 934 -> 923; 2 real bands of 48 x 64 x
+    // 40 32.5 -> 29.5)
+    if (L->g.n[2] <= 16 && pc_shape(L->g, 1, (int)sizeof(V), nin, TILE_NT, 2, &sh, 16))
+        return pc_scaled_go<V, 16>(L, mode, b, out, ph, cb, w, sh, st);
+    if (pc_shape(L->g, 1, (int)sizeof(V), nin, TILE_NT, 2, &sh))
+        return pc_scaled_go<V, 32>(L, mode, b, out, ph, cb, w, sh, st);
+    return hipErrorNotSupported;
 }
 
 // out = mode(L F, aux) with F = I e (b null) or c b - I e; hipErrorNotSupported

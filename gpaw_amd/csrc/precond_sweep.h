@@ -20,13 +20,13 @@ namespace gpaw {
 // F = c b: the register queue and LDS plane of k_star_tile, each loaded value
 // scaled before its ghost phase.  HBM bound: 256 complex128 bands of 32^3 in
 // 51 us (5.2 TB/s), where the scaling and the stencil launch took 61 + 86.
-template <class V, int R, int MODE, int NT>
+template <class V, int R, int MODE, int NT, int TZ>
 __global__ __launch_bounds__(NT) void k_pc_scaled(const V* __restrict__ in, V* __restrict__ out,
                                                   Geom g, Phases ph, TileCoefs sc, double cb,
                                                   double w, TileShape sh, i64 ng)
 {
     typedef typename VT<V>::R RT;
-    constexpr int TZ = 32, TY = NT / TZ;
+    constexpr int TY = NT / TZ;
     constexpr int LW = TZ + 2 * R, LH = TY + 2 * R, NHALO = 2 * R * (TZ + TY);
     static_assert(NHALO <= NT, "one halo cell per thread");
     __shared__ V lds[2 * LH * LW];

@@ -520,7 +520,7 @@ int tile_tz(int)
 bool tile_geometry(const Geom& g, int R, int esize, int nin, int TZ, int q, TileShape& sh,
                    int nt)
 {
-    if (R < 1 || R > 4 || (TZ != 32 && TZ != 64) || q < 1 || nin < 1) return false;
+    if (R < 1 || R > 4 || (TZ != 16 && TZ != 32 && TZ != 64) || q < 1 || nin < 1) return false;
     if (nt != TILE_NT && nt != TILE_NT_WIDE && nt != TILE_NT_MID) return false;
     const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2];
     const int TY = (nt / TZ) * tile_rows(R, esize, nt);

@@ -107,6 +107,10 @@ FUSED = [
     ((36, 28, 44), True, float, 3, 3),
     ((28, 28, 36), (False, True, True), float, 2, 2),
     ((20, 24, 20), False, float, 1, 1),
+    # rows of up to 16 points on level 2: 16 x 16 tiles
+    ((48, 56, 64), True, complex, 14, 3),
+    ((60, 44, 36), (True, False, True), complex, 40, 2),
+    ((64, 40, 60), False, float, 3, 3),
 ]
 
 
