@@ -55,15 +55,21 @@ def interpolate_density(interpolator, finegd, nt_sG, nt_sg, charge=0.0,
     interpolator: a Transformer(gd, finegd, nn) of gpaw_amd.transformers."""
     out = Arg(nt_sg, write=True, name='nt_sg')
     src = Arg(nt_sG, name='nt_sG')
-    interpolator.apply(src.tensor, out.tensor)
-    if not finegd.pbc_c.all():
-        pseudo_charge = -(charge + comp_charge)
-        if abs(pseudo_charge) > 1.0e-14:
-            if np.prod(out.shape[:-3]) <= _lib.GPAW_RENORMALIZE_MAX:
-                ops.renormalize(finegd, out.tensor, pseudo_charge)
-            else:   # numpy adds 8 and more integrals in another order
-                x = pseudo_charge / np.sum(finegd.integrate(out.tensor))
-                ops.scale(out.tensor, x)
+    pseudo_charge = -(charge + comp_charge)
+    scale = not finegd.pbc_c.all() and abs(pseudo_charge) > 1.0e-14
+    few = np.prod(out.shape[:-3]) <= _lib.GPAW_RENORMALIZE_MAX
+    handle = getattr(interpolator, 'transformer', None)
+    if scale and few and isinstance(handle, ops.TransformerHandle) and \
+            src.code == out.code == _lib.GPAW_F64:
+        # one call: the interpolation sums what it stores
+        handle.apply_renormalize(finegd, src.tensor, out.tensor, pseudo_charge)
+    else:
+        interpolator.apply(src.tensor, out.tensor)
+        if scale and few:
+            ops.renormalize(finegd, out.tensor, pseudo_charge)
+        elif scale:   # numpy adds 8 and more integrals in another order
+            x = pseudo_charge / np.sum(finegd.integrate(out.tensor))
+            ops.scale(out.tensor, x)
     out.finish()
 
 

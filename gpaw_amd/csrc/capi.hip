@@ -561,6 +561,30 @@ extern "C" int gpaw_renormalize(double* y, long nin, long n, double scale, doubl
                       "renormalize");
 }
 
+extern "C" int gpaw_transformer_apply_renormalize(gpaw_transformer* tr, const double* in,
+                                                  double* out, long nin, double scale,
+                                                  double target, double* work, void* stream)
+{
+    if (!tr) return gpaw_fail(GPAW_EINVAL, "transformer: NULL handle");
+    int rc = gpaw_check_dtype(tr->real, DT_F64);
+    if (rc) return rc;
+    if (nin < 0 || nin > GPAW_RENORMALIZE_MAX)
+        return gpaw_fail(GPAW_EINVAL, "transformer: nin = %ld (at most %d functions)", nin,
+                         GPAW_RENORMALIZE_MAX);
+    if (nin == 0) return GPAW_OK;
+    if (!in || !out || !work) return gpaw_fail(GPAW_EINVAL, "transformer: NULL array");
+    Phases ph;
+    gpaw_phases(nullptr, ph);
+    const long long n = (long long)tr->t.nout[0] * tr->t.nout[1] * tr->t.nout[2];
+    hipStream_t st = (hipStream_t)stream;
+    int np = 0;
+    hipError_t e = launch_interp_sums(tr->t, in, out, ph, (int)nin, work, &np, st);
+    if (e == hipSuccess)
+        e = np ? launch_renormalize_partials(out, (int)nin, n, scale, target, work, np, st)
+               : launch_renormalize(out, (int)nin, n, scale, target, work, st);
+    return gpaw_check(e, "transformer apply, renormalize");
+}
+
 extern "C" int gpaw_sub_scalar(double* y, const double* x, double b, long n, void* stream)
 {
     if (!y || !x || n < 0) return gpaw_fail(GPAW_EINVAL, "sub_scalar: bad argument");

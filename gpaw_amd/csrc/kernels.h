@@ -209,6 +209,15 @@ hipError_t launch_sum(const double* a, long long n, double* partial, int* nparti
 // partial holds nin * SUM_PARTIALS doubles
 hipError_t launch_renormalize(double* y, int nin, long long n, double scale, double target,
                               double* partial, hipStream_t st);
+// the same from partial sums at hand, rows of np
+hipError_t launch_renormalize_partials(double* y, int nin, long long n, double scale,
+                                       double target, const double* partial, int np,
+                                       hipStream_t st);
+// An FP64 transfer (TR_STORE) that also leaves *nsums partial sums of each
+// output function in a row of `sums` (nin * SUM_PARTIALS doubles) where its
+// kernel can; else *nsums = 0.
+hipError_t launch_interp_sums(const Transfer& t, const void* in, void* out, const Phases& ph,
+                              int nin, double* sums, int* nsums, hipStream_t st);
 // result[j] = scale * sum_g a[g] * b[j n + g] for j < nb (nb <= 65535);
 // partial holds nb * dots_chunks(n) doubles.
 int dots_chunks(long long n);

@@ -227,6 +227,13 @@ hipError_t launch_renormalize(double* y, int nin, long long n, double scale, dou
     if (n <= 0 || nin <= 0) return hipSuccess;
     const int np = sum_blocks(n);
     launch_kernel(k_sum, dim3(np, nin), dim3(256), 0, st, (const double*)y, (i64)n, partial);
+    return launch_renormalize_partials(y, nin, n, scale, target, partial, np, st);
+}
+
+hipError_t launch_renormalize_partials(double* y, int nin, long long n, double scale,
+                                       double target, const double* partial, int np,
+                                       hipStream_t st)
+{
     const i64 total = (i64)nin * n;
     i64 nb = (total + 1023) / 1024;   // 4 points a thread; at most 8 blocks per CU
     if (nb > 2048) nb = 2048;

@@ -93,7 +93,8 @@ inline TileTr tile_tr(const TrArgs& t, bool interpolate, int nin)
 
 template <class V, int K>
 hipError_t tr_launch(const Transfer& tr, int mode, const void* in, void* out, void* zero_out,
-                     const Phases& ph, int nin, hipStream_t st)
+                     const Phases& ph, int nin, hipStream_t st, double* sums = nullptr,
+                     int* nsums = nullptr)
 {
     const TrArgs t = make_trargs(tr);
     dim3 grid((unsigned)((t.ngout + 255) / 256), nin, 1);
@@ -132,10 +133,15 @@ hipError_t tr_launch(const Transfer& tr, int mode, const void* in, void* out, vo
                                (V*)out, t, tt, ph);
         else if (mode == TR_SUBTRACT)
             launch_kernel((k_interp_tile<V, K, 8, 32, TR_SUBTRACT>), gt, dim3(256), 0, st,
-                               (const V*)in, (V*)out, t, tt, ph);
-        else
+                               (const V*)in, (V*)out, t, tt, ph, (double*)nullptr);
+        else {
+            // partial sums of each function's outputs, where a row holds them
+            const int np = tt.nt1 * tt.nt2 * tt.nch;
+            double* s = sums && np <= SUM_PARTIALS ? sums : nullptr;
+            if (s) *nsums = np;
             launch_kernel((k_interp_tile<V, K, 8, 32, TR_STORE>), gt, dim3(256), 0, st,
-                               (const V*)in, (V*)out, t, tt, ph);
+                               (const V*)in, (V*)out, t, tt, ph, s);
+        }
         if (!tr.interpolate && zero_out) return launch_fill(zero_out, VT<V>::cplx ? (sizeof(typename VT<V>::R) == 8 ? DT_C128 : DT_C64) : (sizeof(typename VT<V>::R) == 8 ? DT_F64 : DT_F32), t.ngout * nin, st);
         return launch_error();
     }
@@ -154,13 +160,14 @@ hipError_t tr_launch(const Transfer& tr, int mode, const void* in, void* out, vo
 
 template <class V>
 hipError_t tr_dispatch(const Transfer& tr, int mode, const void* in, void* out, void* zero_out,
-                       const Phases& ph, int nin, hipStream_t st)
+                       const Phases& ph, int nin, hipStream_t st, double* sums = nullptr,
+                       int* nsums = nullptr)
 {
     switch (tr.K) {
-    case 2: return tr_launch<V, 2>(tr, mode, in, out, zero_out, ph, nin, st);
-    case 4: return tr_launch<V, 4>(tr, mode, in, out, zero_out, ph, nin, st);
-    case 6: return tr_launch<V, 6>(tr, mode, in, out, zero_out, ph, nin, st);
-    case 8: return tr_launch<V, 8>(tr, mode, in, out, zero_out, ph, nin, st);
+    case 2: return tr_launch<V, 2>(tr, mode, in, out, zero_out, ph, nin, st, sums, nsums);
+    case 4: return tr_launch<V, 4>(tr, mode, in, out, zero_out, ph, nin, st, sums, nsums);
+    case 6: return tr_launch<V, 6>(tr, mode, in, out, zero_out, ph, nin, st, sums, nsums);
+    case 8: return tr_launch<V, 8>(tr, mode, in, out, zero_out, ph, nin, st, sums, nsums);
     }
     return hipErrorInvalidValue;
 }

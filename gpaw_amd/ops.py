@@ -162,7 +162,7 @@ class TransformerHandle:
                 pass
             self.h = None
 
-    def apply(self, input, output, phases=None):
+    def _args(self, input, output):
         a = Arg(input, name='input')
         b = Arg(output, write=True, name='output')
         if a.shape[-3:] != self.ngpin or b.shape[-3:] != self.ngpout or \
@@ -171,6 +171,22 @@ class TransformerHandle:
                              % (a.shape, b.shape, self.ngpin, self.ngpout))
         if a.code != b.code:
             raise TypeError('transformer apply: input and output dtypes differ')
+        return a, b
+
+    def apply_renormalize(self, gd, input, output, target):
+        """apply, then renormalize(gd, output, target): float64 device tensors
+        of at most 7 functions; gd is the output's grid."""
+        a, b = self._args(input, output)
+        nin = _nin(a.shape, self.ngpin)
+        work = _arrays.torch().empty(max(1, nin) * _lib.GPAW_RENORMALIZE_WORK,
+                                     dtype=b.tensor.dtype, device=b.tensor.device)
+        _lib.check(_lib.lib().gpaw_transformer_apply_renormalize(
+            self.h, a.ptr, b.ptr, nin, float(gd.dv), float(target), work.data_ptr(),
+            _arrays.stream()))
+        b.finish()
+
+    def apply(self, input, output, phases=None):
+        a, b = self._args(input, output)
         _, pp = _phases(phases)
         _lib.check(_lib.lib().gpaw_transformer_apply(
             self.h, a.ptr, b.ptr, _nin(a.shape, self.ngpin), a.code, pp,

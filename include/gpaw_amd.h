@@ -356,6 +356,14 @@ int gpaw_axpby_shared(double* y, const double* x, double a, double b, long nin,
 int gpaw_renormalize(double* y, long nin, long n, double scale, double target,
                      double* work, void* stream);
 
+/* gpaw_transformer_apply of nin float64 functions (at most
+ * GPAW_RENORMALIZE_MAX), then gpaw_renormalize of the results.  An
+ * interpolation sums its outputs as it stores them, in an order of its own, so
+ * the scaled values may differ from the two calls' in the last bits. */
+int gpaw_transformer_apply_renormalize(gpaw_transformer* tr, const double* in, double* out,
+                                       long nin, double scale, double target, double* work,
+                                       void* stream);
+
 /* y = x - b over n doubles (rho - background, phi -= phi_ave:
  * gpaw/poisson.py:138,216). */
 int gpaw_sub_scalar(double* y, const double* x, double b, long n,

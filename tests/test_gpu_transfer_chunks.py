@@ -79,3 +79,41 @@ def test_axpby_shared_equals_axpby(nin, n):
     assert torch.equal(y, want)
     empty = y[:0]
     ops.axpby_shared(empty, x, 1.0, 1.0, 0)
+
+
+@pytest.mark.parametrize('n,pbc,nn,nin', [
+    ((16, 16, 16), False, 3, 1),         # 31^3: partial tiles
+    ((16, 20, 24), (True, True, False), 2, 3),
+    ((10, 16, 34), (False, True, True), 4, 7),
+    ((30, 24, 16), False, 1, 2),         # K = 2: its kernel leaves no sums
+    ((8, 150, 530), False, 2, 1),        # 38 x 34 tiles: more than a row of sums
+    ((64, 12, 12), False, 3, 2),         # many chunks of few tiles
+])
+def test_interpolation_sums_its_outputs(n, pbc, nn, nin):
+    """apply_renormalize against apply and renormalize.  The sums of positive
+    values differ by the rounding of two orders of addition, at most about 300
+    terms deep each: 600 * 1.1e-16 relative, bound 1e-13."""
+    torch = pytest.importorskip('torch')
+    if not torch.cuda.is_available():
+        pytest.skip('no GPU')
+    print('case interpolation sums', n, pbc, nn, nin, flush=True)
+    from gpaw_amd import ops
+    from gpaw_amd.grid_descriptor import GridDescriptor
+    from gpaw_amd.transformers import Transformer
+    gd = GridDescriptor(n, np.array(n) * 0.4, pbc)
+    fine = gd.refine()
+    tr = Transformer(gd, fine, nn)
+    g = torch.Generator(device='cuda').manual_seed(3)
+    a = torch.rand((nin,) + tuple(int(x) for x in gd.n_c), dtype=torch.float64, device='cuda',
+                   generator=g) + 0.5
+    want = torch.empty((nin,) + tuple(int(x) for x in fine.n_c), dtype=torch.float64,
+                       device='cuda')
+    got = torch.full_like(want, 7.0)
+    tr.apply(a, want)
+    ops.renormalize(fine, want, -3.5)
+    tr.transformer.apply_renormalize(fine, a, got, -3.5)
+    assert bool(((got - want).abs() <= 1e-13 * want.abs()).all())
+    total = float(np.sum(fine.integrate(got)))
+    assert abs(total + 3.5) <= 3.5e-13
+    with pytest.raises(Exception):
+        tr.transformer.apply_renormalize(fine, a[..., 1:].contiguous(), got, -3.5)
