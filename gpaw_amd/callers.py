@@ -82,7 +82,11 @@ def restrict_potential(restrictor, vt_sg, vHt_g, vt_sG):
     vH = Arg(vHt_g, name='vHt_g')
     out = Arg(vt_sG, write=True, name='vt_sG')
     t = fine.tensor
-    ops.axpby_shared(t, vH.tensor, 1.0, 1.0, 1 if t.dim() == 3 else t.shape[0])
+    spins = t[None] if t.dim() == 3 else t
+    if spins.shape[0]:
+        # the same fine grid for every spin: nothing is broadcast or cut short
+        vH = Arg(vH.tensor, name='vHt_g', shape=tuple(spins.shape[1:]), code=_lib.GPAW_F64)
+        ops.axpby_shared(spins, vH.tensor, 1.0, 1.0, spins.shape[0])
     restrictor.apply(t, out.tensor)
     fine.finish()
     out.finish()

@@ -259,13 +259,14 @@ def axpby(y, x, a, b):
 
 
 def axpby_shared(y, x, a, b, nin):
-    """y_k = a*y_k + b*x for the nin equal parts y_k of y (float64 device
-    tensors) in one launch."""
+    """y_k = a*y_k + b*x for the nin functions y_k of y (float64 device
+    tensors) in one launch; x has the shape of one of them."""
     yy = Arg(y, write=True, name='y', code=_lib.GPAW_F64)
     xx = Arg(x, name='x', code=_lib.GPAW_F64)
-    n = yy.tensor.numel() // max(nin, 1)
-    if nin and xx.tensor.numel() < n:
-        raise ValueError('axpby_shared: x of shape %s for y of shape %s' % (xx.shape, yy.shape))
+    if yy.shape != (nin,) + xx.shape and not (nin == 1 and yy.shape == xx.shape):
+        raise ValueError('axpby_shared: x of shape %s for %d functions in y of shape %s'
+                         % (xx.shape, nin, yy.shape))
+    n = int(np.prod(xx.shape))
     _lib.check(_lib.lib().gpaw_axpby_shared(yy.ptr, xx.ptr, float(a), float(b), nin, n,
                                             _arrays.stream()))
     yy.finish()

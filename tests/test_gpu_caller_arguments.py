@@ -1,0 +1,73 @@
+"""What the callers refuse, and that they go through the objects they are
+given."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+N = (8, 10, 12)
+
+
+@pytest.fixture(scope='module')
+def torch():
+    t = pytest.importorskip('torch')
+    if not t.cuda.is_available():
+        pytest.skip('no GPU')
+    return t
+
+
+def grids(pbc):
+    from gpaw_amd.grid_descriptor import GridDescriptor
+    gd = GridDescriptor(N, np.array(N) * 0.4, pbc)
+    return gd, gd.refine()
+
+
+def rand(torch, shape, seed=1):
+    g = torch.Generator(device='cuda').manual_seed(seed)
+    return torch.rand(tuple(int(x) for x in shape), dtype=torch.float64, device='cuda',
+                      generator=g) + 0.5
+
+
+# shapes of vHt_g for a fine grid n and two spins that are not n
+WRONG = {'transposed': lambda n: n[::-1],
+         'larger': lambda n: (n[0] + 1,) + n[1:],
+         'spins': lambda n: (2,) + n,
+         'one spin': lambda n: (1,) + n,
+         'flat': lambda n: (int(np.prod(n)),),
+         'smaller': lambda n: n[:2] + (n[2] - 1,)}
+
+
+@pytest.mark.parametrize('spins', [(), (1,), (2,)])
+@pytest.mark.parametrize('wrong', sorted(WRONG))
+def test_restrict_potential_wants_the_fine_grid(torch, spins, wrong):
+    from gpaw_amd.callers import restrict_potential
+    from gpaw_amd.transformers import Transformer
+    print('case restrict_potential', spins, wrong, flush=True)
+    gd, fine = grids(False)
+    n = tuple(int(x) for x in fine.n_c)
+    vt = rand(torch, spins + n)
+    kept = vt.clone()
+    out = rand(torch, spins + tuple(gd.n_c))
+    vH = rand(torch, WRONG[wrong](n), 2)
+    with pytest.raises(ValueError):
+        restrict_potential(Transformer(fine, gd, 3), vt, vH, out)
+    assert torch.equal(vt, kept)
+
+
+def test_restrict_potential_of_no_spins(torch):
+    from gpaw_amd.callers import restrict_potential
+    from gpaw_amd.transformers import Transformer
+    gd, fine = grids(True)
+    restrict_potential(Transformer(fine, gd, 3), rand(torch, (0,) + tuple(fine.n_c)),
+                       rand(torch, fine.n_c), rand(torch, (0,) + tuple(gd.n_c)))
+
+
+@pytest.mark.parametrize('x, nin', [((4, 3), 2), ((2, 3, 4), 2), ((3, 5), 2), ((12,), 2),
+                                    ((3, 4), 1), ((3, 4), 3)])
+def test_axpby_shared_wants_the_shape_of_a_function(torch, x, nin):
+    from gpaw_amd import ops
+    y = rand(torch, (2, 3, 4))
+    kept = y.clone()
+    with pytest.raises(ValueError):
+        ops.axpby_shared(y, rand(torch, x), 1.0, 1.0, nin)
+    assert torch.equal(y, kept)
