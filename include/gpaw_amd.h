@@ -341,7 +341,8 @@ int gpaw_axpby(double* y, const double* x, double a, double b, long n,
                void* stream);
 
 /* y_k = a*y_k + b*x for nin functions of n doubles, x shared by them (the
- * spins' vt_g += vHt_g, gpaw/hamiltonian.py:254-256). */
+ * spins' vt_g += vHt_g, gpaw/hamiltonian.py:254-256), in the order of k: x may
+ * be one of the y_k, else the two must not overlap. */
 int gpaw_axpby_shared(double* y, const double* x, double a, double b, long nin,
                       long n, void* stream);
 

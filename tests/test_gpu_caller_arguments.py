@@ -71,3 +71,20 @@ def test_axpby_shared_wants_the_shape_of_a_function(torch, x, nin):
     with pytest.raises(ValueError):
         ops.axpby_shared(y, rand(torch, x), 1.0, 1.0, nin)
     assert torch.equal(y, kept)
+
+
+@pytest.mark.parametrize('which', [0, 1, 2])
+def test_potential_that_is_one_of_the_spins(torch, which):
+    """vt_g += vHt_g spin by spin: where vHt_g is one spin's vt_g, the later
+    spins get what the earlier addition made of it."""
+    from gpaw_amd.callers import restrict_potential
+    from gpaw_amd.transformers import Transformer
+    print('case vHt_g = vt_sg[%d]' % which, flush=True)
+    gd, fine = grids(False)
+    vt = rand(torch, (3,) + tuple(fine.n_c))
+    want = vt.clone()
+    for s in range(3):
+        want[s] += want[which]
+    restrict_potential(Transformer(fine, gd, 3), vt, vt[which],
+                       rand(torch, (3,) + tuple(gd.n_c)))
+    assert torch.equal(vt, want)
