@@ -82,11 +82,12 @@ def restrict_potential(restrictor, vt_sg, vHt_g, vt_sG):
     vH = Arg(vHt_g, name='vHt_g')
     out = Arg(vt_sG, write=True, name='vt_sG')
     t = fine.tensor
-    spins = t[None] if t.dim() == 3 else t
-    if spins.shape[0]:
-        # the same fine grid for every spin: nothing is broadcast or cut short
-        vH = Arg(vH.tensor, name='vHt_g', shape=tuple(spins.shape[1:]), code=_lib.GPAW_F64)
-        ops.axpby_shared(spins, vH.tensor, 1.0, 1.0, spins.shape[0])
+    nspins, grid = (1, fine.shape) if t.dim() == 3 else (t.shape[0], fine.shape[1:])
+    if nspins:
+        if vH.shape != grid:
+            raise ValueError('restrict_potential: vHt_g of shape %s for vt_sg of shape %s'
+                             % (vH.shape, fine.shape))
+        ops.axpby_shared(t, vH.tensor, 1.0, 1.0, nspins)
     restrictor.apply(t, out.tensor)
     fine.finish()
     out.finish()
