@@ -23,6 +23,17 @@ import numpy as np
 
 from . import _arrays, _lib, ops
 from ._arrays import Arg
+from .grid_descriptor import GridDescriptor
+from .transformers import _Transformer
+
+# what a call may be merged past: these methods and nothing put in their place
+_APPLY, _HANDLE_APPLY = _Transformer.apply, ops.TransformerHandle.apply
+_INTEGRATE = GridDescriptor.integrate
+
+
+def _is(method, own):
+    """Whether a bound method is `own`, not a subclass's or a replacement."""
+    return getattr(method, '__func__', None) is own
 
 
 def apply_local_potential(vt_G, psit_nG, Htpsit_nG):
@@ -57,17 +68,19 @@ def interpolate_density(interpolator, finegd, nt_sG, nt_sg, charge=0.0,
     src = Arg(nt_sG, name='nt_sG')
     pseudo_charge = -(charge + comp_charge)
     scale = not finegd.pbc_c.all() and abs(pseudo_charge) > 1.0e-14
-    few = np.prod(out.shape[:-3]) <= _lib.GPAW_RENORMALIZE_MAX
-    handle = getattr(interpolator, 'transformer', None)
-    if scale and few and isinstance(handle, ops.TransformerHandle) and \
-            src.code == out.code == _lib.GPAW_F64:
+    # numpy adds 8 and more integrals in another order
+    few = scale and np.prod(out.shape[:-3]) <= _lib.GPAW_RENORMALIZE_MAX and \
+        _is(finegd.integrate, _INTEGRATE)
+    if few and src.code == out.code == _lib.GPAW_F64 and \
+            _is(interpolator.apply, _APPLY) and \
+            _is(getattr(interpolator.transformer, 'apply', None), _HANDLE_APPLY):
         # one call: the interpolation sums what it stores
-        handle.apply_renormalize(finegd, src.tensor, out.tensor, pseudo_charge)
+        interpolator.transformer.apply_renormalize(finegd, src.tensor, out.tensor, pseudo_charge)
     else:
         interpolator.apply(src.tensor, out.tensor)
-        if scale and few:
+        if few:
             ops.renormalize(finegd, out.tensor, pseudo_charge)
-        elif scale:   # numpy adds 8 and more integrals in another order
+        elif scale:
             x = pseudo_charge / np.sum(finegd.integrate(out.tensor))
             ops.scale(out.tensor, x)
     out.finish()

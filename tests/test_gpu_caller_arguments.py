@@ -88,3 +88,71 @@ def test_potential_that_is_one_of_the_spins(torch, which):
     restrict_potential(Transformer(fine, gd, 3), vt, vt[which],
                        rand(torch, (3,) + tuple(gd.n_c)))
     assert torch.equal(vt, want)
+
+
+def density(torch, gd, fine, nspins=2):
+    return rand(torch, (nspins,) + tuple(gd.n_c)), rand(torch, (nspins,) + tuple(fine.n_c), 2)
+
+
+@pytest.mark.parametrize('where', ['subclass', 'object', 'class', 'handle'])
+def test_interpolate_density_goes_through_apply(torch, where, monkeypatch):
+    """The interpolator's own apply runs wherever it was put in place of the
+    package's: once, and what it leaves is what is scaled."""
+    from gpaw_amd import ops
+    from gpaw_amd.callers import interpolate_density
+    from gpaw_amd.transformers import Transformer, _Transformer
+    print('case interpolate_density, apply of the', where, flush=True)
+    gd, fine = grids(False)
+    n, out = density(torch, gd, fine)
+    calls = []
+
+    def hook(apply, at=1):            # at: where the output is among the arguments
+        def hooked(*args):
+            calls.append(1)
+            apply(*args)
+            args[at][..., :3] *= 2.0
+        return hooked
+
+    plain = Transformer(gd, fine, 3)
+    if where == 'subclass':
+        class Mine(_Transformer):
+            def apply(self, input, output):
+                hook(super().apply)(input, output)
+        tr = Mine(gd, fine, 3)
+    else:
+        tr = Transformer(gd, fine, 3)
+        if where == 'object':
+            tr.apply = hook(tr.apply)
+        elif where == 'class':
+            monkeypatch.setattr(_Transformer, 'apply', hook(_Transformer.apply, 2))
+        else:
+            tr.transformer.apply = hook(tr.transformer.apply)
+    interpolate_density(tr, fine, n, out, charge=-8.0)
+    monkeypatch.undo()
+    assert len(calls) == 1
+    want = torch.empty_like(out)
+    plain.apply(n, want)
+    want[..., :3] *= 2.0
+    ops.scale(want, 8.0 / np.sum(fine.integrate(want)))
+    assert torch.equal(out, want)
+
+
+def test_interpolate_density_goes_through_integrate(torch):
+    from gpaw_amd import ops
+    from gpaw_amd.callers import interpolate_density
+    from gpaw_amd.grid_descriptor import GridDescriptor
+    from gpaw_amd.transformers import Transformer
+
+    class Half(GridDescriptor):       # one of two equal parts of a larger cell
+        def integrate(self, a_xg, b_xg=None, global_integral=True):
+            return 2.0 * GridDescriptor.integrate(self, a_xg, b_xg)
+
+    gd, plain = grids(False)
+    fine = Half(plain.N_c, plain.cell_cv, plain.pbc_c)
+    n, out = density(torch, gd, fine)
+    tr = Transformer(gd, fine, 3)
+    interpolate_density(tr, fine, n, out, charge=-8.0)
+    want = torch.empty_like(out)
+    tr.apply(n, want)
+    ops.scale(want, 8.0 / np.sum(fine.integrate(want)))
+    assert torch.equal(out, want)
