@@ -156,3 +156,19 @@ def test_interpolate_density_goes_through_integrate(torch):
     tr.apply(n, want)
     ops.scale(want, 8.0 / np.sum(fine.integrate(want)))
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize('pbc', [False, True])
+def test_interpolate_density_of_no_spins(torch, pbc):
+    """Nothing to scale to a charge is an error, as integrating it is; without
+    a scaling there is nothing to do."""
+    from gpaw_amd import _lib
+    from gpaw_amd.callers import interpolate_density
+    from gpaw_amd.transformers import Transformer
+    gd, fine = grids(pbc)
+    n, out = density(torch, gd, fine, 0)
+    if pbc:
+        interpolate_density(Transformer(gd, fine, 3), fine, n, out, charge=-8.0)
+        return
+    with pytest.raises(_lib.GpawAmdError):
+        interpolate_density(Transformer(gd, fine, 3), fine, n, out, charge=-8.0)
