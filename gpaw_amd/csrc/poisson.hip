@@ -531,16 +531,8 @@ extern "C" int gpaw_poisson_vcycles(gpaw_poisson* ps, double* phi, const double*
     return rc;
 }
 
-// What a solve whose V-cycles started before the charge was known still has
-// to read: its charge, and whether that is neutral.
-struct ChargeCheck {
-    double maxcharge;
-    double* charge;
-    int* neutral;
-};
-
 static int solve_loaded(gpaw_poisson* ps, double* phi, double eps, int maxiter, int* niter,
-                        double* error, const ChargeCheck* check, hipStream_t st);
+                        double* error, hipStream_t st);
 
 extern "C" int gpaw_poisson_solve_neutral(gpaw_poisson* ps, double* phi, const double* rho,
                                           double eps, int maxiter, int* niter, double* error,
@@ -550,7 +542,7 @@ extern "C" int gpaw_poisson_solve_neutral(gpaw_poisson* ps, double* phi, const d
     hipStream_t st = (hipStream_t)stream;
     int rc = load_inputs(ps, phi, rho, st);
     if (rc) return rc;
-    return solve_loaded(ps, phi, eps, maxiter, niter, error, nullptr, st);
+    return solve_loaded(ps, phi, eps, maxiter, niter, error, st);
 }
 
 // The charge dv * sum(rho) of gd.integrate into h_err[0] (same kernels and
@@ -566,12 +558,11 @@ static int launch_neutralize(gpaw_poisson* ps, const double* rho, hipStream_t st
 }
 
 // the charge once the launches above are done
-static void read_charge(gpaw_poisson* ps, const ChargeCheck& c)
+static void read_charge(gpaw_poisson* ps, double maxcharge, double* charge, int* neutral)
 {
     const double q = ps->h_err[0];
-    *c.charge = q;
-    *c.neutral = std::fabs(q) <= c.maxcharge;   // charged: the caller's branches
-    ps->was_neutral = *c.neutral != 0;
+    *charge = q;
+    *neutral = std::fabs(q) <= maxcharge;   // charged: the caller's branches
 }
 
 extern "C" int gpaw_poisson_neutralize(gpaw_poisson* ps, const double* rho, double maxcharge,
@@ -583,7 +574,7 @@ extern "C" int gpaw_poisson_neutralize(gpaw_poisson* ps, const double* rho, doub
     int rc = launch_neutralize(ps, rho, st);
     if (!rc) rc = gpaw_check(hipStreamSynchronize(st), "poisson: charge");
     if (rc) return rc;
-    read_charge(ps, {maxcharge, charge, neutral});
+    read_charge(ps, maxcharge, charge, neutral);
     ps->rho_loaded = *neutral != 0;
     return GPAW_OK;
 }
@@ -595,26 +586,23 @@ extern "C" int gpaw_poisson_solve(gpaw_poisson* ps, double* phi, const double* r
     if (!ps || !phi || !rho || !charge || !neutral || maxiter < 1)
         return gpaw_fail(GPAW_EINVAL, "poisson: bad argument");
     hipStream_t st = (hipStream_t)stream;
-    // After a neutral density (as in every step of an SCF loop) the first
-    // V-cycles are launched before the charge is read: waiting for it first left
-    // the GPU idle for about 40 us.  On a charged one they are thrown away: phi is
-    // written only once the charge is known.
-    const ChargeCheck check = {maxcharge, charge, neutral};
-    const bool early = ps->was_neutral;
-    int rc;
-    if (early) {
-        *neutral = 0;
-        rc = launch_neutralize(ps, rho, st);
-        if (!rc) rc = gpaw_check(hipEventRecord(ps->charge_ev, st), "poisson: charge");
-    } else {
-        rc = gpaw_poisson_neutralize(ps, rho, maxcharge, charge, neutral, stream);
-        if (!rc && !*neutral) return GPAW_OK;
-    }
+    *neutral = 0;
+    int rc = launch_neutralize(ps, rho, st);
+    // Every V-cycle waits for the charge, a charged density runs none.  phi is
+    // copied into the plan meanwhile: with that a neutral solve takes what it took
+    // when its cycles were launched before the charge was known (48x48x64 551
+    // against 548 us, 95^3 809 both), and a charged density after a neutral one no
+    // longer waits for cycles that are thrown away (1143 and 1980 us a solve, now
+    // 623 and 1200)
+    if (!rc) rc = gpaw_check(hipEventRecord(ps->charge_ev, st), "poisson: charge");
+    if (!rc)
+        rc = gpaw_check(launch_copy(ps->phiA[0], phi, DT_F64, ps->npts[0], st), "poisson: load");
+    if (!rc) rc = gpaw_check(hipEventSynchronize(ps->charge_ev), "poisson: charge");
     if (rc) return rc;
-    ps->rho_loaded = false;
-    rc = gpaw_check(launch_copy(ps->phiA[0], phi, DT_F64, ps->npts[0], st), "poisson: load");
-    if (rc) return rc;
-    return solve_loaded(ps, phi, eps, maxiter, niter, error, early ? &check : nullptr, st);
+    read_charge(ps, maxcharge, charge, neutral);
+    if (!*neutral)   // nothing of the call is left on the stream
+        return gpaw_check(hipStreamSynchronize(st), "poisson: charge");
+    return solve_loaded(ps, phi, eps, maxiter, niter, error, st);
 }
 
 extern "C" int gpaw_poisson_remove_mean(gpaw_poisson* ps, int on)
@@ -631,7 +619,7 @@ hipError_t gpaw_poisson_store(gpaw_poisson* ps, double* phi, const double* resul
 }
 
 static int solve_loaded(gpaw_poisson* ps, double* phi, double eps, int maxiter, int* niter,
-                        double* error, const ChargeCheck* check, hipStream_t st)
+                        double* error, hipStream_t st)
 {
     int rc = ensure_chunks(ps);
     if (rc) return rc;
@@ -661,14 +649,6 @@ static int solve_loaded(gpaw_poisson* ps, double* phi, double eps, int maxiter, 
         rc = run_chunk(ps, k, state, st);
         if (rc) return rc;
         hipError_t e = hipSuccess;
-        if (check) {           // the charge came back while the chunk was launched
-            e = hipEventSynchronize(ps->charge_ev);
-            if (e != hipSuccess) return gpaw_check(e, "poisson: charge");
-            read_charge(ps, *check);
-            if (!*check->neutral)
-                return gpaw_check(hipStreamSynchronize(st), "poisson: charge");
-            check = nullptr;
-        }
         stored = jac && expect;
         if (stored) e = gpaw_poisson_store(ps, phi, ps->snap[k - 1], st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);

@@ -46,9 +46,6 @@ struct gpaw_poisson {
     } rot;
     double* d_sum = nullptr;   // partial sums of the charge and mean integrals
     hipEvent_t charge_ev = nullptr;   // after the charge integral
-    // the last density was neutral: the next solve starts its V-cycles before
-    // it has read the charge back
-    bool was_neutral = false;
     // solutions leave with their mean removed (gpaw_poisson_remove_mean)
     bool remove_mean = false;
     // rho[0] holds a density gpaw_poisson_neutralize wrote (a solve may

@@ -144,8 +144,7 @@ int gpaw_poisson_neutralize(gpaw_poisson* ps, const double* rho, double maxcharg
 
 /* gpaw_poisson_neutralize, then for a neutral density solve_neutral as
  * above (*neutral = 1); a charged one returns with *neutral = 0 and phi as it
- * was.  After a neutral density the V-cycles are launched before the charge is
- * read back. */
+ * was. */
 int gpaw_poisson_solve(gpaw_poisson* ps, double* phi, const double* rho, double eps,
                        int maxiter, double maxcharge, double* charge, int* neutral,
                        int* niter, double* error, void* stream);
