@@ -636,12 +636,27 @@ extern "C" int gpaw_tile_shape(int threads, int tz, int planes)
     return GPAW_OK;
 }
 
+// stencil kernel families 0 .. 4 of kernels.h in the header's numbering
+static const int kernel_header[5] = {4, 3, 1, 2, 5};
+
 extern "C" int gpaw_stencil_kernel(int kind)
 {
-    // header numbering: 0 default, 1 tile, 2 box, 3 queue, 4 generic
-    static const int to_internal[5] = {-1, 2, 3, 1, 0};
-    static const int to_header[5] = {4, 3, 1, 2, 0};   // internal 0..3 -> header
-    if (kind < -1 || kind > 4) return -1;
+    // header numbering: 0 default, 1 tile, 2 box, 3 queue, 4 generic, 5 pair
+    static const int to_internal[6] = {-1, 2, 3, 1, 0, 4};
+    if (kind < -1 || kind > 5) return -1;
     const int prev = stencil_kernel_set(kind < 0 ? -2 : to_internal[kind]);
-    return prev < 0 ? 0 : to_header[prev];
+    return prev < 0 ? 0 : kernel_header[prev];
+}
+
+extern "C" int gpaw_operator_kernel(const gpaw_operator* op, long nin, int dtype, int potential,
+                                    int* columns, int* planes)
+{
+    if (!op || !columns || !planes) return gpaw_fail(GPAW_EINVAL, "operator kernel: NULL argument");
+    int rc = gpaw_check_dtype(op->real, dtype);
+    if (rc) return rc;
+    if (potential && dtype != DT_F64 && dtype != DT_C128)
+        return gpaw_fail(GPAW_EINVAL, "operator kernel: float64 or complex128 bands");
+    if (nin < 1 || nin > 65535) return gpaw_fail(GPAW_EINVAL, "operator kernel: nin = %ld", nin);
+    return kernel_header[stencil_choice(op->st, dtype, potential ? ST_HPSI : ST_APPLY, op->g,
+                                        (int)nin, columns, planes)];
 }

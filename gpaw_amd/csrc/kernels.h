@@ -105,7 +105,7 @@ struct Stencil {
 // table of the choices made.
 int autotune_set(int on);
 // Kernel family of star-stencil launches without partial sums: -1 default,
-// 0 generic, 1 register queue, 2 tile, 3 box; returns the previous value.
+// 0 generic, 1 register queue, 2 tile, 3 box, 4 pair; returns the previous value.
 int stencil_kernel_set(int kind);
 int tile_shape_set(int nt, int tz, int q);   // gpaw_tile_shape
 long autotune_report(char* buf, long len);
@@ -175,6 +175,10 @@ hipError_t launch_stencil(const Stencil& s, int dtype, int mode, const void* in,
                           const void* aux, const Geom& g, const Phases& ph, int nin,
                           double w, double* partial, int* npartial, bool write,
                           hipStream_t st);
+// The kernel family (numbered as in stencil_kernel_set), columns and planes
+// that launch_stencil takes for a launch without partial sums that the tuner
+// has no entry for.
+int stencil_choice(const Stencil& s, int dtype, int mode, const Geom& g, int nin, int* TZ, int* q);
 
 // Restriction / interpolation.
 struct Transfer {

@@ -405,7 +405,7 @@ int tile_shape_set(int nt, int tz, int q)
 int stencil_kernel_set(int kind)
 {
     const int prev = g_kind_override.load();
-    if (kind >= -1 && kind <= K_BOX) g_kind_override.store(kind);
+    if (kind >= -1 && kind <= K_PAIR) g_kind_override.store(kind);
     return prev;
 }
 
@@ -937,56 +937,79 @@ long autotune_report(char* buf, long len)
     return (long)r.size();
 }
 
-hipError_t launch_stencil(const Stencil& s, int dtype, int mode, const void* in, void* out,
-                          const void* aux, const Geom& g, const Phases& ph, int nin, double w,
-                          double* partial, int* npartial, bool write, hipStream_t st)
+// The configuration of a launch before the tuner: the default rules, or the
+// family that gpaw_stencil_kernel asks for (*asked) where it can run the launch.
+static LaunchCfg choose(const Stencil& s, int dtype, int mode, const Geom& g, int nin,
+                        bool partial, bool* asked)
 {
+    *asked = false;
     LaunchCfg c{K_GENERIC, 64, TileShape{}};
     // complex applies of range <= 3 use 1024-thread tiles
     const int nt = (dtype_complex(dtype) && (mode == ST_APPLY || mode == ST_HPSI) && s.star_r <= 3)
                        ? TILE_NT_WIDE
                        : TILE_NT;
     c.kind = stencil_kind(s, g, dtype, mode, nin, c.TZ, c.sh, nt);
-    if (npartial) *npartial = stencil_partials(s, g, nin);
+    if (partial) return c;
     // 4-byte real data on grids of 2^19 points or more: boxes of 8 planes
     // (measured 6.0 / 9.2 / 14.5 us against 6.4 / 10.6 / 17.9 us for 4 planes
     // on 95^3 / 127^3 / 159^3); launches with partial sums keep the shared
     // layout above, whose block count sizes the callers' buffers
-    if (!partial && c.kind == K_BOX && dtype == DT_F32 &&
+    if (c.kind == K_BOX && dtype == DT_F32 &&
         (long)g.n[0] * g.n[1] * g.n[2] * nin >= (1L << 19)) {
         TileShape b8;
         if (box_geometry(g, s.star_r, nin, 8, b8)) c.sh = b8;
     }
-    if (!partial && c.kind == K_TILE && forced_kind() < 0) large_cfg(s, g, dtype, mode, nin, c);
+    if (c.kind == K_TILE && forced_kind() < 0) large_cfg(s, g, dtype, mode, nin, c);
     const int ov = g_kind_override.load();
-    if (!partial && ov >= 0 && ov != c.kind) {
-        // the requested family when it can run this launch, else the default
-        LaunchCfg o{ov, 64, TileShape{}};
-        bool ok = false;
-        if (ov == K_BOX) {
-            ok = box_mode_ok(dtype, mode) && s.star_r >= 1 && s.star_r <= 4 &&
+    if (ov < 0 || ov == c.kind) return c;
+    // the requested family when it can run this launch, else the default
+    LaunchCfg o{ov, 64, TileShape{}};
+    if (ov == K_BOX) {
+        *asked = box_mode_ok(dtype, mode) && s.star_r >= 1 && s.star_r <= 4 &&
                  box_geometry(g, s.star_r, nin, box_default_q(g, s.star_r, nin), o.sh);
-            o.TZ = BOX_TZ;
-        } else if (ov == K_TILE) {
-            ok = s.star_r >= 1 && tile_shape(g, s.star_r, dtype_size(dtype), nin, o.TZ, o.sh, nt);
-            const int fnt = g_tile_nt.load();
-            // a forced shape where the kernel is compiled for it (wide blocks:
-            // complex data of range <= 3)
-            if (ok && fnt && (fnt == TILE_NT || (dtype_complex(dtype) && s.star_r <= 3))) {
-                TileShape fs;
-                if (tile_geometry(g, s.star_r, dtype_size(dtype), nin, g_tile_tz.load(),
-                                  g_tile_q.load(), fs, fnt)) {
-                    o.TZ = g_tile_tz.load();
-                    o.sh = fs;
-                }
+        o.TZ = BOX_TZ;
+    } else if (ov == K_PAIR) {
+        *asked = pair_shape(s, g, dtype, mode, nin, o.TZ, o.sh);
+    } else if (ov == K_TILE) {
+        *asked = s.star_r >= 1 && tile_shape(g, s.star_r, dtype_size(dtype), nin, o.TZ, o.sh, nt);
+        const int fnt = g_tile_nt.load();
+        // a forced shape where the kernel is compiled for it (wide blocks:
+        // complex data of range <= 3)
+        if (*asked && fnt && (fnt == TILE_NT || (dtype_complex(dtype) && s.star_r <= 3))) {
+            TileShape fs;
+            if (tile_geometry(g, s.star_r, dtype_size(dtype), nin, g_tile_tz.load(),
+                              g_tile_q.load(), fs, fnt)) {
+                o.TZ = g_tile_tz.load();
+                o.sh = fs;
             }
-        } else if (ov == K_QUEUE) {
-            ok = s.star_r > 0;
-        } else {
-            ok = s.d_coefs != nullptr;
         }
-        if (ok) return launch_cfg(o, s, dtype, mode, in, out, aux, g, ph, nin, w, nullptr, write, st);
+    } else if (ov == K_QUEUE) {
+        *asked = s.star_r > 0;
+    } else {
+        *asked = s.d_coefs != nullptr;
     }
+    return *asked ? o : c;
+}
+
+int stencil_choice(const Stencil& s, int dtype, int mode, const Geom& g, int nin, int* TZ, int* q)
+{
+    bool asked;
+    const LaunchCfg c = choose(s, dtype, mode, g, nin, false, &asked);
+    const bool shaped = c.kind >= K_TILE;
+    *TZ = shaped ? c.TZ : 0;
+    *q = shaped ? c.sh.q : 0;
+    return c.kind;
+}
+
+hipError_t launch_stencil(const Stencil& s, int dtype, int mode, const void* in, void* out,
+                          const void* aux, const Geom& g, const Phases& ph, int nin, double w,
+                          double* partial, int* npartial, bool write, hipStream_t st)
+{
+    if (npartial) *npartial = stencil_partials(s, g, nin);
+    bool asked;
+    LaunchCfg c = choose(s, dtype, mode, g, nin, partial != nullptr, &asked);
+    if (asked)
+        return launch_cfg(c, s, dtype, mode, in, out, aux, g, ph, nin, w, nullptr, write, st);
     if (!partial && s.star_r >= 1 && s.star_r <= 4 && forced_kind() < 0 && tune_enabled()) {
         const TuneKey key{dtype, mode, s.star_r, g.n[0], g.n[1], g.n[2],
                           g.per[0] | g.per[1] << 1 | g.per[2] << 2, nin};
@@ -1014,7 +1037,7 @@ hipError_t launch_stencil(const Stencil& s, int dtype, int mode, const void* in,
         return hipErrorInvalidValue;
     // stencils without a star form; partial sums (whose layout the callers
     // size) and a forced generic kernel keep k_generic
-    if (c.kind == K_GENERIC && !s.star_r && !partial && ov != K_GENERIC &&
+    if (c.kind == K_GENERIC && !s.star_r && !partial && g_kind_override.load() != K_GENERIC &&
         forced_kind() != K_GENERIC) {
         bool handled = false;
         hipError_t e = hipSuccess;

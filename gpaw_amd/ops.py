@@ -92,6 +92,18 @@ class OperatorHandle:
             _arrays.stream()))
         b.finish()
 
+    def kernel(self, in_xg, potential=False):
+        """(family, columns, planes) of the launch that apply, or
+        apply_potential, makes for in_xg where the tuner has not timed it
+        (columns and planes 0 for the families without tiles)."""
+        a = Arg(in_xg, name='input')
+        tz, q = ctypes.c_int(0), ctypes.c_int(0)
+        k = _lib.lib().gpaw_operator_kernel(self.h, _nin(a.shape, self.shape), a.code,
+                                            int(potential), ctypes.byref(tz), ctypes.byref(q))
+        if k < 0:
+            _lib.check(k)
+        return {v: n for n, v in STENCIL_KERNELS.items()}[k], tz.value, q.value
+
     def relax(self, relax_method, f_g, s_g, nrelax, w=1.0):
         if w is None:   # PyArg_ParseTuple("iOOi|d") rejects None
             raise TypeError('a float is required')
@@ -340,7 +352,7 @@ def autotune(enable=True):
     return bool(_lib.lib().gpaw_autotune(int(bool(enable))))
 
 
-STENCIL_KERNELS = {'default': 0, 'tile': 1, 'box': 2, 'queue': 3, 'generic': 4}
+STENCIL_KERNELS = {'default': 0, 'tile': 1, 'box': 2, 'queue': 3, 'generic': 4, 'pair': 5}
 
 
 def tile_shape(threads=0, tz=32, planes=1):
@@ -351,8 +363,8 @@ def tile_shape(threads=0, tz=32, planes=1):
 
 def stencil_kernel(kind='default'):
     """Kernel family for star-stencil launches without partial sums
-    ('default', 'tile', 'box', 'queue' or 'generic'; every family gives the
-    same bits); returns the previous family."""
+    ('default', 'tile', 'box', 'queue', 'generic' or 'pair'; every family gives
+    the same bits); returns the previous family."""
     prev = _lib.lib().gpaw_stencil_kernel(STENCIL_KERNELS[kind])
     return {v: k for k, v in STENCIL_KERNELS.items()}[prev]
 

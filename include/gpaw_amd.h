@@ -293,11 +293,20 @@ long gpaw_autotune_report(char* buf, long len);
  * carry no partial sums, for parity tests of every family and timing
  * experiments.  kind: 0 the default choice (heuristic or tuner), 1 the
  * plane-sweeping tile kernel, 2 the one-shot box kernel, 3 the register-
- * queue column kernel, 4 the generic kernel; a family that cannot run a
- * launch (grid too small, stencil not a star) leaves it to the default;
- * -1 only queries.  Returns the previous setting.  Every family gives
+ * queue column kernel, 4 the generic kernel, 5 the tile kernel of two planes a
+ * step; a family that cannot run a launch (grid too small, stencil not a star,
+ * for 5 also a range above 3 or another pass than an apply, with or without a
+ * potential) leaves it to the default; -1 only queries.  Returns the previous setting.  Every family gives
  * bit-identical results. */
 int gpaw_stencil_kernel(int kind);
+
+/* The family (1 .. 5 as above) that gpaw_operator_apply takes for nin
+ * functions, or gpaw_operator_apply_potential where potential is not 0, unless
+ * the tuner has timed that launch; with the columns and planes per block of
+ * families 1, 2 and 5 (0 for the others).  A negative value is an error
+ * code. */
+int gpaw_operator_kernel(const gpaw_operator* op, long nin, int dtype, int potential,
+                         int* columns, int* planes);
 
 /* Launch shape of the tile kernel, with gpaw_stencil_kernel(1), for launches
  * without partial sums (tests and timing experiments; no reference
