@@ -174,9 +174,9 @@ class TransformerHandle:
                 pass
             self.h = None
 
-    def _args(self, input, output):
-        a = Arg(input, name='input')
-        b = Arg(output, write=True, name='output')
+    def _args(self, input, output, code=None):
+        a = Arg(input, name='input', code=code)
+        b = Arg(output, write=True, name='output', code=code)
         if a.shape[-3:] != self.ngpin or b.shape[-3:] != self.ngpout or \
                 a.shape[:-3] != b.shape[:-3]:
             raise ValueError('transformer apply: shapes %s -> %s for %s -> %s'
@@ -186,8 +186,8 @@ class TransformerHandle:
         return a, b
 
     def apply_renormalize(self, gd, input, output, target):
-        """apply, then renormalize(gd, output, target): float64 device tensors
-        of at most 7 functions; gd is the output's grid."""
+        """apply, then renormalize(gd, output, target): float64 arrays of at
+        most 7 functions; gd is the output's grid."""
         a, b = self._args(input, output)
         nin = _nin(a.shape, self.ngpin)
         work = _arrays.torch().empty(max(1, nin) * _lib.GPAW_RENORMALIZE_WORK,

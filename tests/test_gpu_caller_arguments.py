@@ -172,3 +172,15 @@ def test_interpolate_density_of_no_spins(torch, pbc):
         return
     with pytest.raises(_lib.GpawAmdError):
         interpolate_density(Transformer(gd, fine, 3), fine, n, out, charge=-8.0)
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'complex64', 'complex128'])
+def test_apply_renormalize_is_of_float64(torch, dtype):
+    """The library is told float64: another type would be read past its end, or
+    as something else."""
+    from gpaw_amd.transformers import Transformer
+    gd, fine = grids(False)
+    n, out = density(torch, gd, fine)
+    t = getattr(torch, dtype)
+    with pytest.raises(TypeError):
+        Transformer(gd, fine, 3).transformer.apply_renormalize(fine, n.to(t), out.to(t), 8.0)
