@@ -604,14 +604,23 @@ int setup(gpaw_poisson* ps, int pr)
         // on the null stream, which the caller's stream need not wait for
         if (!rc) rc = gpaw_check(hipMemset(m->S, 0, sizeof(double) * S_N), "mixed: scalars");
         if (!rc) rc = gpaw_check(hipStreamSynchronize(nullptr), "mixed: scalars");
-        if (rc) return rc;
+        if (rc) {   // leave no half-built state behind
+            gpaw_mixed_free(m);
+            ps->mixed = nullptr;
+            return rc;
+        }
     }
     MixedState* m = ps->mixed;
     if (m->ready[pr]) return GPAW_OK;
     int rc = pr ? setup_v64(ps, m) : setup_v32(ps, m);
+    if (rc) {   // nor a half-built hierarchy
+        for (void* p : m->v[pr].owned) hipFree(p);
+        m->v[pr] = VLevels();
+        return rc;
+    }
     for (int t = 0; t < 2; t++) m->g_ba[pr][t].assign(MIXED_CHUNK_MAX, nullptr);
-    if (!rc) m->ready[pr] = true;
-    return rc;
+    m->ready[pr] = true;
+    return GPAW_OK;
 }
 
 void destroy_graphs(MixedState* m, int pr)
