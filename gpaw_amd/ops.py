@@ -188,7 +188,7 @@ class TransformerHandle:
     def apply_renormalize(self, gd, input, output, target):
         """apply, then renormalize(gd, output, target): float64 arrays of at
         most 7 functions; gd is the output's grid."""
-        a, b = self._args(input, output)
+        a, b = self._args(input, output, _lib.GPAW_F64)
         nin = _nin(a.shape, self.ngpin)
         work = _arrays.torch().empty(max(1, nin) * _lib.GPAW_RENORMALIZE_WORK,
                                      dtype=b.tensor.dtype, device=b.tensor.device)
