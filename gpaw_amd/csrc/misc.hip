@@ -70,21 +70,15 @@ __global__ __launch_bounds__(256) void k_axpby(double* __restrict__ y, const dou
 }
 
 // y_k = a*y_k + b*x for nin functions of n points, x shared by them (one
-// read of x and one launch instead of nin of each; bound by HBM).  x may be
-// one of the y_k: the later functions then see what was stored to it, as
-// after nin single calls.
-__global__ __launch_bounds__(256) void k_axpby_shared(double* y, const double* x, double a,
+// read of x and one launch instead of nin of each; bound by HBM)
+__global__ __launch_bounds__(256) void k_axpby_shared(double* __restrict__ y,
+                                                      const double* __restrict__ x, double a,
                                                       double b, int nin, i64 n)
 {
     const i64 i = (i64)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    double xi = x[i];
-    for (int k = 0; k < nin; k++) {
-        double* yk = y + k * n;
-        const double v = a * yk[i] + b * xi;
-        yk[i] = v;
-        if (yk == x) xi = v;
-    }
+    const double bx = b * x[i];
+    for (int k = 0; k < nin; k++) y[k * n + i] = a * y[k * n + i] + bx;
 }
 
 // y = x - b  (numpy's rho - background, phi -= phi_ave)
@@ -252,6 +246,12 @@ hipError_t launch_axpby_shared(double* y, const double* x, double a, double b, i
                                long long n, hipStream_t st)
 {
     if (n <= 0 || nin <= 0) return hipSuccess;
+    if (x < y + (i64)nin * n && y < x + n) {   // x is among the y_k: in the order of k
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < nin && e == hipSuccess; k++)
+            e = launch_axpby(y + k * n, x, a, b, n, st);
+        return e;
+    }
     launch_kernel(k_axpby_shared, grid1(n), dim3(256), 0, st, y, x, a, b, nin, (i64)n);
     return launch_error();
 }
