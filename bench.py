@@ -24,6 +24,7 @@ python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu] [--no-extra]
                 [--only fd_laplace|preconditioner|mixed_precision|serving|copy]
 """
 import argparse
+import gc
 import json
 import os
 import sys
@@ -81,7 +82,20 @@ def eps_for(np, gd, rho, rel=1e-10, eps_ref=2e-10):
 def event_time(torch, fn, reps, warm_s=0.03):
     """Average seconds per call of fn over `reps` calls, HIP events on the
     current stream, after at least `warm_s` seconds of untimed calls (the
-    GPU clocks ramp up under load; short warm-ups read 10% slow)."""
+    GPU clocks ramp up under load; short warm-ups read 10% slow).  Without the
+    interpreter's garbage collection, as in timeit: one of its full passes
+    takes about 30 ms here, in which the GPU idles."""
+    gc.collect()
+    on = gc.isenabled()
+    gc.disable()
+    try:
+        return _event_time(torch, fn, reps, warm_s)
+    finally:
+        if on:
+            gc.enable()
+
+
+def _event_time(torch, fn, reps, warm_s):
     st = torch.cuda.current_stream()
     e0 = torch.cuda.Event(enable_timing=True)
     e1 = torch.cuda.Event(enable_timing=True)
