@@ -16,8 +16,15 @@ import numpy as np
 from . import _arrays, _lib, ops
 from ._arrays import Arg
 from .fd_operators import Laplace, LaplaceA, LaplaceB
+from .grid_descriptor import GridDescriptor
 from .transformers import Transformer
 from .utilities import Gaussian, madelung
+
+
+# what phi's mean is formed with: the plan forms it itself where these are the
+# grid's own
+_INTEGRATE = GridDescriptor.integrate
+_GLOBAL_SIZE = GridDescriptor.get_size_of_global_array
 
 
 class PoissonConvergenceError(RuntimeError):
@@ -201,6 +208,29 @@ class PoissonSolver:
         solve_neutral."""
         return self.B is None and type(self).solve_neutral is PoissonSolver.solve_neutral
 
+    def _run(self, solve, *args):
+        """A solve of the library: its return code, and whether phi's mean is
+        left to _finish, as on a periodic grid with an integral or a size of its
+        own."""
+        own = getattr(self.gd.integrate, '__func__', None) is _INTEGRATE and \
+            getattr(self.gd.get_size_of_global_array, '__func__', None) is _GLOBAL_SIZE
+        if own or not np.all(self.gd.pbc_c):
+            return solve(self._plan, *args), False
+        L = _lib.lib()
+        _lib.check(L.gpaw_poisson_remove_mean(self._plan, 0))
+        try:
+            return solve(self._plan, *args), True
+        finally:
+            L.gpaw_poisson_remove_mean(self._plan, 1)
+
+    def _finish(self, P, mean):
+        """After a solve; mean: whether phi's mean is still to be removed."""
+        if mean:
+            phi_ave = self.gd.integrate(P.tensor) / self.gd.dv
+            phi_ave /= np.prod(self.gd.get_size_of_global_array())
+            ops.sub_scalar(P.tensor, P.tensor, phi_ave)
+        P.finish()
+
     def _solve_device(self, P, R, eps, maxcharge):
         """gpaw_poisson_solve: (niter, charge) when rho was neutral and the
         solve ran, else (None, charge) for the charged branches."""
@@ -209,9 +239,9 @@ class PoissonSolver:
         neutral = ctypes.c_int(0)
         niter = ctypes.c_int(0)
         err = ctypes.c_double(0.0)
-        rc = _lib.lib().gpaw_poisson_solve(
-            self._plan, P.ptr, R.ptr, float(eps), int(self.maxiter), float(maxcharge),
-            ctypes.byref(q), ctypes.byref(neutral), ctypes.byref(niter), ctypes.byref(err),
+        rc, mean = self._run(
+            _lib.lib().gpaw_poisson_solve, P.ptr, R.ptr, float(eps), int(self.maxiter),
+            float(maxcharge), ctypes.byref(q), ctypes.byref(neutral), ctypes.byref(niter), ctypes.byref(err),
             _arrays.stream())
         if not neutral.value:
             _lib.check(rc)
@@ -223,7 +253,7 @@ class PoissonSolver:
                 'Poisson solver did not converge in %d iterations!' %
                 self.maxiter)
         _lib.check(rc)
-        P.finish()
+        self._finish(P, mean)
         return niter.value, q.value
 
     def _args(self, phi, rho):
@@ -244,9 +274,9 @@ class PoissonSolver:
         self.phis[0] = P.tensor
         niter = ctypes.c_int(0)
         err = ctypes.c_double(0.0)
-        rc = _lib.lib().gpaw_poisson_solve_neutral(
-            self._plan, P.ptr, R.ptr, float(eps), int(self.maxiter),
-            ctypes.byref(niter), ctypes.byref(err), _arrays.stream())
+        rc, mean = self._run(
+            _lib.lib().gpaw_poisson_solve_neutral, P.ptr, R.ptr, float(eps),
+            int(self.maxiter), ctypes.byref(niter), ctypes.byref(err), _arrays.stream())
         self.error = err.value
         if rc == _lib.GPAW_ENOCONV:
             P.finish()
@@ -254,7 +284,7 @@ class PoissonSolver:
                 'Poisson solver did not converge in %d iterations!' %
                 self.maxiter)
         _lib.check(rc)
-        P.finish()
+        self._finish(P, mean)
         return niter.value
 
     def iterate2(self, step, level=0):
@@ -356,9 +386,9 @@ class MixedPoissonSolver(PoissonSolver):
         density gpaw_poisson_neutralize left in the plan)."""
         niter = ctypes.c_int(0)
         rel = ctypes.c_double(0.0)
-        rc = _lib.lib().gpaw_poisson_solve_mixed(
-            self._plan, P.ptr, rho_ptr, float(self.rel_tol), int(self.maxiter),
-            (1 if self.outer == 'pcg' else 0) |
+        rc, mean = self._run(
+            _lib.lib().gpaw_poisson_solve_mixed, P.ptr, rho_ptr, float(self.rel_tol),
+            int(self.maxiter), (1 if self.outer == 'pcg' else 0) |
             (2 if self.inner_precision == 'fp64' else 0) |
             (4 if self.reuse_history else 0), int(self.inner),
             ctypes.byref(niter), ctypes.byref(rel), _arrays.stream())
@@ -369,7 +399,7 @@ class MixedPoissonSolver(PoissonSolver):
                 'mixed-precision Poisson solver did not converge in %d '
                 'iterations' % self.maxiter)
         _lib.check(rc)
-        P.finish()
+        self._finish(P, mean)
         return niter.value
 
     def smoothing_weights(self, level=0):
