@@ -19,6 +19,8 @@ package):
 The spins (or bands) of one call go to the device as the band axis of ONE
 stencil / transfer launch.
 """
+from math import prod
+
 import numpy as np
 
 from . import _arrays, _lib, ops
@@ -69,7 +71,7 @@ def interpolate_density(interpolator, finegd, nt_sG, nt_sg, charge=0.0,
     pseudo_charge = -(charge + comp_charge)
     scale = not finegd.pbc_c.all() and abs(pseudo_charge) > 1.0e-14
     # numpy adds 8 and more integrals in another order; none cannot be scaled
-    few = scale and 1 <= np.prod(out.shape[:-3]) <= _lib.GPAW_RENORMALIZE_MAX and \
+    few = scale and 1 <= prod(out.shape[:-3]) <= _lib.GPAW_RENORMALIZE_MAX and \
         _is(finegd.integrate, _INTEGRATE)
     if few and src.code == out.code == _lib.GPAW_F64 and \
             _is(interpolator.apply, _APPLY) and \

@@ -278,9 +278,8 @@ def axpby_shared(y, x, a, b, nin):
     if yy.shape != (nin,) + xx.shape and not (nin == 1 and yy.shape == xx.shape):
         raise ValueError('axpby_shared: x of shape %s for %d functions in y of shape %s'
                          % (xx.shape, nin, yy.shape))
-    n = int(np.prod(xx.shape))
-    _lib.check(_lib.lib().gpaw_axpby_shared(yy.ptr, xx.ptr, float(a), float(b), nin, n,
-                                            _arrays.stream()))
+    _lib.check(_lib.lib().gpaw_axpby_shared(yy.ptr, xx.ptr, float(a), float(b), nin,
+                                            xx.tensor.numel(), _arrays.stream()))
     yy.finish()
 
 
