@@ -634,46 +634,78 @@ static bool pair_shape(const Stencil& s, const Geom& g, int dtype, int mode, int
 }
 
 // The kernel and shape of an apply (or kinetic + potential pass) of range <= 3
-// that is too large for the real-data box default, by storage type and range.
-// Measured on sets of 0.1 .. 2 GB (us; tile = k_star_tile with 256 or 1024
-// threads, box = k_star_box with 8 planes):
-//   float64    96 x 79x87x95   apply  pair 279  box 277  tile 290
-//                              + v         325      310       348
-//              256 x 64^3      apply       244      256       262
-//              128 x 63^3      + v         156      163       172
-//   complex64  60 x 56x60x51               60        54   58 / 60
-//              64 x 48^3                   46        40   43 / 53
-//   float32    256 x 64^3                 150       166       178
-//   complex128 R = 3: 256 x 64^3          468             470 / 449
-//              256 x 47^3                 220       263   247 / 283
-//              100 x 28x36x44              48        51    49 / 97
-//              12 x 96x80x72               71        61    61 / 82
-//              100 x 30x46x42  + v         63        60    56 / 73
-//              R = 2, 1: 60 x 60x50x70     93, 72  139, 109  125, 112 / 120, 92
-// 1024-thread tiles have the smallest halo but need planes that fill their
-// 32 x 32 columns.  The other modes and range 4 keep the tile kernel.
+// that is too large for the real-data box default, by storage type, range, row
+// length and the bytes read and written, S: sets that fit the 256 MB last-level
+// cache favour kernels with more blocks per CU.  Measured on 1760 drawn grids
+// of 20 .. 112 points an axis, 30 MB .. 1 GB a set: time over that of
+// k_star_tile with 256 threads (real data) or 1024 (complex data), geometric
+// means, on new arrays each call / on the same ones, one figure where S leaves
+// no difference; box = k_star_box with 8 planes, 256 = 256-thread tiles, and the
+// choice in brackets:
+//   float64, R = 3   rows        apply: pair, box          + v: pair, box
+//     S < 320 MB     .. 32   1.07/1.00   .99/1.03 [tile]   1.13/1.11   .99/1.01 [tile]
+//                   33 .. 48 [.85/.95] 1.03/1.09           [.97/1.03] 1.01/1.03
+//                   49 .. 64 [.80/.85]  .92/.91             .93/1.12  [.94/.98]
+//                   65 ..    [.93/1.02] .96/1.01           1.03/1.13  [.95/1.02]
+//     S >= 320 MB    .. 32   1.04       1.02     [tile]    1.10        .98     [tile]
+//                   33 .. 48 [.77]      1.01                [.84]      .93
+//                   49 .. 64 [.80]       .97                [.90]      .93
+//                   65 ..    [.88]       .95                [.87]      .94 [full boxes]
+//   float64, R < 3           [.76 .. .98]  .87 .. .98      [.81 .. 1.03]  .91 .. .99
+//   float32                  [.86/.88]     .91/.95
+//   complex64        R = 3    .80/.82     [.72/.74]   256 .79/.77
+//                    R < 3    .63/.68     [.66/.74]       .74/.78
+//   complex128, R = 3        apply: pair, 256                + v: pair, 256
+//     S < 256 MB     .. 32   [.81/.84]  .83/.76             .76/.79  [.78/.71]
+//                   33 .. 48  .96/.99  [.79/.74]            .92/.96  [.76/.72]
+//                   49 .. 64 [.73/.74]  .84/.75            [.75/.76]  .84/.80
+//                   65 .. 96 1.12/1.17 [.84/.81]           1.10/1.15 [.81/.82]
+//                   97 ..     .83/.79  [.84/.74]            .82/.81  [.83/.75]
+//     S >= 256 MB    .. 32   [.86]      .87                 .81      [.83]
+//                   33 .. 48  .96      [.84]                .95      [.83]
+//                   49 .. 64 [.77]      .87                [.79]      .92
+//                   65 .. 96 1.29      [.88]               1.22      [.88]
+//                   97 ..    [.84]      .90                [.80]      .86
+//   complex128, R < 3   .. 64, 97 ..   [.74 .. .93]  .72 .. 1.10
+//     65 .. 96, S < 200 MB    .91 .. 1.01  [.78 .. .88]; larger, R = 2, lanes filled
+//                             to less than 0.7: 1.00 [.92/.96], else [.94] .97
+// Single sets spread by +-10 % about these, on arrays that are still in the cache
+// some by 40 %.  1024-thread tiles have the smallest halo and stay where planes
+// fill their 32 x 32 columns (complex128 256 x 64^3: 451, pair 459 us); boxes stay
+// for float64 + v where 8 x 8 x 32 points of them are filled (96 x 79x87x95: 307,
+// pair 336, tile 351 us; 66 x 67x111x86, filled to 0.77: 311, 242, 255).  The other
+// modes and range 4 keep the tile kernel.
 static void large_cfg(const Stencil& s, const Geom& g, int dtype, int mode, int nin, LaunchCfg& c)
 {
-    const int R = s.star_r;
+    const int R = s.star_r, n0 = g.n[0], n1 = g.n[1], row = g.n[2];
     if (R < 1 || R > 3 || (mode != ST_APPLY && mode != ST_HPSI)) return;
-    LaunchCfg p{K_PAIR, 0, TileShape{}};
-    const bool row = g.n[2] <= 64;   // one tile per row
-    if (dtype == DT_C64 || (dtype == DT_F64 && mode == ST_HPSI && !row)) {
-        p.kind = K_BOX;
-        p.TZ = BOX_TZ;
-        if (box_geometry(g, R, nin, 8, p.sh)) c = p;
-        return;
+    const double MB = 2e-6 * dtype_size(dtype) * nin * n0 * n1 * row;
+    // share of the lanes that have a point, where each axis is cut into tiles
+    auto filled = [](int n, int tile) { return (double)n / ((n + tile - 1) / tile * tile); };
+    int kind = K_PAIR;
+    if (dtype == DT_C64) {
+        kind = K_BOX;
+    } else if (dtype == DT_F64) {
+        const bool pot = mode == ST_HPSI, cached = MB < 320;
+        if (R == 3 && row <= 32) return;
+        if (pot && row > 64)
+            kind = cached || filled(n0, 8) * filled(n1, 8) * filled(row, 32) >= 0.9 ? K_BOX : K_PAIR;
+        else if (pot && R == 3 && cached && row > 48)
+            kind = K_BOX;
+    } else if (dtype == DT_C128 && R == 3) {
+        if (filled(n1, 32) * filled(row, 32) >= 0.9) return;
+        const bool pair = row <= 32   ? mode == ST_APPLY
+                          : row <= 64 ? row > 48
+                                      : row > 96 && row <= 128 && MB >= 256;
+        kind = pair ? K_PAIR : K_TILE;
+    } else if (dtype == DT_C128 && row > 64 && row <= 96) {
+        if (MB < 200 || (R == 2 && filled(n1, 8) * filled(row, 48) < 0.7)) kind = K_TILE;
     }
-    if (dtype == DT_C128 && R == 3) {
-        const double lanes = (double)((g.n[1] + 31) / 32 * 32) * ((g.n[2] + 31) / 32 * 32);
-        if (g.n[1] * (double)g.n[2] >= 0.9 * lanes) return;   // 1024-thread tiles
-        if (mode == ST_HPSI || !row) {
-            p.kind = K_TILE;
-            if (tile_shape(g, R, dtype_size(dtype), nin, p.TZ, p.sh, TILE_NT)) c = p;
-            return;
-        }
-    }
-    if (pair_shape(s, g, dtype, mode, nin, p.TZ, p.sh)) c = p;
+    LaunchCfg p{kind, BOX_TZ, TileShape{}};
+    const bool ok = kind == K_BOX    ? box_geometry(g, R, nin, 8, p.sh)
+                    : kind == K_TILE ? tile_shape(g, R, dtype_size(dtype), nin, p.TZ, p.sh, TILE_NT)
+                                     : pair_shape(s, g, dtype, mode, nin, p.TZ, p.sh);
+    if (ok) c = p;
 }
 
 // `dtype` and `mode` decide whether the box kernel applies; partial-sum

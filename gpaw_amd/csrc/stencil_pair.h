@@ -11,13 +11,13 @@
 // a thread's own point only and stay in R registers.
 // Terms in k_star_tile's order with the same epilogue: bit-identical.
 //
-// HBM bound (R = 3): float64 96 x 79 x 87 x 95 295 -> 262 us (3.8 TB/s), with
-// the potential 365 -> 327; 128 x 79 x 87 x 63 254 -> 206; 256 x 64^3 269 -> 238;
-// complex128 256 x 47^3 283 -> 212, 100 x 28 x 36 x 44 97 -> 53; complex64
-// 60 x 56 x 60 x 51 79 -> 58.  Rings of R + 4 slots (one barrier per pair) and
-// tiles of 16 or 32 rows leave fewer blocks per CU and were no faster; two or
-// four bands per block, to share the potential, were slower (327 -> 357 us), and
-// so was running the bands of one tile together.
+// HBM bound.  R = 3, where the launch rule (large_cfg, stencil.hip) takes it:
+// float64 256 x 64^3 264 us with k_star_tile, 240 here (4.5 TB/s); 96 x 79x87x95
+// 290 and 264, 128 x 79x87x63 252 and 206; with the potential 128 x 63^3 176 and
+// 152; float32 256 x 64^3 182 and 149.  Rings of R + 4 slots (one barrier per pair)
+// and tiles of 16 or 32 rows leave fewer blocks per CU and were no faster; two or
+// four bands per block, to share the potential, were slower (96 x 79x87x95 327 ->
+// 357 us), and so was running the bands of one tile together.
 #pragma once
 #include "stencil_tile.h"
 
