@@ -650,7 +650,7 @@ static bool pair_shape(const Stencil& s, const Geom& g, int dtype, int mode, int
 //     S >= 320 MB    .. 32   1.04       1.02     [tile]    1.10        .98     [tile]
 //                   33 .. 48 [.77]      1.01                [.84]      .93
 //                   49 .. 64 [.80]       .97                [.90]      .93
-//                   65 ..    [.88]       .95                [.87]      .94 [full boxes]
+//                   65 ..    [.88]       .95                [.87]     [.94: < 512 MB or full]
 //   float64, R < 3           [.76 .. .98]  .87 .. .98      [.81 .. 1.03]  .91 .. .99
 //   float32                  [.86/.88]     .91/.95
 //   complex64        R = 3    .80/.82     [.72/.74]   256 .79/.77
@@ -689,7 +689,8 @@ static void large_cfg(const Stencil& s, const Geom& g, int dtype, int mode, int 
         const bool pot = mode == ST_HPSI, cached = MB < 320;
         if (R == 3 && row <= 32) return;
         if (pot && row > 64)
-            kind = cached || filled(n0, 8) * filled(n1, 8) * filled(row, 32) >= 0.9 ? K_BOX : K_PAIR;
+            kind = MB < 512 || filled(n0, 8) * filled(n1, 8) * filled(row, 32) >= 0.9 ? K_BOX
+                                                                                      : K_PAIR;
         else if (pot && R == 3 && cached && row > 48)
             kind = K_BOX;
     } else if (dtype == DT_C128 && R == 3) {

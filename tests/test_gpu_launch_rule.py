@@ -15,6 +15,7 @@ CASES = [
     ('float64', 66, (67, 111, 86), 3, True, 'pair'),       # tile 255; box 311, pair 242
     ('float64', 66, (71, 111, 96), 3, True, 'box'),        # filled boxes
     ('float64', 46, (66, 72, 91), 3, True, 'box'),         # in the last-level cache
+    ('float64', 44, (101, 64, 87), 3, True, 'box'),        # tile 142; pair 155
     ('float64', 95, (94, 48, 40), 3, False, 'pair'),
     ('float64', 95, (94, 48, 32), 2, False, 'pair'),
     ('complex128', 256, (26, 26, 37), 3, False, 'tile'),   # 95; pair 108
