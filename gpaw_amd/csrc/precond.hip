@@ -141,10 +141,16 @@ hipError_t pc_interp(const gpaw_operator* L, const Transfer& t, const void* b, c
     const i64 points = nin * pc_points(g.n);
     // complex bands below 2^18 points in all: every launch is a few us there, and
     // a block's serial planes cost what the launch saved (1 / 4 / 16 bands of
-    // 32^3: 49 / 51 / 54 us fused, 47 / 50 / 58 in steps); real bands gain at
-    // every size (3 bands of 79 x 63 x 71: 38 us instead of 41, one of 96^3: 33
-    // instead of 37)
+    // 32^3: 49 / 51 / 54 us fused, 47 / 50 / 58 in steps); real bands gain on most
+    // grids (3 bands of 79 x 63 x 71: 38 us instead of 41, one of 96^3: 33 instead
+    // of 37)
     if (VT<V>::cplx && points < 1 << 18) return hipErrorNotSupported;
+    // the level-0 pass of wider stencils where there is little to read: real rows
+    // of one tile (7 bands of 23 x 27 x 27: 32.6 us a call in steps, 36.9 fused; 24
+    // such grids 4 % slower fused), complex bands between walls (12 bands of
+    // 47 x 19 x 59: 52.5 and 55; 11 such grids 2 %; from 2^21 points fused is faster)
+    if (!b && !VT<V>::cplx && R > 1 && g.n[2] <= 32 && points < 1 << 18) return hipErrorNotSupported;
+    if (!b && VT<V>::cplx && R > 2 && !g.per[0] && points < 1 << 21) return hipErrorNotSupported;
     // 16 rows per block on large sets where they pad no more rows than 8 do
     // (complex128, 256 x 64^3: 1075 us a call with 8, 1001 with 16, 1009 with 32
     // rows; 64 x 32^3: 90 with 8, 82 with 16; real 16 x 48^3: 47 with 8, 50 with 16)
