@@ -68,23 +68,64 @@ __global__ __launch_bounds__(256) void k_interp2(const V* __restrict__ in, V* __
 
 // Tiles and i0 chunks of the tile kernels.  A block's planes are a serial
 // chain of about 1 us each, so few bands on one chunk leave the chip idle:
-// 2 x 127^3 -> 63^3 K = 6 is 32 blocks of 135 planes.  The axis is split until
-// there are TR_BLOCKS_RESTRICT / TR_BLOCKS_INTERP blocks (two / four per CU);
-// beyond that the 2 K - 3 (K - 1) planes that every chunk sweeps again cost
-// more than the blocks gain.  Measured, 1 / 256 / 512 / 1024 / 2048 blocks:
-// that restriction 121 / 27 / 25 / 36 / 54 us, the K = 6 interpolation
-// 2 x 63^3 -> 127^3 54 / 31 / 21 / 18.5 / 20 us.
+// 2 x 127^3 -> 63^3 K = 6 is 32 blocks of 135 planes.  The axis is split, but every
+// chunk sweeps 2 K - 3 (restriction; K - 1) planes again.
+// Interpolation: until there are TR_BLOCKS_INTERP blocks (four per CU); 1 / 256 /
+// 512 / 1024 / 2048 blocks on 2 x 63^3 -> 127^3, K = 6: 54 / 31 / 21 / 18.5 / 20 us.
+// Restriction: until there are TR_BLOCKS_RESTRICT blocks (121 / 27 / 25 / 36 / 54 us on
+// 2 x 127^3 -> 63^3), unless whole axes are estimated to take no longer; complex128,
+// whose blocks fill the chip at 512, by the estimate alone.  On 2500 drawn
+// grids of 40 .. 700 blocks complex128 loses 2 % to the best of 1 .. 8 chunks and never
+// to whole axes; splitting it until there are 512 blocks lost 12 %, and on 156 of
+// 974 to whole axes, for a few blocks more than a round (29 x 111x121x95 ->
+// 55x59x47, 464 blocks: 178 us, in two chunks 220).  Other types lose 5 .. 7 %.
 constexpr i64 TR_BLOCKS_RESTRICT = 512, TR_BLOCKS_INTERP = 1024;
 
-inline TileTr tile_tr(const TrArgs& t, bool interpolate, int nin)
+// planes a restriction in chunks of cq sweeps one after another: rounds of
+// `slots` blocks, the last one half as a whole one and half by its share
+inline double restrict_planes(int n0, int cq, int K, i64 base, int slots, double more)
+{
+    const i64 b = base * ((n0 + cq - 1) / cq);
+    const double rounds = 0.5 * ((double)((b + slots - 1) / slots) + (double)b / slots) + more;
+    return (rounds > 1.0 ? rounds : 1.0) * (2 * cq + 2 * K - 3);
+}
+
+inline i64 restrict_chunks(int n0, int K, i64 base, bool c128)
+{
+    if (!c128) {
+        i64 nch = (TR_BLOCKS_RESTRICT + base - 1) / base;
+        if (nch > n0) nch = n0;
+        const bool split = nch > 1 && restrict_planes(n0, (int)((n0 + nch - 1) / nch), K, base, 768, 0.25) <
+                                          restrict_planes(n0, n0, K, base, 768, 0.25);
+        return split ? nch : 1;
+    }
+    const double whole = restrict_planes(n0, n0, K, base, 512, 0.0);
+    double least = 0.95 * whole;
+    i64 best = 1;
+    // each chunk length once, while there are at most four rounds
+    for (int cq = n0; cq > 1;) {
+        const int next = (n0 + cq - 2) / (cq - 1);
+        cq = (n0 + next - 1) / next;
+        const i64 nch = (n0 + cq - 1) / cq;
+        if (base * nch > 2048) break;
+        const double planes = restrict_planes(n0, cq, K, base, 512, 0.0);
+        if (planes < least) {
+            least = 0.97 * planes;
+            best = nch;
+        }
+    }
+    return best;
+}
+
+inline TileTr tile_tr(const TrArgs& t, bool interpolate, int nin, int K, bool c128)
 {
     TileTr tt;
     tt.nt1 = (t.nout[1] + 7) / 8;
     tt.nt2 = (t.nout[2] + 31) / 32;
     const int n0 = interpolate ? interp2_cells(t, 0) : t.nout[0];   // outputs or centres
     const i64 base = (i64)tt.nt1 * tt.nt2 * nin;
-    const i64 want = interpolate ? TR_BLOCKS_INTERP : TR_BLOCKS_RESTRICT;
-    i64 nch = (want + base - 1) / base;
+    i64 nch = interpolate ? (TR_BLOCKS_INTERP + base - 1) / base
+                          : restrict_chunks(n0, K, base, c128);
     if (nch > n0) nch = n0;
     tt.cq = (int)((n0 + nch - 1) / nch);
     tt.nch = (n0 + tt.cq - 1) / tt.cq;
@@ -118,7 +159,7 @@ hipError_t tr_launch(const Transfer& tr, int mode, const void* in, void* out, vo
     const bool big2 = K == 2 && !tr.interpolate && t.ngout * nin >= (1 << 20);
     if ((K >= 4 || big2) && t.nout[1] >= 4 && t.nout[2] >= 16 &&
         (long)t.gin.n[1] * t.gin.n[2] < PLANE_REF_MAX && !getenv("GPAW_AMD_POINTWISE_TRANSFER")) {
-        const TileTr tt = tile_tr(t, tr.interpolate, nin);
+        const TileTr tt = tile_tr(t, tr.interpolate, nin, K, sizeof(V) == 16);
         const dim3 gt((unsigned)(tt.nt1 * tt.nt2 * tt.nch * nin));
         // chunked real restrictions (few blocks per CU) take two planes per
         // step: 25 us against 27 on 2 x 127^3 -> 63^3, K = 6; one plane is
