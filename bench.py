@@ -85,7 +85,6 @@ def event_time(torch, fn, reps, warm_s=0.03):
     GPU clocks ramp up under load; short warm-ups read 10% slow).  Without the
     interpreter's garbage collection, as in timeit: one of its full passes
     takes about 30 ms here, in which the GPU idles."""
-    gc.collect()
     on = gc.isenabled()
     gc.disable()
     try:
@@ -336,7 +335,7 @@ def preconditioner_c3(torch, np):
     256 complex128 bands of 64^3, periodic, Bloch phases, nn=3 kinetic
     operator on the fine grid.  Algorithmic bytes per call: every array a
     launch reads or writes counted once per launch, 16 B per point:
-    3 fine + 7 coarse-1 + 7 coarse-2 grid functions per band (the scaled
+    3 fine + 7 coarse-1 + 4 coarse-2 grid functions per band (the scaled
     residuals and the interpolations are formed inside the stencil passes)."""
     from gpaw_amd.fd_operators import Laplace
     from gpaw_amd.grid_descriptor import GridDescriptor
@@ -354,7 +353,7 @@ def preconditioner_c3(torch, np):
                     generator=g)
     t = event_time(torch, lambda: pc(r, Kpt), 5)
     n0 = N ** 3
-    algo = 16.0 * nb * (3 * n0 + 7 * n0 / 8 + 7 * n0 / 64)
+    algo = 16.0 * nb * (3 * n0 + 7 * n0 / 8 + 4 * n0 / 64)
     del r
     return {'config': 'Preconditioner(nn=3 kin), complex128, 256 bands x '
                       '64^3, Bloch phases',
