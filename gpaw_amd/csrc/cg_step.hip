@@ -10,8 +10,9 @@
 // Bound by memory: on 159^3 (32 MB a field) p and phi are read once and
 // phi, p', q written, 176 MB with the FP32 z; the separate launches also read p
 // once more for phi and p' once more for the operator (16.7 + 21.8 us and
-// 14 us of the update that subtracted alpha p).  The values are those of the
-// separate launches, bit for bit.
+// 14 us of the update that subtracted alpha p).  Each point is rounded as in the
+// separate launches; z.q is summed by 512 threads in the larger tiles and p.q over
+// other blocks, so beta and alpha can differ from theirs in the last bits.
 #include "cg_step.h"
 #include "stencil_box.h"
 

@@ -20,9 +20,12 @@
 // one, the first pass waited for three round trips), each thread keeps its
 // points' right-hand sides and neighbour indices in registers for all passes of
 // a level, and only the phi pair of every level lives in LDS (the residual
-// takes the array the last sweep read).  The block has no more waves than the
-// first level needs.  11^3 + 5^3 (16 sweeps): 17.6 us before, 12.7 now;
-// 6 x 6 x 8 + 3 x 3 x 4: 13.0 and 7.8; 9^3 alone (8 sweeps): 6.6 and 5.0.
+// takes the array the last sweep read).  With 1024 threads a lane has 128
+// registers: one point a thread and up to two levels of two points fit (123 at
+// four levels, 103), two points on three or four levels spill 12 and 84 bytes a
+// lane.  The block has no more waves than the first level needs.  11^3 + 5^3 (16
+// sweeps): 17.6 us before, 12.7 now; 6 x 6 x 8 + 3 x 3 x 4: 13.0 and 7.8; 9^3 alone
+// (8 sweeps): 6.6 and 5.0.
 #include "kernels.h"
 #include "coarse.h"
 #include "transfer_common.h"

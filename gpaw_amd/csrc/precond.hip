@@ -17,7 +17,7 @@
 //
 // Six launches where the levels allow it (pc_scaled, pc_interp): d1 = 4s r1, d2 = 16s r2,
 // d1 - I2(d2) and e0 = I1(d1) are formed inside the stencil passes that read
-// them (precond_sweep.h), so E0, D1 and D2 are never stored; 4.3 instead of
+// them (precond_sweep.h), so E0, D1 and D2 are never stored; 4.2 instead of
 // 7.4 GB on 256 complex128 bands of 64^3.  A pass that cannot be fused runs
 // its steps one by one.
 //

@@ -636,7 +636,7 @@ static bool pair_shape(const Stencil& s, const Geom& g, int dtype, int mode, int
 // The kernel and shape of an apply (or kinetic + potential pass) of range <= 3
 // that is too large for the real-data box default, by storage type, range, row
 // length and the bytes read and written, S: sets that fit the 256 MB last-level
-// cache favour kernels with more blocks per CU.  Measured on 1760 drawn grids
+// cache favour kernels with more blocks per CU.  Measured on 2200 drawn grids
 // of 20 .. 112 points an axis, 30 MB .. 1 GB a set: time over that of
 // k_star_tile with 256 threads (real data) or 1024 (complex data), geometric
 // means, on new arrays each call / on the same ones, one figure where S leaves
@@ -670,7 +670,8 @@ static bool pair_shape(const Stencil& s, const Geom& g, int dtype, int mode, int
 //     65 .. 96, S < 200 MB    .91 .. 1.01  [.78 .. .88]; larger, R = 2, lanes filled
 //                             to less than 0.7: 1.00 [.92/.96], else [.94] .97
 // Single sets spread by +-10 % about these, on arrays that are still in the cache
-// some by 40 %.  1024-thread tiles have the smallest halo and stay where planes
+// some by 40 %: 52 of the 2200 are more than 4 % slower than k_star_tile on new
+// arrays, 116 on the same ones.  1024-thread tiles have the smallest halo and stay where planes
 // fill their 32 x 32 columns (complex128 256 x 64^3: 451, pair 459 us); boxes stay
 // for float64 + v where 8 x 8 x 32 points of them are filled (96 x 79x87x95: 307,
 // pair 336, tile 351 us; 66 x 67x111x86, filled to 0.77: 311, 242, 255).  The other

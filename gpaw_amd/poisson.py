@@ -241,8 +241,8 @@ class PoissonSolver:
         err = ctypes.c_double(0.0)
         rc, mean = self._run(
             _lib.lib().gpaw_poisson_solve, P.ptr, R.ptr, float(eps), int(self.maxiter),
-            float(maxcharge), ctypes.byref(q), ctypes.byref(neutral), ctypes.byref(niter), ctypes.byref(err),
-            _arrays.stream())
+            float(maxcharge), ctypes.byref(q), ctypes.byref(neutral), ctypes.byref(niter),
+            ctypes.byref(err), _arrays.stream())
         if not neutral.value:
             _lib.check(rc)
             return None, q.value

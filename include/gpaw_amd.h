@@ -296,8 +296,8 @@ long gpaw_autotune_report(char* buf, long len);
  * queue column kernel, 4 the generic kernel, 5 the tile kernel of two planes a
  * step; a family that cannot run a launch (grid too small, stencil not a star,
  * for 5 also a range above 3 or another pass than an apply, with or without a
- * potential) leaves it to the default; -1 only queries.  Returns the previous setting.  Every family gives
- * bit-identical results. */
+ * potential) leaves it to the default; -1 only queries.  Returns the previous
+ * setting.  Every family gives bit-identical results. */
 int gpaw_stencil_kernel(int kind);
 
 /* The family (1 .. 5 as above) that gpaw_operator_apply takes for nin
