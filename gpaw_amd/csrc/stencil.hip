@@ -671,11 +671,11 @@ static bool pair_shape(const Stencil& s, const Geom& g, int dtype, int mode, int
 //                             to less than 0.7: 1.00 [.92/.96], else [.94] .97
 // Single sets spread by +-10 % about these, on arrays that are still in the cache
 // some by 40 %: 52 of the 2200 are more than 4 % slower than k_star_tile on new
-// arrays, 116 on the same ones.  1024-thread tiles have the smallest halo and stay where planes
-// fill their 32 x 32 columns (complex128 256 x 64^3: 451, pair 459 us); boxes stay
-// for float64 + v where 8 x 8 x 32 points of them are filled (96 x 79x87x95: 307,
-// pair 336, tile 351 us; 66 x 67x111x86, filled to 0.77: 311, 242, 255).  The other
-// modes and range 4 keep the tile kernel.
+// arrays, 116 on the same ones.  1024-thread tiles have the smallest halo and stay
+// where planes fill their 32 x 32 columns (complex128 256 x 64^3: 451, pair 459 us);
+// boxes stay for float64 + v where 8 x 8 x 32 points of them are filled
+// (96 x 79x87x95: 307, pair 336, tile 351 us; 66 x 67x111x86, filled to 0.77: 311,
+// 242, 255).  The other modes and range 4 keep the tile kernel.
 static void large_cfg(const Stencil& s, const Geom& g, int dtype, int mode, int nin, LaunchCfg& c)
 {
     const int R = s.star_r, n0 = g.n[0], n1 = g.n[1], row = g.n[2];
