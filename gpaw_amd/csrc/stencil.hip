@@ -637,10 +637,10 @@ static bool pair_shape(const Stencil& s, const Geom& g, int dtype, int mode, int
 // that is too large for the real-data box default, by storage type, range, row
 // length and the bytes read and written, S: sets that fit the 256 MB last-level
 // cache favour kernels with more blocks per CU.  Measured on 2200 drawn grids
-// of 20 .. 112 points an axis, 30 MB .. 1 GB a set: time over that of
-// k_star_tile with 256 threads (real data) or 1024 (complex data), geometric
-// means, on new arrays each call / on the same ones, one figure where S leaves
-// no difference; box = k_star_box with 8 planes, 256 = 256-thread tiles, and the
+// of 20 .. 112 points an axis, 30 MB .. 1 GB a set (and 881 complex128 ones from
+// 3 MB): time over that of k_star_tile with 256 threads (real data) or 1024
+// (complex data), geometric means, on new arrays each call / on the same ones, one
+// figure where S leaves no difference; box = k_star_box with 8 planes, 256 = 256-thread tiles, and the
 // choice in brackets:
 //   float64, R = 3   rows        apply: pair, box          + v: pair, box
 //     S < 320 MB     .. 32   1.07/1.00   .99/1.03 [tile]   1.13/1.11   .99/1.01 [tile]
@@ -656,6 +656,7 @@ static bool pair_shape(const Stencil& s, const Geom& g, int dtype, int mode, int
 //   complex64        R = 3    .80/.82     [.72/.74]   256 .79/.77
 //                    R < 3    .63/.68     [.66/.74]       .74/.78
 //   complex128, R = 3        apply: pair, 256                + v: pair, 256
+//     S < 16 MB      .. 128  [.72 .. .79] .73 .. .94       [.73 .. .76] .81 .. .90
 //     S < 256 MB     .. 32   [.81/.84]  .83/.76             .76/.79  [.78/.71]
 //                   33 .. 48  .96/.99  [.79/.74]            .92/.96  [.76/.72]
 //                   49 .. 64 [.73/.74]  .84/.75            [.75/.76]  .84/.80
@@ -667,6 +668,7 @@ static bool pair_shape(const Stencil& s, const Geom& g, int dtype, int mode, int
 //                   65 .. 96 1.29      [.88]               1.22      [.88]
 //                   97 ..    [.84]      .90                [.80]      .86
 //   complex128, R < 3   .. 64, 97 ..   [.74 .. .93]  .72 .. 1.10
+//     65 .. 96, S < 16 MB    [.93 .. .95]  .97 .. 1.01
 //     65 .. 96, S < 200 MB    .91 .. 1.01  [.78 .. .88]; larger, R = 2, lanes filled
 //                             to less than 0.7: 1.00 [.92/.96], else [.94] .97
 // Single sets spread by +-10 % about these, on arrays that are still in the cache
@@ -696,12 +698,14 @@ static void large_cfg(const Stencil& s, const Geom& g, int dtype, int mode, int 
             kind = K_BOX;
     } else if (dtype == DT_C128 && R == 3) {
         if (filled(n1, 32) * filled(row, 32) >= 0.9) return;
-        const bool pair = row <= 32   ? mode == ST_APPLY
+        const bool pair = MB < 16     ? row <= 128
+                          : row <= 32 ? mode == ST_APPLY
                           : row <= 64 ? row > 48
                                       : row > 96 && row <= 128 && MB >= 256;
         kind = pair ? K_PAIR : K_TILE;
     } else if (dtype == DT_C128 && row > 64 && row <= 96) {
-        if (MB < 200 || (R == 2 && filled(n1, 8) * filled(row, 48) < 0.7)) kind = K_TILE;
+        if (MB >= 16 && (MB < 200 || (R == 2 && filled(n1, 8) * filled(row, 48) < 0.7)))
+            kind = K_TILE;
     }
     LaunchCfg p{kind, BOX_TZ, TileShape{}};
     const bool ok = kind == K_BOX    ? box_geometry(g, R, nin, 8, p.sh)

@@ -20,6 +20,9 @@ CASES = [
     ('float64', 95, (94, 48, 32), 2, False, 'pair'),
     ('complex128', 256, (26, 26, 37), 3, False, 'tile'),   # 95; pair 108
     ('complex128', 256, (26, 26, 48), 3, False, 'tile'),
+    ('complex128', 10, (23, 53, 39), 3, False, 'pair'),    # 15.7; tile 16.5
+    ('complex128', 6, (23, 43, 70), 3, True, 'pair'),
+    ('complex128', 24, (23, 53, 39), 3, False, 'tile'),
     ('complex128', 128, (26, 36, 49), 3, False, 'pair'),
     ('complex128', 128, (26, 36, 49), 3, True, 'pair'),
     ('complex128', 128, (26, 36, 32), 3, False, 'pair'),
